@@ -32,28 +32,23 @@ template <typename R> __device__ __forceinline__ R vexp(R x);
 template <> __device__ __forceinline__ double vexp<double>(double x) { return exp(x); }
 template <> __device__ __forceinline__ float vexp<float>(float x) { return __expf(x); }
 // 1/x and 1/sqrt(x) for the positive, normal arguments of the set-up
-// (zeta, eta, zeta + eta, T >= BOYS_TMAX): hardware estimate refined by two
-// Newton steps in FP64 (each step squares the relative error), the estimate
-// alone in FP32.
+// (zeta, eta, zeta + eta, T >= BOYS_TMAX): the hardware estimate (relative error about 2^-24) and
+// one third-order correction in FP64, r (1 + e + e^2) and y (1 + e/2 + 3 e^2 / 8), whose error is
+// of order e^3 < 2^-68; the estimate alone in FP32.
 template <typename R> __device__ __forceinline__ R vrcp(R x);
 template <> __device__ __forceinline__ double vrcp<double>(double x)
 {
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-x, r, 1.0);
-    return fma(r, e, r);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
 }
 template <> __device__ __forceinline__ float vrcp<float>(float x) { return __builtin_amdgcn_rcpf(x); }
 template <typename R> __device__ __forceinline__ R vrsqrt(R x);
 template <> __device__ __forceinline__ double vrsqrt<double>(double x)
 {
-    double y = __builtin_amdgcn_rsq(x);
-    const double h = 0.5 * x;
-    double e = fma(-h * y, y, 0.5);
-    y = fma(y, e, y);
-    e = fma(-h * y, y, 0.5);
-    return fma(y, e, y);
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-(x * y), y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
 }
 template <> __device__ __forceinline__ float vrsqrt<float>(float x) { return __builtin_amdgcn_rsqf(x); }
 
@@ -63,13 +58,12 @@ template <> __device__ __forceinline__ float vrsqrt<float>(float x) { return __b
 template <int la, int lb, int lc, int ld>
 struct EriClass;
 
-// Boys function F_0..F_L(T).  T < BOYS_TMAX: F_L and F_{L-1} from their
-// order-BOYS_ORDER Taylor expansions around the nearest grid point (the two
-// blocks of table row k hold F_{L+j}(T_k) (-1)^j / j! and F_{L-1+j}(T_k)
-// (-1)^j / j!), then downward recursion F_m = (2T F_{m+1} + e^-T) / (2m+1).
+// Boys function F_0..F_L(T).  T < BOYS_TMAX: F_L from the polynomial of its grid row and e^-T from
+// the row's e^-T_k (vlx_boys.h), then downward recursion F_m = (2T F_{m+1} + e^-T) / (2m+1).
 // T >= BOYS_TMAX: F_0 = sqrt(pi/T)/2 (erf(sqrt(T)) = 1 to double precision
 // there) and upward recursion F_{m+1} = ((2m+1) F_m - e^-T) / (2T), stable
-// for T > L.
+// for T > L.  ROWS: the table is row-major (in HBM); else coefficient-major (in LDS, where the lanes
+// then read one coefficient at unrelated rows of a contiguous run: fewest bank conflicts).
 // FP32 quartets keep Boys arguments near zero in FP64: below BOYS_T_FP64 the FP32 kernels take F_L
 // from its series at T = 0, F_L(T) = sum_k (-T)^k / (k! (2L + 2k + 1)), and e^-T from its own series
 // (18 terms each: 1^18 / 18! < 2e-16), then the downward recursion in FP64.
@@ -102,12 +96,12 @@ __device__ __forceinline__ void boys_near_zero_fp64(const double t, float* __res
     }
 }
 
-template <int L, typename R>
+template <int L, typename R, bool ROWS = false>
 __device__ __forceinline__ void boys_eval(const R T, const R* __restrict__ tab, R* __restrict__ F)
 {
-    // Taylor orders: full table order in FP64; 5 terms reach FP32 rounding
-    // (0.125^6 / 6! ~ 5e-9)
+    // degree: the full row in FP64; degree 5 is far below FP32 rounding (the d^6 term is < 1e-11)
     constexpr int ORD = (sizeof(R) == 8) ? BOYS_ORDER : 5;
+    constexpr int RS = ROWS ? BOYS_ROW : 1, CS = ROWS ? 1 : BOYS_NGRID;
     if constexpr (sizeof(R) == 4) {
         if (T < R(BOYS_T_FP64)) {
             boys_near_zero_fp64<L>(static_cast<double>(T), F);
@@ -117,26 +111,19 @@ __device__ __forceinline__ void boys_eval(const R T, const R* __restrict__ tab, 
     if (T < R(BOYS_TMAX)) {
         const int k = static_cast<int>(T * R(BOYS_INV_DT) + R(0.5));
         const R d = T - R(BOYS_DT) * R(k);
-        const R* c = tab + k * BOYS_ROW;
-        R f = c[ORD];
+        const R* c = tab + k * RS;
+        R f = c[ORD * CS];
 #pragma unroll
-        for (int j = ORD - 1; j >= 0; j--) f = fma(f, d, c[j]);
+        for (int j = ORD - 1; j >= 0; j--) f = fma(f, d, c[j * CS]);
         F[L] = f;
         if constexpr (L > 0) {
-            // F_{L-1} from its own Taylor block of the row; then e^-T = (2L - 1) F_{L-1} - 2T F_L
-            // (the recursion at m = L - 1) for the downward steps.  At large T the difference
-            // cancels, but its error enters F_m with weight <= (2L - 1) F_{L-1} / ((2m + 1) F_m) <= 1
-            const R* c1 = c + (BOYS_ORDER + 1);
-            R g = c1[ORD];
+            R et = R(BOYS_EXPD[ORD]);
 #pragma unroll
-            for (int j = ORD - 1; j >= 0; j--) g = fma(g, d, c1[j]);
-            F[L - 1] = g;
-            if constexpr (L > 1) {
-                const R tt = R(2.0) * T;
-                const R et = R(2 * L - 1) * g - tt * f;
+            for (int j = ORD - 1; j >= 0; j--) et = fma(et, d, R(BOYS_EXPD[j]));
+            et *= c[BOYS_EXP_COL * CS];
+            const R tt = R(2.0) * T;
 #pragma unroll
-                for (int m = L - 2; m >= 0; m--) F[m] = (tt * F[m + 1] + et) * R(1.0 / (2 * m + 1));
-            }
+            for (int m = L - 1; m >= 0; m--) F[m] = fma(tt, F[m + 1], et) * R(1.0 / (2 * m + 1));
         }
     } else {
         const R rs = vrsqrt<R>(T);
@@ -164,6 +151,30 @@ __device__ __forceinline__ void boys_eval(const R T, const R* __restrict__ tab, 
     }
 }
 
+// Primitives of the lane's ket entry in the tiled kernel's lane-transposed layout: field f of
+// primitive ik at p[(ik * NF + f) * VLX_WAVE] (p: the chunk's block plus the lane).  NF = 5 (zeta, P,
+// K) for an (ss| ket, 8 with P - A otherwise.  The 64 lanes read consecutive words; as PrimPair
+// records every lane's primitive is a cache line of its own, 64 of them per load instruction, read
+// again for every bra.
+template <int NF>
+struct KetLane {
+    const double* __restrict__ p;
+    __device__ __forceinline__ PrimPair operator[](const int ik) const
+    {
+        const double* q = p + ik * (NF * VLX_WAVE);
+        PrimPair k;
+        k.zeta = q[0];
+        k.px = q[VLX_WAVE];
+        k.py = q[2 * VLX_WAVE];
+        k.pz = q[3 * VLX_WAVE];
+        k.k = q[4 * VLX_WAVE];
+        k.pax = NF > 5 ? q[5 * VLX_WAVE] : 0.0;
+        k.pay = NF > 5 ? q[6 * VLX_WAVE] : 0.0;
+        k.paz = NF > 5 ? q[7 * VLX_WAVE] : 0.0;
+        return k;
+    }
+};
+
 // FP64 quartet (all FP64 kernels); RS selects the erf(omega r)/r operator
 template <int la, int lb, int lc, int ld, bool RS = false>
 __device__ __forceinline__ void eri_quartet(const PrimPair* __restrict__ bra_prims, const int bra_np, const double ABx,
@@ -172,7 +183,7 @@ __device__ __forceinline__ void eri_quartet(const PrimPair* __restrict__ bra_pri
                                             const double* __restrict__ boys_tab, const double omega2,
                                             double* __restrict__ out)
 {
-    EriClass<la, lb, lc, ld>::template quartet<double, RS>(bra_prims, bra_np, ABx, ABy, ABz, ket_prims, ket_np, CDx, CDy,
+    EriClass<la, lb, lc, ld>::template quartet<double, RS, const PrimPair* __restrict__>(bra_prims, bra_np, ABx, ABy, ABz, ket_prims, ket_np, CDx, CDy,
                                                        CDz, boys_tab, omega2, out);
 }
 
@@ -224,10 +235,12 @@ __device__ __forceinline__ R wave_sum(R v)
     return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
 }
 
-template <typename R>
+// The class's Boys table from HBM into LDS: coefficient-major, or row-major as it is (ROWS).
+template <bool ROWS = false, typename R>
 __device__ __forceinline__ void stage_boys(R* lds, const R* __restrict__ tab)
 {
-    for (int t = threadIdx.x; t < BOYS_TAB_SIZE; t += blockDim.x) lds[t] = tab[t];
+    for (int t = threadIdx.x; t < BOYS_TAB_SIZE; t += blockDim.x)
+        lds[ROWS ? t : (t % BOYS_ROW) * BOYS_NGRID + t / BOYS_ROW] = tab[t];
     __syncthreads();
 }
 
@@ -831,30 +844,57 @@ __global__ void __launch_bounds__(NW * VLX_WAVE)
 }
 
 // LDS-tiled digestion.  A work-group takes one TileItem: bras of atom groups
-// (ga, gb) and up to 64 kets of groups (gc, gd).  Every F' contribution of
-// the item lands in six small dense tiles indexed by group-local AOs,
+// (ga, gb) and one or more 64-entry chunks of kets of groups (gc, gd).  Every F'
+// contribution of the item lands in six small dense tiles indexed by group-local AOs,
 //   J_AB, J_CD, K_AC, K_AD, K_BC, K_BD,
-// accumulated with LDS atomics and flushed to HBM once per item.  The four
-// wavefronts share the kets and split the bras.  MULTI: the item's integrals
+// accumulated with LDS atomics and flushed to HBM once per item.  S of the NW
+// wavefronts share a chunk and split its bras, so that every wavefront takes some eight bras or more
+// per chunk; the NW / S groups of wavefronts take the chunks in turn, without a barrier between them.
+// What an item costs beside its quartets (two barriers, the flush, its waves' wait for each other)
+// was over half of the time of the classes with few bras per segment when an item was one chunk.
+// MULTI: the item's integrals
 // are digested into a.ndens densities (layout and factors as in
 // fock_kernel_multi), with one set of six tiles per density in LDS.  DLDS: the
 // six D blocks the item reads (D_AB, D_CD, D_AC, D_AD, D_BC, D_BD, shapes of the
 // F' tiles) are staged in LDS after the F' tiles once per item, and every lane
 // reads D from there instead of gathering it from HBM (single density only).
-__device__ __forceinline__ void flush_tile(double* __restrict__ F, const int n, const double* __restrict__ tile,
+
+// Adds a tile to F' and clears it: a wavefront per row, the lanes along the columns.
+template <int NW>
+__device__ __forceinline__ void flush_tile(double* __restrict__ F, const int n, double* __restrict__ tile,
                                            const int nr, const int nc, const int* __restrict__ rows,
-                                           const int* __restrict__ cols, const double f)
+                                           const int* __restrict__ cols, const double f, const int wave, const int lane)
 {
-    for (int e = threadIdx.x; e < nr * nc; e += blockDim.x) {
-        const double v = tile[e];
-        if (v != 0.0) unsafeAtomicAdd(&F[(size_t)rows[e / nc] * n + cols[e % nc]], f * v);
+    for (int c = lane; c < nc; c += VLX_WAVE) {
+        const int col = cols[c];
+        for (int r = wave; r < nr; r += NW) {
+            const double v = tile[r * nc + c];
+            tile[r * nc + c] = 0.0;
+            if (v != 0.0) unsafeAtomicAdd(&F[(size_t)rows[r] * n + col], f * v);
+        }
     }
 }
 
+// Minimum over the wavefront.
+__device__ __forceinline__ int wave_min(int v)
+{
+    for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, VLX_WAVE));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+
+// Waves per SIMD the tiled kernel's registers are held to: 6 (80 VGPRs) for the classes in 12-wave
+// blocks; 2 (256 VGPRs) for the 4-wave classes that miss it by a few registers otherwise ((ds|ds) at
+// 260: 1.31 -> 0.86 ms on a 20-water def2-TZVP build) and spill next to nothing for it.
+constexpr int tiled_occupancy(int la, int lb, int lc, int ld, int nw)
+{
+    if (nw == 12) return 6;
+    return nw == 4 && (lc + ld == 0 || (lb + ld == 0 && la + lc <= 4)) ? 2 : 1;
+}
+
 template <int la, int lb, int lc, int ld, typename R, int NW, bool RS, bool MULTI = false, bool DLDS = false>
-__global__ void __launch_bounds__(NW * VLX_WAVE)
+__global__ void __launch_bounds__(NW * VLX_WAVE) __attribute__((amdgpu_waves_per_eu(tiled_occupancy(la, lb, lc, ld, NW))))
     fock_kernel_tiled(const PairInfo* __restrict__ pairs_bra, const PrimPair* __restrict__ bra_prims,
-                      const PairInfo* __restrict__ pairs_ket, const PrimPair* __restrict__ ket_prims,
+                      const PairInfo* __restrict__ pairs_ket, const double* __restrict__ ket_lanes,
                       const TileItem* __restrict__ items, const int2* __restrict__ kentries,
                       const R* __restrict__ boys_tab, const double* __restrict__ D0, double* __restrict__ F0,
                       const MolDesc* __restrict__ mols, const int* __restrict__ k32, const int* __restrict__ glim,
@@ -863,9 +903,13 @@ __global__ void __launch_bounds__(NW * VLX_WAVE)
 {
     constexpr int na = 2 * la + 1, nb = 2 * lb + 1, nc = 2 * lc + 1, nd = 2 * ld + 1;
     constexpr int nsph = na * nb * nc * nd;
+    constexpr int NF = vlx_ket_fields(lc, ld);
+    
     __shared__ R tab[BOYS_TAB_SIZE];
     extern __shared__ double tiles[];
-    stage_boys<R>(tab, boys_tab);
+    // the F' tiles are zero between items: cleared here, and again by every flush
+    for (int e = threadIdx.x; e < a.tile_doubles; e += NW * VLX_WAVE) tiles[e] = 0.0;
+    stage_boys(tab, boys_tab);
 
     const int lane = threadIdx.x & (VLX_WAVE - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / VLX_WAVE);
@@ -877,300 +921,284 @@ __global__ void __launch_bounds__(NW * VLX_WAVE)
         const double* __restrict__ D = D0 + md.base;
         double* __restrict__ F = F0 + md.base;
         const int n = md.nao;
-        // bras [b0, b1) of the item: all of them, or, with the precision split on the device, those
-        // whose bin plus the smallest ket bin of the item is below k32 (FP64 kernel) or not (FP32
-        // kernel).  The item's bras are sorted by bin, so the split is one point, found by bisection.
-        int b0 = ti.i0, b1 = ti.i1;
-        if (k32 != nullptr) {
-            const int lim = k32[ti.mol] - ti.bin_lo;  // FP32 from the first bra with bin >= lim
-            int lo = ti.i0, hi = ti.i1;
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (pairs_bra[mid].bin < lim) lo = mid + 1;
-                else hi = mid;
-            }
-            if (sizeof(R) == sizeof(double)) b1 = lo;
-            else b0 = lo;
-            if (b0 >= b1) continue;  // block-uniform: every thread skips the item together
-        }
         // density-weighted screening: every quartet of the item reads the D blocks of its four atom
         // groups, so the item has one bin-sum limit; bras past it (sorted by bin) are cut off
         int ilim = a.ithreshold;
-        if (glim != nullptr) {
-            int ql = quartet_bin_limit(glim, a.ngroups, ti.ga, ti.gb, ti.gc, ti.gd);
-            if (ti.gd2 >= 0) ql = max(ql, quartet_bin_limit(glim, a.ngroups, ti.ga, ti.gb, ti.gc, ti.gd2));
-            ilim = min(ilim, ql);
-            const int bl = ilim - ti.bin_lo;  // a bra needs bin <= bl for one quartet with the item's kets
-            int lo = b0, hi = b1;
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (pairs_bra[mid].bin <= bl) lo = mid + 1;
-                else hi = mid;
-            }
-            b1 = lo;
-            if (b0 >= b1) continue;  // block-uniform
-        }
+        if (glim != nullptr) ilim = min(ilim, quartet_bin_limit(glim, a.ngroups, ti.ga, ti.gb, ti.gc, ti.gd));
+        // smallest bin sum of the item: past the limit it has no quartet (block-uniform skip)
+        if (a.ithreshold >= 0 && pairs_bra[ti.i0].bin + ti.bin_lo > ilim) continue;
         const int nA = grp_n[ti.ga * 4 + la], nB = grp_n[ti.gb * 4 + lb];
-        const int nC = grp_n[ti.gc * 4 + lc];
-        // D groups: gd, and gd2 for the entries [jm, j1) of a chunk spanning two ket segments
-        const bool two = ti.gd2 >= 0;
-        const int nD0 = grp_n[ti.gd * 4 + ld], nD1 = two ? grp_n[ti.gd2 * 4 + ld] : 0;
-        // tiles of one density: J_AB, K_AC, K_BC, then per D group J_CD, K_AD, K_BD
-        const int nshared = nA * nB + nA * nC + nB * nC;
-        const int nseg0 = (nC + nA + nB) * nD0;
-        const int ntile = nshared + nseg0 + (nC + nA + nB) * nD1;
-        for (int e = threadIdx.x; e < nds * ntile; e += blockDim.x) tiles[e] = 0.0;
+        const int nC = grp_n[ti.gc * 4 + lc], nD = grp_n[ti.gd * 4 + ld];
+        // tiles of one density: J_AB, K_AC, K_BC, J_CD, K_AD, K_BD
+        const int dofs = nA * nB + nA * nC + nB * nC;
+        const int ntile = dofs + (nC + nA + nB) * nD;
         const int* ra = grp_ao + grp_off[ti.ga * 4 + la];
         const int* rb = grp_ao + grp_off[ti.gb * 4 + lb];
         const int* rc = grp_ao + grp_off[ti.gc * 4 + lc];
-        const int* rd0 = grp_ao + grp_off[ti.gd * 4 + ld];
-        const int* rd1 = two ? grp_ao + grp_off[ti.gd2 * 4 + ld] : rd0;
+        const int* rd = grp_ao + grp_off[ti.gd * 4 + ld];
         // D blocks in LDS (DLDS) after the F' tiles, in the same layout
-        double* dtiles = tiles + ntile;
-        if constexpr (DLDS) {
-            auto stage = [&](double* dst, const int* rows, const int nr, const int* cols, const int ncol) {
-                for (int x = threadIdx.x; x < nr * ncol; x += blockDim.x)
-                    dst[x] = D[(size_t)rows[x / ncol] * n + cols[x % ncol]];
-            };
-            stage(dtiles, ra, nA, rb, nB);
-            stage(dtiles + nA * nB, ra, nA, rc, nC);
-            stage(dtiles + nA * nB + nA * nC, rb, nB, rc, nC);
-            for (int sgi = 0; sgi < (two ? 2 : 1); sgi++) {
-                const int nDs = sgi ? nD1 : nD0;
-                const int* rds = sgi ? rd1 : rd0;
-                double* base = dtiles + nshared + (sgi ? nseg0 : 0);
-                stage(base, rc, nC, rds, nDs);
-                stage(base + nC * nDs, ra, nA, rds, nDs);
-                stage(base + nC * nDs + nA * nDs, rb, nB, rds, nDs);
-            }
-        }
-        __syncthreads();
-
-        // lane = a run of primitive pairs of one ket pair (first | count << 16):
-        // the contraction over the pair's runs happens in the LDS tiles (every
-        // step after the VRR is linear)
-        const int e = ti.j0 + lane;
-        const bool lane_ok = e < ti.j1;
-        const int esel = lane_ok ? e : ti.j0;
-        const int2 ke = kentries[esel];
-        const int kq0 = ke.y & 0xffff, kqn = ke.y >> 16;
-        const PairInfo kp = pairs_ket[ke.x];
-        // the lane's D group: the tiles J_CD, K_AD, K_BD (and D_CD, D_AD, D_BD) of its segment
-        const int sg = (two && esel >= ti.jm) ? 1 : 0;
-        const int nD = sg ? nD1 : nD0;
-        const int dofs = nshared + (sg ? nseg0 : 0);
+        double* dtiles = tiles + a.tile_doubles;
         const double* d_ab = dtiles;
         const double* d_ac = d_ab + nA * nB;
         const double* d_bc = d_ac + nA * nC;
         const double* d_cd = dtiles + dofs;
         const double* d_ad = d_cd + nC * nD;
         const double* d_bd = d_ad + nA * nD;
-        int r[nc], t[nd], rl[nc], tl[nd];
-#pragma unroll
-        for (int k = 0; k < nc; k++) {
-            r[k] = kp.ao_a + k * kp.str_a;
-            rl[k] = kp.loc_a + k;
+        if constexpr (DLDS) {
+            auto stage = [&](const double* dst, const int* rows, const int nr, const int* cols, const int ncol) {
+                for (int c = lane; c < ncol; c += VLX_WAVE) {
+                    const int col = cols[c];
+                    for (int r = wave; r < nr; r += NW) const_cast<double*>(dst)[r * ncol + c] = D[(size_t)rows[r] * n + col];
+                }
+            };
+            stage(d_ab, ra, nA, rb, nB);
+            stage(d_ac, ra, nA, rc, nC);
+            stage(d_bc, rb, nB, rc, nC);
+            stage(d_cd, rc, nC, rd, nD);
+            stage(d_ad, ra, nA, rd, nD);
+            stage(d_bd, rb, nB, rd, nD);
+            __syncthreads();
         }
-#pragma unroll
-        for (int l = 0; l < nd; l++) {
-            t[l] = kp.ao_b + l * kp.str_b;
-            tl[l] = kp.loc_b + l;
-        }
-        R dcd[nc][nd];
-        if constexpr (!MULTI) {
-#pragma unroll
-            for (int k = 0; k < nc; k++)
-#pragma unroll
-                for (int l = 0; l < nd; l++)
-                    dcd[k][l] = DLDS ? R(d_cd[rl[k] * nD + tl[l]]) : R(D[(size_t)r[k] * n + t[l]]);
-        }
-        // J_CD depends on the lane's ket only: small ket blocks accumulate it in
-        // registers over all bras of the item (one LDS atomic per element at the end)
-        constexpr bool jcd_in_regs = !MULTI && nc * nd <= 9;
-        double jcd[jcd_in_regs ? nc : 1][jcd_in_regs ? nd : 1];
-#pragma unroll
-        for (int k = 0; k < (jcd_in_regs ? nc : 1); k++)
-#pragma unroll
-            for (int l = 0; l < (jcd_in_regs ? nd : 1); l++) jcd[k][l] = 0.0;
+        // wavefronts per chunk: as few as leave each some eight bras, but no group without a chunk
+        const int nch = (ti.j1 - ti.j0) / VLX_WAVE;
+        int S = NW;
+        while (S > 1 && NW / S < nch && ti.i1 - ti.i0 < 8 * S) S >>= 1;
+        const int sub = wave % S;
 
-        for (int ib = b0 + wave; ib < b1; ib += NW) {
-            const PairInfo bp = pairs_bra[ib];
-            bool active = lane_ok;
-            if (a.ithreshold >= 0) active = active && (bp.bin + kp.bin <= ilim);
-            if (a.same_class) active = active && (bp.rank >= kp.rank);
-            R s = active ? R(1) : R(0);
-            if (bp.same) s *= R(0.5);
-            if (kp.same) s *= R(0.5);
-            if (a.same_class && bp.rank == kp.rank) s *= R(0.5);
-            R I[nsph];
-            EriClass<la, lb, lc, ld>::template quartet<R, RS>(bra_prims + bp.prim_start, bp.nprim, R(bp.abx), R(bp.aby),
-                                                          R(bp.abz), ket_prims + kp.prim_start + kq0, active ? kqn : 0,
-                                                          R(kp.abx), R(kp.aby), R(kp.abz), tab, R(a.omega2), I);
-#pragma unroll
-            // masked lanes contribute exact zeros: multiplying their integrals by s = 0 would turn
-            // a non-finite value left in a masked lane's registers into NaN (seen in the L = 5
-            // tiled kernels, depending on what ran before them)
-            for (int x = 0; x < nsph; x++) I[x] = active ? I[x] * s : R(0);
-            int p[na], q[nb];
-#pragma unroll
-            for (int i = 0; i < na; i++) p[i] = bp.ao_a + i * bp.str_a;
-#pragma unroll
-            for (int jb = 0; jb < nb; jb++) q[jb] = bp.ao_b + jb * bp.str_b;
-            for (int dd = 0; dd < nds; dd++) {
-                const double* __restrict__ Dd = MULTI ? D + dd * a.dstride : D;
-                double* t_jab = tiles + dd * ntile;
-                double* t_kac = t_jab + nA * nB;
-                double* t_kbc = t_kac + nA * nC;
-                double* t_jcd = tiles + dd * ntile + dofs;
-                double* t_kad = t_jcd + nC * nD;
-                double* t_kbd = t_kad + nA * nD;
-                const bool do_j = (MULTI ? dfac[2 * dd] : a.fj) != 0.0;
-                const bool do_k = (MULTI ? dfac[2 * dd + 1] : a.fk) != 0.0;
-                if constexpr (MULTI) {
-#pragma unroll
-                    for (int k = 0; k < nc; k++)
-#pragma unroll
-                        for (int l = 0; l < nd; l++) dcd[k][l] = R(Dd[(size_t)r[k] * n + t[l]]);
+        for (int ch = wave / S; ch < nch; ch += NW / S) {
+            // lane = a run of primitive pairs of one ket pair (first | count << 16; count 0: padding):
+            // the contraction over the pair's runs happens in the LDS tiles (every
+            // step after the VRR is linear)
+            const int e0 = ti.j0 + ch * VLX_WAVE;
+            const int2 ke = kentries[e0 + lane];
+            const int kqn = ke.y >> 16;
+            const bool lane_ok = kqn > 0;
+            const PairInfo kp = pairs_ket[ke.x];
+            const KetLane<NF> kprims{ket_lanes + (size_t)e0 * (a.ket_slots * NF) + lane};
+            // a chunk's entries go by bin: its first lane has the smallest
+            const int bin_lo = __builtin_amdgcn_readfirstlane(kp.bin);
+            const int blim = a.ithreshold >= 0 ? ilim - bin_lo : 0x7fffffff;
+            int b0 = ti.i0, b1 = ti.i1;
+            if (k32 != nullptr) {
+                // precision split on the device: FP32 from the first bra with bin >= lim (bras are
+                // sorted by bin, so the split is one point, found by bisection), FP64 before it
+                const int lim = k32[ti.mol] - bin_lo;
+                int lo = ti.i0, hi = ti.i1;
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (pairs_bra[mid].bin < lim) lo = mid + 1;
+                    else hi = mid;
                 }
-                if (do_j) {
-#pragma unroll
-                    for (int i = 0; i < na; i++)
-#pragma unroll
-                        for (int jb = 0; jb < nb; jb++) {
-                            R v = R(0);
-#pragma unroll
-                            for (int k = 0; k < nc; k++)
-#pragma unroll
-                                for (int l = 0; l < nd; l++) v = fma(I[((i * nb + jb) * nc + k) * nd + l], dcd[k][l], v);
-                            // row sums by DPP; the four rows meet in the tile through LDS atomics
-                            // (the LDS pipe has room where the VALU does not)
-                            v = row_sum(v);
-                            if ((lane & 15) == 0 && v != R(0))
-                                unsafeAtomicAdd(&t_jab[(bp.loc_a + i) * nB + bp.loc_b + jb], static_cast<double>(v));
-                        }
-                    if (jcd_in_regs || active) {
-                        R vcd[nc][nd];
-#pragma unroll
-                        for (int k = 0; k < nc; k++)
-#pragma unroll
-                            for (int l = 0; l < nd; l++) vcd[k][l] = R(0);
-#pragma unroll
-                        for (int i = 0; i < na; i++)
-#pragma unroll
-                            for (int jb = 0; jb < nb; jb++) {
-                                const R dab = DLDS ? R(d_ab[(bp.loc_a + i) * nB + bp.loc_b + jb])
-                                               : R(Dd[(size_t)p[i] * n + q[jb]]);
-#pragma unroll
-                                for (int k = 0; k < nc; k++)
-#pragma unroll
-                                    for (int l = 0; l < nd; l++)
-                                        vcd[k][l] = fma(I[((i * nb + jb) * nc + k) * nd + l], dab, vcd[k][l]);
-                            }
-                        if constexpr (jcd_in_regs) {
-                            // inactive lanes add zeros (their integrals were replaced by exact zeros)
-#pragma unroll
-                            for (int k = 0; k < nc; k++)
-#pragma unroll
-                                for (int l = 0; l < nd; l++) jcd[k][l] += static_cast<double>(vcd[k][l]);
-                        } else {
-#pragma unroll
-                            for (int k = 0; k < nc; k++)
-#pragma unroll
-                                for (int l = 0; l < nd; l++)
-                                    unsafeAtomicAdd(&t_jcd[rl[k] * nD + tl[l]], static_cast<double>(vcd[k][l]));
-                        }
-                    }
-                }
-                if (do_k && active) {
-#pragma unroll
-                    for (int i = 0; i < na; i++) {
-#pragma unroll
-                        for (int k = 0; k < nc; k++) {  // K_ac += I D_bd
-                            R v = R(0);
-#pragma unroll
-                            for (int jb = 0; jb < nb; jb++)
-#pragma unroll
-                                for (int l = 0; l < nd; l++)
-                                    v = fma(I[((i * nb + jb) * nc + k) * nd + l],
-                                            DLDS ? R(d_bd[(bp.loc_b + jb) * nD + tl[l]]) : R(Dd[(size_t)q[jb] * n + t[l]]),
-                                            v);
-                            unsafeAtomicAdd(&t_kac[(bp.loc_a + i) * nC + rl[k]], static_cast<double>(v));
-                        }
-#pragma unroll
-                        for (int l = 0; l < nd; l++) {  // K_ad += I D_bc
-                            R v = R(0);
-#pragma unroll
-                            for (int jb = 0; jb < nb; jb++)
-#pragma unroll
-                                for (int k = 0; k < nc; k++)
-                                    v = fma(I[((i * nb + jb) * nc + k) * nd + l],
-                                            DLDS ? R(d_bc[(bp.loc_b + jb) * nC + rl[k]]) : R(Dd[(size_t)q[jb] * n + r[k]]),
-                                            v);
-                            unsafeAtomicAdd(&t_kad[(bp.loc_a + i) * nD + tl[l]], static_cast<double>(v));
-                        }
-                    }
-#pragma unroll
-                    for (int jb = 0; jb < nb; jb++) {
-#pragma unroll
-                        for (int k = 0; k < nc; k++) {  // K_bc += I D_ad
-                            R v = R(0);
-#pragma unroll
-                            for (int i = 0; i < na; i++)
-#pragma unroll
-                                for (int l = 0; l < nd; l++)
-                                    v = fma(I[((i * nb + jb) * nc + k) * nd + l],
-                                            DLDS ? R(d_ad[(bp.loc_a + i) * nD + tl[l]]) : R(Dd[(size_t)p[i] * n + t[l]]),
-                                            v);
-                            unsafeAtomicAdd(&t_kbc[(bp.loc_b + jb) * nC + rl[k]], static_cast<double>(v));
-                        }
-#pragma unroll
-                        for (int l = 0; l < nd; l++) {  // K_bd += I D_ac
-                            R v = R(0);
-#pragma unroll
-                            for (int i = 0; i < na; i++)
-#pragma unroll
-                                for (int k = 0; k < nc; k++)
-                                    v = fma(I[((i * nb + jb) * nc + k) * nd + l],
-                                            DLDS ? R(d_ac[(bp.loc_a + i) * nC + rl[k]]) : R(Dd[(size_t)p[i] * n + r[k]]),
-                                            v);
-                            unsafeAtomicAdd(&t_kbd[(bp.loc_b + jb) * nD + tl[l]], static_cast<double>(v));
-                        }
-                    }
-                }
+                if (sizeof(R) == sizeof(double)) b1 = lo;
+                else b0 = lo;
             }
-        }
-        if constexpr (jcd_in_regs) {
-            if (a.fj != 0.0 && lane_ok) {
+            // the tiled bra and ket orders of one pair class are the same permutation (position =
+            // rank): bras before the chunk's lowest ket pair would run fully masked
+            if (a.same_class) b0 = max(b0, wave_min(ke.x));
+            int r[nc], t[nd], rl[nc], tl[nd];
+#pragma unroll
+            for (int k = 0; k < nc; k++) {
+                r[k] = kp.ao_a + k * kp.str_a;
+                rl[k] = kp.loc_a + k;
+            }
+#pragma unroll
+            for (int l = 0; l < nd; l++) {
+                t[l] = kp.ao_b + l * kp.str_b;
+                tl[l] = kp.loc_b + l;
+            }
+            R dcd[nc][nd];
+            if constexpr (!MULTI) {
 #pragma unroll
                 for (int k = 0; k < nc; k++)
 #pragma unroll
                     for (int l = 0; l < nd; l++)
-                        if (jcd[k][l] != 0.0) unsafeAtomicAdd(&tiles[dofs + rl[k] * nD + tl[l]], jcd[k][l]);
+                        dcd[k][l] = DLDS ? R(d_cd[rl[k] * nD + tl[l]]) : R(D[(size_t)r[k] * n + t[l]]);
+            }
+            // J_CD depends on the lane's ket only: small ket blocks accumulate it in
+            // registers over the wavefront's bras of the chunk (one LDS atomic per element at the end)
+            constexpr bool jcd_in_regs = !MULTI && nc * nd <= 9;
+            double jcd[jcd_in_regs ? nc : 1][jcd_in_regs ? nd : 1];
+#pragma unroll
+            for (int k = 0; k < (jcd_in_regs ? nc : 1); k++)
+#pragma unroll
+                for (int l = 0; l < (jcd_in_regs ? nd : 1); l++) jcd[k][l] = 0.0;
+
+            for (int ib = b0 + sub; ib < b1; ib += S) {
+                const PairInfo bp = pairs_bra[ib];
+                if (bp.bin > blim) break;  // bras go by bin (wave-uniform)
+                bool active = lane_ok;
+                if (a.ithreshold >= 0) active = active && (bp.bin + kp.bin <= ilim);
+                if (a.same_class) active = active && (bp.rank >= kp.rank);
+                R s = active ? R(1) : R(0);
+                if (bp.same) s *= R(0.5);
+                if (kp.same) s *= R(0.5);
+                if (a.same_class && bp.rank == kp.rank) s *= R(0.5);
+                R I[nsph];
+                EriClass<la, lb, lc, ld>::template quartet<R, RS>(
+                    bra_prims + bp.prim_start, bp.nprim, R(bp.abx), R(bp.aby), R(bp.abz), kprims, active ? kqn : 0,
+                    R(kp.abx), R(kp.aby), R(kp.abz), tab, R(a.omega2), I);
+#pragma unroll
+                // masked lanes contribute exact zeros: multiplying their integrals by s = 0 would turn
+                // a non-finite value left in a masked lane's registers into NaN (seen in the L = 5
+                // tiled kernels, depending on what ran before them)
+                for (int x = 0; x < nsph; x++) I[x] = active ? I[x] * s : R(0);
+                int p[na], q[nb];
+#pragma unroll
+                for (int i = 0; i < na; i++) p[i] = bp.ao_a + i * bp.str_a;
+#pragma unroll
+                for (int jb = 0; jb < nb; jb++) q[jb] = bp.ao_b + jb * bp.str_b;
+                for (int dd = 0; dd < nds; dd++) {
+                    const double* __restrict__ Dd = MULTI ? D + dd * a.dstride : D;
+                    double* t_jab = tiles + dd * ntile;
+                    double* t_kac = t_jab + nA * nB;
+                    double* t_kbc = t_kac + nA * nC;
+                    double* t_jcd = t_jab + dofs;
+                    double* t_kad = t_jcd + nC * nD;
+                    double* t_kbd = t_kad + nA * nD;
+                    const bool do_j = (MULTI ? dfac[2 * dd] : a.fj) != 0.0;
+                    const bool do_k = (MULTI ? dfac[2 * dd + 1] : a.fk) != 0.0;
+                    if constexpr (MULTI) {
+#pragma unroll
+                        for (int k = 0; k < nc; k++)
+#pragma unroll
+                            for (int l = 0; l < nd; l++) dcd[k][l] = R(Dd[(size_t)r[k] * n + t[l]]);
+                    }
+                    if (do_j) {
+#pragma unroll
+                        for (int i = 0; i < na; i++)
+#pragma unroll
+                            for (int jb = 0; jb < nb; jb++) {
+                                R v = R(0);
+#pragma unroll
+                                for (int k = 0; k < nc; k++)
+#pragma unroll
+                                    for (int l = 0; l < nd; l++) v = fma(I[((i * nb + jb) * nc + k) * nd + l], dcd[k][l], v);
+                                // row sums by DPP; the four rows meet in the tile through LDS atomics
+                                // (the LDS pipe has room where the VALU does not)
+                                v = row_sum(v);
+                                if ((lane & 15) == 0 && v != R(0))
+                                    unsafeAtomicAdd(&t_jab[(bp.loc_a + i) * nB + bp.loc_b + jb], static_cast<double>(v));
+                            }
+                        if (jcd_in_regs || active) {
+                            R vcd[nc][nd];
+#pragma unroll
+                            for (int k = 0; k < nc; k++)
+#pragma unroll
+                                for (int l = 0; l < nd; l++) vcd[k][l] = R(0);
+#pragma unroll
+                            for (int i = 0; i < na; i++)
+#pragma unroll
+                                for (int jb = 0; jb < nb; jb++) {
+                                    const R dab = DLDS ? R(d_ab[(bp.loc_a + i) * nB + bp.loc_b + jb])
+                                                   : R(Dd[(size_t)p[i] * n + q[jb]]);
+#pragma unroll
+                                    for (int k = 0; k < nc; k++)
+#pragma unroll
+                                        for (int l = 0; l < nd; l++)
+                                            vcd[k][l] = fma(I[((i * nb + jb) * nc + k) * nd + l], dab, vcd[k][l]);
+                                }
+                            if constexpr (jcd_in_regs) {
+                                // inactive lanes add zeros (their integrals were replaced by exact zeros)
+#pragma unroll
+                                for (int k = 0; k < nc; k++)
+#pragma unroll
+                                    for (int l = 0; l < nd; l++) jcd[k][l] += static_cast<double>(vcd[k][l]);
+                            } else {
+#pragma unroll
+                                for (int k = 0; k < nc; k++)
+#pragma unroll
+                                    for (int l = 0; l < nd; l++)
+                                        unsafeAtomicAdd(&t_jcd[rl[k] * nD + tl[l]], static_cast<double>(vcd[k][l]));
+                            }
+                        }
+                    }
+                    if (do_k && active) {
+#pragma unroll
+                        for (int i = 0; i < na; i++) {
+#pragma unroll
+                            for (int k = 0; k < nc; k++) {  // K_ac += I D_bd
+                                R v = R(0);
+#pragma unroll
+                                for (int jb = 0; jb < nb; jb++)
+#pragma unroll
+                                    for (int l = 0; l < nd; l++)
+                                        v = fma(I[((i * nb + jb) * nc + k) * nd + l],
+                                                DLDS ? R(d_bd[(bp.loc_b + jb) * nD + tl[l]]) : R(Dd[(size_t)q[jb] * n + t[l]]),
+                                                v);
+                                unsafeAtomicAdd(&t_kac[(bp.loc_a + i) * nC + rl[k]], static_cast<double>(v));
+                            }
+#pragma unroll
+                            for (int l = 0; l < nd; l++) {  // K_ad += I D_bc
+                                R v = R(0);
+#pragma unroll
+                                for (int jb = 0; jb < nb; jb++)
+#pragma unroll
+                                    for (int k = 0; k < nc; k++)
+                                        v = fma(I[((i * nb + jb) * nc + k) * nd + l],
+                                                DLDS ? R(d_bc[(bp.loc_b + jb) * nC + rl[k]]) : R(Dd[(size_t)q[jb] * n + r[k]]),
+                                                v);
+                                unsafeAtomicAdd(&t_kad[(bp.loc_a + i) * nD + tl[l]], static_cast<double>(v));
+                            }
+                        }
+#pragma unroll
+                        for (int jb = 0; jb < nb; jb++) {
+#pragma unroll
+                            for (int k = 0; k < nc; k++) {  // K_bc += I D_ad
+                                R v = R(0);
+#pragma unroll
+                                for (int i = 0; i < na; i++)
+#pragma unroll
+                                    for (int l = 0; l < nd; l++)
+                                        v = fma(I[((i * nb + jb) * nc + k) * nd + l],
+                                                DLDS ? R(d_ad[(bp.loc_a + i) * nD + tl[l]]) : R(Dd[(size_t)p[i] * n + t[l]]),
+                                                v);
+                                unsafeAtomicAdd(&t_kbc[(bp.loc_b + jb) * nC + rl[k]], static_cast<double>(v));
+                            }
+#pragma unroll
+                            for (int l = 0; l < nd; l++) {  // K_bd += I D_ac
+                                R v = R(0);
+#pragma unroll
+                                for (int i = 0; i < na; i++)
+#pragma unroll
+                                    for (int k = 0; k < nc; k++)
+                                        v = fma(I[((i * nb + jb) * nc + k) * nd + l],
+                                                DLDS ? R(d_ac[(bp.loc_a + i) * nC + rl[k]]) : R(Dd[(size_t)p[i] * n + r[k]]),
+                                                v);
+                                unsafeAtomicAdd(&t_kbd[(bp.loc_b + jb) * nD + tl[l]], static_cast<double>(v));
+                            }
+                        }
+                    }
+                }
+            }
+            if constexpr (jcd_in_regs) {
+                if (a.fj != 0.0 && lane_ok) {
+#pragma unroll
+                    for (int k = 0; k < nc; k++)
+#pragma unroll
+                        for (int l = 0; l < nd; l++)
+                            if (jcd[k][l] != 0.0) unsafeAtomicAdd(&tiles[dofs + rl[k] * nD + tl[l]], jcd[k][l]);
+                }
             }
         }
         __syncthreads();
         for (int dd = 0; dd < nds; dd++) {
             double* __restrict__ Fd = MULTI ? F + dd * a.dstride : F;
             const double fj = MULTI ? dfac[2 * dd] : a.fj, fk = MULTI ? dfac[2 * dd + 1] : a.fk;
-            const double* t_jab = tiles + dd * ntile;
-            const double* t_kac = t_jab + nA * nB;
-            const double* t_kbc = t_kac + nA * nC;
-            if (fj != 0.0) flush_tile(Fd, n, t_jab, nA, nB, ra, rb, fj);
-            if (fk != 0.0) {
-                flush_tile(Fd, n, t_kac, nA, nC, ra, rc, fk);
-                flush_tile(Fd, n, t_kbc, nB, nC, rb, rc, fk);
+            double* t_jab = tiles + dd * ntile;
+            double* t_kac = t_jab + nA * nB;
+            double* t_kbc = t_kac + nA * nC;
+            double* t_jcd = t_jab + dofs;
+            double* t_kad = t_jcd + nC * nD;
+            double* t_kbd = t_kad + nA * nD;
+            if (fj != 0.0) {
+                flush_tile<NW>(Fd, n, t_jab, nA, nB, ra, rb, fj, wave, lane);
+                flush_tile<NW>(Fd, n, t_jcd, nC, nD, rc, rd, fj, wave, lane);
             }
-            for (int sgi = 0; sgi < (two ? 2 : 1); sgi++) {
-                const int nDs = sgi ? nD1 : nD0;
-                const int* rds = sgi ? rd1 : rd0;
-                const double* t_jcd = tiles + dd * ntile + nshared + (sgi ? nseg0 : 0);
-                const double* t_kad = t_jcd + nC * nDs;
-                const double* t_kbd = t_kad + nA * nDs;
-                if (fj != 0.0) flush_tile(Fd, n, t_jcd, nC, nDs, rc, rds, fj);
-                if (fk != 0.0) {
-                    flush_tile(Fd, n, t_kad, nA, nDs, ra, rds, fk);
-                    flush_tile(Fd, n, t_kbd, nB, nDs, rb, rds, fk);
-                }
+            if (fk != 0.0) {
+                flush_tile<NW>(Fd, n, t_kac, nA, nC, ra, rc, fk, wave, lane);
+                flush_tile<NW>(Fd, n, t_kbc, nB, nC, rb, rc, fk, wave, lane);
+                flush_tile<NW>(Fd, n, t_kad, nA, nD, ra, rd, fk, wave, lane);
+                flush_tile<NW>(Fd, n, t_kbd, nB, nD, rb, rd, fk, wave, lane);
             }
         }
         __syncthreads();
@@ -1248,7 +1276,7 @@ __global__ void __launch_bounds__(VLX_BLOCK) diag_kernel(const DiagArgs a)
 // items).
 #define VLX_TILED_LAUNCH(la, lb, lc, ld, R, NW, RS, tab, MULTI, DLDS)                                   \
     hipLaunchKernelGGL((fock_kernel_tiled<la, lb, lc, ld, R, NW, RS, MULTI, DLDS>), dim3(grid),           \
-                       dim3((NW) * VLX_WAVE), a.tile_lds_bytes, s, a.bra, a.bra_prims, a.ket, a.ket_prims,   \
+                       dim3((NW) * VLX_WAVE), a.tile_lds_bytes, s, a.bra, a.bra_prims, a.ket, a.ket_lanes,   \
                        a.titems, a.kentries, tab, a.D, a.F, a.mols, a.k32, a.glim, a.grp_off, a.grp_n,      \
                        a.grp_ao, a.dfac, a.sc)
 #define VLX_INSTANTIATE_TILED(la, lb, lc, ld, NWB)                                                      \

@@ -152,10 +152,11 @@ def gen_class(la, lb, lc, ld):
     w(f'struct EriClass<{la}, {lb}, {lc}, {ld}> {{')
     # RS: erf(omega r)/r (range-separated) attenuation, a compile-time switch so
     # that plain Coulomb builds carry no per-primitive attenuation arithmetic
-    w('template <typename R, bool RS>')
+    # KP: where the ket primitives come from (a PrimPair array, or the lane's entry staged in LDS)
+    w('template <typename R, bool RS, typename KP>')
     w('static __device__ __forceinline__ void quartet(')
     w('    const PrimPair* __restrict__ bra_prims, const int bra_np, const R ABx, const R ABy, const R ABz,')
-    w('    const PrimPair* __restrict__ ket_prims, const int ket_np, const R CDx, const R CDy, const R CDz,')
+    w('    const KP ket_prims, const int ket_np, const R CDx, const R CDy, const R CDz,')
     w('    const R* __restrict__ boys_tab, const R omega2, R* __restrict__ out)')
     w('{')
     w(f'    R acc[{nacc}];')
@@ -295,8 +296,13 @@ def variant(la, lb, lc, ld, nlines):
 def tiled_waves(la, lb, lc, ld):
     """Waves per block of the tiled kernel: more waves share one set of LDS
     tiles where the integrals need few registers (the VGPR budget per lane is
-    512 / waves-per-SIMD)."""
+    512 / waves-per-SIMD).  12 where 80 VGPRs hold the recursion almost without spills: two blocks
+    are then resident on a CU (6 waves per SIMD) instead of one of 16 (4 per SIMD, 51% of the wave
+    cycles spent waiting); (ss|ss) 1.41 -> 1.15 ms, (ps|ss) 3.15 -> 2.83, (ds|ss) 1.37 -> 1.18 on a
+    20-water def2-TZVP build, while (ps|ps), (pp|ss) and (fs|ss) spill and lose."""
     L = la + lb + lc + ld
+    if lb + lc + ld == 0 and la <= 2:
+        return 12
     return 16 if L <= 2 else (8 if L == 3 else 4)
 
 

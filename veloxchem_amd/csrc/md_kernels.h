@@ -211,7 +211,7 @@ __device__ void quartet(const PrimPair* __restrict__ bra_prims, int bra_np, cons
             const double pq[3] = {bp.px - kp.px, bp.py - kp.py, bp.pz - kp.pz};
             if (threadIdx.x == 3) {
                 double F[L + 1];
-                boys_eval<L, double>(rho * (pq[0] * pq[0] + pq[1] * pq[1] + pq[2] * pq[2]), tab, F);
+                boys_eval<L, double, true>(rho * (pq[0] * pq[0] + pq[1] * pq[1] + pq[2] * pq[2]), tab, F);
                 for (int m = 0; m <= L; m++) scal[m] = F[m];
             }
             __syncthreads();
@@ -513,7 +513,7 @@ __global__ void __launch_bounds__(VLX_WAVE) __attribute__((amdgpu_waves_per_eu(4
                         }
                         const double pqx = pb.px - pk.px, pqy = pb.py - pk.py, pqz = pb.pz - pk.pz;
                         double Fm[L + 1];
-                        boys_eval<L, double>(rho * (pqx * pqx + pqy * pqy + pqz * pqz), boys_tab, Fm);
+                        boys_eval<L, double, true>(rho * (pqx * pqx + pqy * pqy + pqz * pqz), boys_tab, Fm);
                         // R levels n = L .. 0, ping-pong in rbuf; R^n_000 = w (-2 rho)^n F_n, lane n
                         // keeps level n's seed in LDS (the level loop then needs no register array)
                         {
@@ -661,7 +661,7 @@ __global__ void __launch_bounds__(VLX_WAVE) eri_out_kernel_md(const EriArgs a)
     __shared__ double work[S::lds];
     __shared__ double out[S::nsab * S::nscd];
     const double* tab = S::tab_in_lds ? tab_lds : a.boys_tab;
-    if constexpr (S::tab_in_lds) stage_boys(tab_lds, a.boys_tab);
+    if constexpr (S::tab_in_lds) stage_boys<true>(tab_lds, a.boys_tab);
     for (int qi = blockIdx.x; qi < a.nquartets; qi += gridDim.x) {
         const int2 qq = a.quartets[qi];
         const PairInfo bp = a.bra[qq.x];
@@ -683,7 +683,7 @@ __global__ void __launch_bounds__(VLX_WAVE) diag_kernel_md(const DiagArgs a)
     __shared__ double work[S::lds];
     __shared__ double out[S::nsab * S::nscd];
     const double* tab = S::tab_in_lds ? tab_lds : a.boys_tab;
-    if constexpr (S::tab_in_lds) stage_boys(tab_lds, a.boys_tab);
+    if constexpr (S::tab_in_lds) stage_boys<true>(tab_lds, a.boys_tab);
     for (int pi = blockIdx.x; pi < a.npairs; pi += gridDim.x) {
         const PairInfo pp = a.pairs[pi];
         const double abv[3] = {pp.abx, pp.aby, pp.abz};

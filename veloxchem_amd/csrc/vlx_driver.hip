@@ -65,6 +65,9 @@ constexpr int MAX_DEVICES = 64;
 double* g_scratch_ptr[MAX_DEVICES] = {};  // device address of `scratch` per device (set at context creation)
 std::mutex g_scratch_mutex;
 
+// LDS of a tiled block left for its tiles: the 160 KB of a CU less the FP64 Boys table (static) and 1 KB.
+constexpr int TILED_LDS_ROOM = 160 * 1024 - static_cast<int>(BOYS_TAB_SIZE * sizeof(double)) - 1024;
+
 int npair_classes() { return (VLX_GEN_LMAX + 1) * (VLX_GEN_LMAX + 2) / 2; }
 
 int pair_class_index(int la, int lb)  // la >= lb; order (0,0),(1,0),(1,1),(2,0),...
@@ -142,11 +145,16 @@ struct PairSet {
     };
     std::vector<Segment> segs;  // tiled order only: runs of equal (group A, group B)
     // tiled ket order: lane entries (pair, first primitive | count << 16) and the entry range
-    // of each segment, for runs of up to ket_prims primitives and for single primitives
+    // of each segment, for runs of up to ket_prims primitives and for single primitives.  Segments are
+    // padded to whole chunks of 64 entries (padding: count 0).  lanes: the entries' primitives, lane-transposed,
+    // [chunk][slot < slots][field < vlx_ket_fields][64]
     struct Entries {
+        int slots = 1;
         std::vector<int2> kentries;
         std::vector<int> seg_e0, seg_e1;
+        std::vector<double> lanes;
         DevView<int2> d_kentries;
+        DevView<double> d_lanes;
     };
     Entries runs, singles;
     // device copies of pairs, prims and both entry lists, in one allocation
@@ -238,6 +246,9 @@ struct BatchPlan {
 
 constexpr int BRA_CHUNK = 128;  // default upper bound of bras per work item
 
+// largest tiled item, in (bra, 64-entry ket chunk) units: its tiles' flush is then a small share
+constexpr long long TILE_ITEM_UNITS = 1024;
+
 constexpr int NSIDE = 4;  // side streams that run class kernels concurrently
 
 constexpr int NO_FP32 = 99;  // bin-sum threshold that sends no quartet to FP32
@@ -255,7 +266,7 @@ enum {
     VARIANT_TILED_WIDE_P1 = 5,
     VARIANT_KSL = 6,  // ket-stationary items with lane-private LDS accumulators (bra-stationary classes)
     VARIANT_TILED_DLDS = 7,  // tiled wide block with the item's D blocks staged in LDS
-    VARIANT_TILED_2SEG = 8,  // tiled wide block, chunks spanning two ket segments of one C group
+    VARIANT_TILED_2SEG = 8,  // accepted, runs as the wide tiled form
     NVARIANTS = 9
 };
 bool variant_tiled(int v)
@@ -291,6 +302,9 @@ struct vlx_context {
     // largest grid of a tiled launch, blocks striding over the items (VLX_TILED_GRID); 2048 measured
     // best on the 32-water build (42.2 builds/s against 41.7 at 4096 and 40.2 at 8192)
     int tiled_grid = 2048;
+    // tiled items a class aims at (VLX_TILE_ITEMS): 1024 / 2048 / 4096 / 8192 / 16384 measured 118.4 / 119.0 /
+    // 120.6 / 122.6 / 125.8 ms for a 20-water def2-TZVP build, 27.9 / 28.5 / 28.8 / 30.2 / 32.6 ms for 32-water def2-SVP
+    int tile_items = 1024;
     int untiled_wave_cap = 8192;  // largest wavefront count of an untiled launch (VLX_UNTILED_WAVES)
     // largest grid (one wavefront per block) of a matrix-core MD launch (VLX_MMD_GRID): on the 64-water
     // def2-TZVP build 16384 / 32768 / 65536 measured 0.775 / 0.786 / 0.793 builds/s
@@ -368,7 +382,9 @@ struct vlx_screener {
         int cls = -1, idx = -1, swapped = 0;
     };
     std::vector<PairRef> pair_ref;  // nshells x nshells -> position in all[]
-    std::map<int, std::vector<std::unique_ptr<ClassSchedule>>> schedules;  // by (ithreshold, FP32 bin-sum threshold)
+    // by (ithreshold, FP32 bin-sum threshold, forced variant) and the tiled items aimed at
+    std::map<std::pair<int, int>, std::vector<std::unique_ptr<ClassSchedule>>> schedules;
+    bool unscreened_ready = false;  // all_bra, all_tiled and all_tiled_bra are built on first use
     std::map<int, int> variant;  // class entry -> VARIANT_* chosen by vlx_fock_autotune
     std::map<int, double> tuned_ms;  // class entry -> its measured time (ms) under that variant
     DevBuf<double> d_faccum;  // F' of this screener's molecule in batched builds
@@ -566,27 +582,40 @@ void build_tiled(const vlx_screener& s, const PairSet& src, PairSet& ket, PairSe
         out.kentries.clear();
         out.seg_e0.clear();
         out.seg_e1.clear();
-        std::vector<long long> eoff(ket.size() + 1, 0);
-        for (int k = 0; k < ket.size(); k++) {
-            const int np = ket.pairs[k].nprim;
-            const int m = (np + pmax - 1) / pmax;
-            for (int t = 0, q = 0; t < m; t++) {
-                const int cnt = np / m + (t < np % m ? 1 : 0);
-                out.kentries.push_back(make_int2(k, q | (cnt << 16)));
-                q += cnt;
-            }
-            eoff[k + 1] = eoff[k] + m;
-        }
+        out.slots = 1;
+        std::vector<int2> seg;
         for (const auto& sg : ket.segs) {
-            const int e0 = static_cast<int>(eoff[sg.start]), e1 = static_cast<int>(eoff[sg.end]);
-            out.seg_e0.push_back(e0);
-            out.seg_e1.push_back(e1);
-            std::stable_sort(out.kentries.begin() + e0, out.kentries.begin() + e1,
-                             [&](const int2& x, const int2& y) {
-                                 const int bx = ket.pairs[x.x].bin, by = ket.pairs[y.x].bin;
-                                 if (bx != by) return bx < by;
-                                 return (x.y >> 16) > (y.y >> 16);
-                             });
+            seg.clear();
+            for (int k = sg.start; k < sg.end; k++) {
+                const int np = ket.pairs[k].nprim;
+                const int m = (np + pmax - 1) / pmax;
+                for (int t = 0, q = 0; t < m; t++) {
+                    const int cnt = np / m + (t < np % m ? 1 : 0);
+                    seg.push_back(make_int2(k, q | (cnt << 16)));
+                    out.slots = std::max(out.slots, cnt);
+                    q += cnt;
+                }
+            }
+            std::stable_sort(seg.begin(), seg.end(), [&](const int2& x, const int2& y) {
+                const int bx = ket.pairs[x.x].bin, by = ket.pairs[y.x].bin;
+                if (bx != by) return bx < by;
+                return (x.y >> 16) > (y.y >> 16);
+            });
+            out.seg_e0.push_back(static_cast<int>(out.kentries.size()));
+            out.kentries.insert(out.kentries.end(), seg.begin(), seg.end());
+            while (out.kentries.size() % VLX_WAVE != 0) out.kentries.push_back(make_int2(seg.back().x, 0));
+            out.seg_e1.push_back(static_cast<int>(out.kentries.size()));
+        }
+        const int nf = vlx_ket_fields(ket.la, ket.lb);
+        out.lanes.assign(out.kentries.size() * out.slots * nf, 0.0);
+        for (size_t e = 0; e < out.kentries.size(); e++) {
+            const int2 ke = out.kentries[e];
+            const PrimPair* p = &ket.prims[ket.pairs[ke.x].prim_start + (ke.y & 0xffff)];
+            double* dst = &out.lanes[(e / VLX_WAVE) * ((size_t)VLX_WAVE * out.slots * nf) + e % VLX_WAVE];
+            for (int t = 0; t < (ke.y >> 16); t++, dst += VLX_WAVE * nf) {
+                const double f[8] = {p[t].zeta, p[t].px, p[t].py, p[t].pz, p[t].k, p[t].pax, p[t].pay, p[t].paz};
+                for (int k = 0; k < nf; k++) dst[k * VLX_WAVE] = f[k];
+            }
         }
     };
     // runs of up to ket_prims primitives (they share a pair's contracted work: HRR,
@@ -617,12 +646,17 @@ int upload_set(PairSet& ps)
     const size_t b_pairs = up(ps.pairs.size() * sizeof(PairInfo)), b_prims = up(ps.prims.size() * sizeof(PrimPair));
     const size_t b_runs = up(ps.runs.kentries.size() * sizeof(int2));
     const size_t b_singles = up(ps.singles.kentries.size() * sizeof(int2));
-    HIP_TRY(ps.d_arena.alloc(b_pairs + b_prims + b_runs + b_singles));
+    const size_t b_rlanes = up(ps.runs.lanes.size() * sizeof(double));
+    const size_t b_slanes = up(ps.singles.lanes.size() * sizeof(double));
+    HIP_TRY(ps.d_arena.alloc(b_pairs + b_prims + b_runs + b_singles + b_rlanes + b_slanes));
     char* base = ps.d_arena.ptr;
     ps.d_pairs.ptr = reinterpret_cast<PairInfo*>(base);
     ps.d_prims.ptr = reinterpret_cast<PrimPair*>(base + b_pairs);
     ps.runs.d_kentries.ptr = b_runs ? reinterpret_cast<int2*>(base + b_pairs + b_prims) : nullptr;
     ps.singles.d_kentries.ptr = b_singles ? reinterpret_cast<int2*>(base + b_pairs + b_prims + b_runs) : nullptr;
+    char* lanes = base + b_pairs + b_prims + b_runs + b_singles;
+    ps.runs.d_lanes.ptr = b_rlanes ? reinterpret_cast<double*>(lanes) : nullptr;
+    ps.singles.d_lanes.ptr = b_slanes ? reinterpret_cast<double*>(lanes + b_rlanes) : nullptr;
     auto copy = [](void* dst, const void* src, size_t bytes) {
         return bytes ? hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) : hipSuccess;
     };
@@ -630,6 +664,8 @@ int upload_set(PairSet& ps)
     HIP_TRY(copy(ps.d_prims.ptr, ps.prims.data(), ps.prims.size() * sizeof(PrimPair)));
     HIP_TRY(copy(ps.runs.d_kentries.ptr, ps.runs.kentries.data(), ps.runs.kentries.size() * sizeof(int2)));
     HIP_TRY(copy(ps.singles.d_kentries.ptr, ps.singles.kentries.data(), ps.singles.kentries.size() * sizeof(int2)));
+    HIP_TRY(copy(ps.runs.d_lanes.ptr, ps.runs.lanes.data(), ps.runs.lanes.size() * sizeof(double)));
+    HIP_TRY(copy(ps.singles.d_lanes.ptr, ps.singles.lanes.data(), ps.singles.lanes.size() * sizeof(double)));
     return VLX_OK;
 }
 
@@ -752,16 +788,41 @@ __global__ void split_kernel(const double* __restrict__ d, double* __restrict__ 
     }
 }
 
+// The orders of the unscreened lists (every pair, bins ignored), built on the first unscreened build.
+int ensure_unscreened(vlx_screener* s)
+{
+    if (s->unscreened_ready) return VLX_OK;
+    for (size_t x = 0; x < s->all.size(); x++) {
+        PairSet& ps = s->all[x];
+        if (ps.size() == 0) continue;
+        std::vector<int> order(ps.size());
+        std::iota(order.begin(), order.end(), 0);
+        std::stable_sort(order.begin(), order.end(), [&](int i, int j) { return ps.shell_a[i] < ps.shell_a[j]; });
+        reorder_set(*s, ps, order, s->all_bra[x]);
+        build_tiled(*s, ps, s->all_tiled[x], s->all_tiled_bra[x]);
+        // the screener's creation uploaded `all` before its bins were known
+        for (PairSet* up : {&ps, &s->all_bra[x], &s->all_tiled[x], &s->all_tiled_bra[x]}) {
+            const int rc = upload_set(*up);
+            if (rc) return rc;
+        }
+    }
+    s->unscreened_ready = true;
+    return VLX_OK;
+}
+
 // Work items of every class at ithreshold.  k32 < NO_FP32 also splits the
 // tiled items: the bras of an item whose bin plus the smallest ket bin of
 // its chunk reaches k32 form an FP32 item (every quartet in it has
 // Schwarz bound < 10^(2 - k32)); the rest stay FP64.
 // create = false: only a schedule built earlier is returned (no host or device allocation);
 // without one the call fails.
+// share: the builds that run side by side in one launch (a batch's molecules), each aiming at its
+// share of the tiled items.
 int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_ptr<ClassSchedule>>** out,
-                  bool create = true)
+                  bool create = true, int share = 1)
 {
-    const int key = ((ithr + 1) * 128 + k32) * (NVARIANTS + 1) + (s->ctx->force_variant + 1);
+    const int tile_items = std::max(1, s->ctx->tile_items / share);
+    const std::pair<int, int> key{((ithr + 1) * 128 + k32) * (NVARIANTS + 1) + (s->ctx->force_variant + 1), tile_items};
     auto it = s->schedules.find(key);
     if (it != s->schedules.end()) {
         *out = &it->second;
@@ -773,6 +834,10 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
     std::vector<std::unique_ptr<ClassSchedule>> list;
     const int nentries = static_cast<int>(sizeof(g_class_table) / sizeof(g_class_table[0]));
     const bool unscreened = ithr < 0;
+    if (unscreened) {
+        const int rc = ensure_unscreened(s);
+        if (rc) return rc;
+    }
     for (int e = 0; e < nentries; e++) {
         const auto& ce = g_class_table[e];
         const PairSet& bra = unscreened ? s->all_bra[ce.x] : s->kept_bra[ce.x];
@@ -816,89 +881,73 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         }
         if (variant_tiled(var) && !can_tile) var = VARIANT_UNTILED;
         if (var == VARIANT_MMD && !ce.mmd) var = VARIANT_UNTILED;
+        if (var == VARIANT_TILED_2SEG) var = can_tile ? VARIANT_TILED_WIDE : VARIANT_UNTILED;
         if (var == VARIANT_KSL && !ce.ksl) var = VARIANT_UNTILED;
         // D tiles double the LDS of the F' tiles: beside the FP64 Boys table, or the plain wide tiles
         if (var == VARIANT_TILED_DLDS &&
-            (!ce.tiled_dlds || 2 * tile_lds > 160 * 1024 - static_cast<int>(BOYS_TAB_SIZE * sizeof(double)) - 1024))
+            (!ce.tiled_dlds || 2 * tile_lds > TILED_LDS_ROOM))
             var = VARIANT_TILED_WIDE;
-        // two D groups per chunk: the J_CD, K_AD and K_BD tiles twice
-        const int tile_lds2 = 8 * (gm[ce.la] * gm[ce.lb] + gm[ce.la] * gm[ce.lc] + gm[ce.lb] * gm[ce.lc] +
-                                   2 * (gm[ce.lc] + gm[ce.la] + gm[ce.lb]) * gm[ce.ld]);
-        if (var == VARIANT_TILED_2SEG && tile_lds2 > s->ctx->max_tile_lds) var = VARIANT_TILED_WIDE;
         if (ce.variant == VLX_WAVE_MD) var = VARIANT_MMD;  // no generated kernel
         sch->variant = var;
         sch->mmd = var == VARIANT_MMD;
         sch->ksl = var == VARIANT_KSL;
         sch->dlds = var == VARIANT_TILED_DLDS;
         if (variant_tiled(var)) {
-            // tiled items: (bra segment prefix, chunk of <= 64 kets of a ket segment)
             const PairSet& tb = unscreened ? s->all_tiled_bra[ce.x] : s->kept_tiled_bra[ce.x];
             const PairSet& tk = unscreened ? s->all_tiled[ce.y] : s->kept_tiled[ce.y];
             sch->tiled = true;
             sch->singles = var == VARIANT_TILED4_P1 || var == VARIANT_TILED_WIDE_P1;
             const PairSet::Entries& en = sch->singles ? tk.singles : tk.runs;
             sch->tiled_waves = (var == VARIANT_TILED4 || var == VARIANT_TILED4_P1) ? 4 : 0;
-            sch->tile_lds = var == VARIANT_TILED_2SEG ? tile_lds2 : tile_lds;
-            // chunks of <= 64 lane entries of one ket segment; with VARIANT_TILED_2SEG the last, partly
-            // filled chunk of a segment takes the first entries of the next segment when both have the
-            // same C group (their entry ranges are adjacent): {j0, j1, first segment, gd2, jm}
-            std::vector<std::array<int, 5>> chunks;
-            int open = -1;  // a one-segment chunk with room left
+            sch->tile_lds = tile_lds;
+            // bras of segment sb that a chunk of smallest bin `bin` meets: [start, start + count)
+            auto bras = [&](const PairSet::Segment& bs, int bin) {
+                if (unscreened) return bs.end - bs.start;
+                return ithr - bin < 0 ? 0 : bs.cnt_le[std::min(ithr - bin, NBINS - 1)];
+            };
+            auto bin_of = [&](int e) { return std::max(tk.pairs[en.kentries[e].x].bin, 0); };
+            // (bra, chunk) units of the class, and the units an item aims at: enough items for every
+            // CU, and no more, since every item flushes its tiles
+            long long units = 0;
+            for (size_t sk = 0; sk < tk.segs.size(); sk++)
+                for (int j = en.seg_e0[sk]; j < en.seg_e1[sk]; j += VLX_WAVE)
+                    for (size_t sb = same ? sk : 0; sb < tb.segs.size(); sb++) units += bras(tb.segs[sb], bin_of(j));
+            const long long target = std::max(1LL, std::min(TILE_ITEM_UNITS, units / tile_items));
             for (size_t sk = 0; sk < tk.segs.size(); sk++) {
-                int j = en.seg_e0[sk];
-                const int e1 = en.seg_e1[sk];
-                if (var == VARIANT_TILED_2SEG && open >= 0 && tk.segs[chunks[open][2]].ga == tk.segs[sk].ga &&
-                    chunks[open][1] == j) {
-                    auto& c = chunks[open];
-                    const int take = std::min(64 - (c[1] - c[0]), e1 - j);
-                    c[3] = tk.segs[sk].gb;
-                    c[4] = j;
-                    c[1] = j + take;
-                    j += take;
-                }
-                open = -1;
-                for (; j < e1; j += 64) {
-                    const int j1 = std::min(e1, j + 64);
-                    chunks.push_back({j, j1, static_cast<int>(sk), -1, j1});
-                    if (j1 - j < 64) open = static_cast<int>(chunks.size()) - 1;
-                }
-            }
-            for (const auto& ch : chunks) {
-                const size_t sk = static_cast<size_t>(ch[2]);
                 const auto& ks = tk.segs[sk];
-                const int j0 = ch[0], j1 = ch[1], gd2 = ch[3], jm = ch[4];
-                {
-                    int bin_lo = NBINS, kmin = en.kentries[j0].x;
-                    for (int j = j0; j < j1; j++) {
-                        bin_lo = std::min(bin_lo, std::max(tk.pairs[en.kentries[j].x].bin, 0));
-                        kmin = std::min(kmin, en.kentries[j].x);
-                    }
-                    const int lim = unscreened ? NBINS - 1 : ithr - bin_lo;
-                    if (lim < 0) continue;
-                    // same class: bra segments at or after the (first) ket segment (segment order is
-                    // identical in both lists); the diagonal segment is masked by rank
-                    for (size_t sb = same ? sk : 0; sb < tb.segs.size(); sb++) {
-                        const auto& bs = tb.segs[sb];
-                        int i0 = bs.start;
-                        const int i1 = bs.start + (unscreened ? bs.end - bs.start : bs.cnt_le[std::min(lim, NBINS - 1)]);
-                        // diagonal segment: the tiled bra and ket orders are the same permutation
-                        // (position = rank), so bras before the chunk's lowest ket pair have a lower
-                        // rank than every ket of the chunk and would run fully masked
-                        if (same && sb == sk) i0 = std::max(i0, kmin);
-                        if (i1 <= i0) continue;
-                        // bras [im, i1) have bin >= k32 - bin_lo: FP32 for every lane of the chunk
-                        int im = i1;
+                const int e0 = en.seg_e0[sk], e1 = en.seg_e1[sk];
+                // same class: bra segments at or after the ket segment (segment order is
+                // identical in both lists); the diagonal segment is masked by rank
+                for (size_t sb = same ? sk : 0; sb < tb.segs.size(); sb++) {
+                    const auto& bs = tb.segs[sb];
+                    for (int j0 = e0, j1; j0 < e1; j0 = j1) {
+                        const int bin_lo = bin_of(j0), nb = bras(bs, bin_lo);
+                        j1 = j0 + VLX_WAVE;
+                        if (nb == 0) break;  // later chunks of the segment have larger bins
+                        // bras [im, nb) have bin >= k32 - bin_lo: FP32 for every lane of the chunk
+                        // (one chunk an item, since the split is each chunk's own)
+                        int im = nb;
                         if (k32 < NO_FP32 && !unscreened) {
                             const int b = k32 - bin_lo - 1;
-                            im = (b < 0) ? i0 : std::min(i1, bs.start + bs.cnt_le[std::min(b, NBINS - 1)]);
-                            im = std::max(im, i0);
+                            im = (b < 0) ? 0 : std::min(nb, bs.cnt_le[std::min(b, NBINS - 1)]);
+                        } else {
+                            while (j1 < e1 && (long long)nb * ((j1 - j0) / VLX_WAVE + 1) <= target && bras(bs, bin_of(j1)) > 0)
+                                j1 += VLX_WAVE;
                         }
-                        if (im > i0) sch->titems.push_back({i0, im, j0, j1, bs.ga, bs.gb, ks.ga, ks.gb, 0, bin_lo, gd2, jm});
-                        if (i1 > im)
-                            sch->titems32.push_back({im, i1, j0, j1, bs.ga, bs.gb, ks.ga, ks.gb, 0, bin_lo, gd2, jm});
+                        // long bra ranges split where the class has few items otherwise
+                        const int step = static_cast<int>(std::max(std::min<long long>(target, nb), std::min(16LL, (long long)nb)));
+                        for (int i = 0; i < im; i += step)
+                            sch->titems.push_back({bs.start + i, bs.start + std::min(im, i + step), j0, j1, bs.ga, bs.gb,
+                                                   ks.ga, ks.gb, 0, bin_lo});
+                        if (nb > im)
+                            sch->titems32.push_back({bs.start + im, bs.start + nb, j0, j1, bs.ga, bs.gb, ks.ga, ks.gb, 0, bin_lo});
                     }
                 }
             }
+            // longest items first, so that the launch ends on short ones
+            auto units_of = [](const TileItem& t) { return (long long)(t.i1 - t.i0) * ((t.j1 - t.j0) / VLX_WAVE); };
+            std::stable_sort(sch->titems.begin(), sch->titems.end(),
+                             [&](const TileItem& x, const TileItem& y) { return units_of(x) > units_of(y); });
         } else if (!sch->mmd && (ce.variant == VLX_KET_STATIONARY || sch->ksl)) {
             // work items: 64 consecutive kets x a chunk of bras; the chunk shrinks
             // for classes with little work so that the launch still has enough items
@@ -947,21 +996,27 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         if (sch->tiled) {
             const PairSet& tb = unscreened ? s->all_tiled_bra[ce.x] : s->kept_tiled_bra[ce.x];
             const PairSet& tk = unscreened ? s->all_tiled[ce.y] : s->kept_tiled[ce.y];
-            // a chunk's lanes loop over the largest primitive count among its entries
+            // a chunk's lanes loop over the largest primitive count among its entries, over the bras
+            // its smallest bin allows
             const PairSet::Entries& en = sch->singles ? tk.singles : tk.runs;
-            auto kmax = [&](const TileItem& ti) {
-                int m = 1;
-                for (int j = ti.j0; j < ti.j1; j++) m = std::max(m, en.kentries[j].y >> 16);
-                return static_cast<long long>(m);
+            auto count = [&](const TileItem& ti, long long& prim_slots) {
+                for (int e0 = ti.j0; e0 < ti.j1; e0 += VLX_WAVE) {
+                    int kmax = 1, kmin = en.kentries[e0].x;
+                    for (int e = e0; e < e0 + VLX_WAVE; e++) {
+                        kmax = std::max(kmax, en.kentries[e].y >> 16);
+                        kmin = std::min(kmin, en.kentries[e].x);
+                    }
+                    const int lim = unscreened ? NBINS : ithr - tk.pairs[en.kentries[e0].x].bin;
+                    const int i1 = static_cast<int>(
+                        std::partition_point(tb.pairs.begin() + ti.i0, tb.pairs.begin() + ti.i1,
+                                             [&](const PairInfo& b) { return b.bin <= lim; }) - tb.pairs.begin());
+                    const int i0 = std::min(i1, same ? std::max(ti.i0, kmin) : ti.i0);
+                    sch->lane_slots += 64LL * (i1 - i0);
+                    prim_slots += (tb.nprim_prefix[i1] - tb.nprim_prefix[i0]) * 64 * kmax;
+                }
             };
-            for (const auto& ti : sch->titems) {
-                sch->lane_slots += 64LL * (ti.i1 - ti.i0);
-                sch->prim_slots += (tb.nprim_prefix[ti.i1] - tb.nprim_prefix[ti.i0]) * 64 * kmax(ti);
-            }
-            for (const auto& ti : sch->titems32) {
-                sch->lane_slots += 64LL * (ti.i1 - ti.i0);
-                sch->prim_slots32 += (tb.nprim_prefix[ti.i1] - tb.nprim_prefix[ti.i0]) * 64 * kmax(ti);
-            }
+            for (const auto& ti : sch->titems) count(ti, sch->prim_slots);
+            for (const auto& ti : sch->titems32) count(ti, sch->prim_slots32);
             sch->prim_slots += sch->prim_slots32;
         } else if (!sch->mmd) {
             // estimated cost of an item in FLOPs of one lane: primitive iterations times the
@@ -1090,11 +1145,11 @@ int vlx_context_create(int device, vlx_context** out)
     if (const char* e = std::getenv("VLX_BALANCE_ITEMS")) ctx->balance_items = std::atoi(e) != 0;
     if (const char* e = std::getenv("VLX_LAUNCH_ORDER")) ctx->launch_by_cost = std::atoi(e) != 0;
     if (const char* e = std::getenv("VLX_TILED_GRID")) ctx->tiled_grid = std::max(1, std::atoi(e));
+    if (const char* e = std::getenv("VLX_TILE_ITEMS")) ctx->tile_items = std::max(1, std::atoi(e));
     if (const char* e = std::getenv("VLX_MMD_GRID")) ctx->mmd_grid = std::max(1, std::atoi(e));
     if (const char* e = std::getenv("VLX_MMD_KETS")) ctx->mmd_kets = std::max(1, std::min(64, std::atoi(e)));
-    // dynamic LDS of a tiled block: the Boys table (static) and the tiles share the 160 KB of a CU
-    if (const char* e = std::getenv("VLX_MAX_TILE_LDS"))
-        ctx->max_tile_lds = std::max(16 * 1024, std::min(160 * 1024 - (int)(BOYS_TAB_SIZE * sizeof(double)), std::atoi(e)));
+    if (const char* e = std::getenv("VLX_MAX_TILE_LDS")) ctx->max_tile_lds = std::max(16 * 1024, std::atoi(e));
+    ctx->max_tile_lds = std::min(ctx->max_tile_lds, TILED_LDS_ROOM);
     if (const char* e = std::getenv("VLX_UNTILED_WAVES"))
         ctx->untiled_wave_cap = std::max(VLX_WAVES_PER_BLOCK, std::atoi(e));
     if (const char* e = std::getenv("VLX_SOLO_FRAC")) ctx->solo_frac = std::max(0.0, std::atof(e));
@@ -1473,17 +1528,10 @@ int vlx_screener_create(vlx_context* ctx, int nshells, const int* l, const int* 
             return ks.pairs[i].nprim < ks.pairs[j].nprim;
         });
         reorder_set(*s, ks, border, s->kept_bra[x]);
-        // unscreened lists: every pair, bins ignored
         for (int k = 0; k < ps.size(); k++) ps.pairs[k].rank = k;
         finalize_set(ps);
-        std::vector<int> aorder(ps.size());
-        std::iota(aorder.begin(), aorder.end(), 0);
-        std::stable_sort(aorder.begin(), aorder.end(), [&](int i, int j) { return ps.shell_a[i] < ps.shell_a[j]; });
-        reorder_set(*s, ps, aorder, s->all_bra[x]);
         build_tiled(*s, ks, s->kept_tiled[x], s->kept_tiled_bra[x]);
-        build_tiled(*s, ps, s->all_tiled[x], s->all_tiled_bra[x]);
-        for (PairSet* up : {&ps, &ks, &s->kept_bra[x], &s->all_bra[x], &s->kept_tiled[x], &s->all_tiled[x],
-                            &s->kept_tiled_bra[x], &s->all_tiled_bra[x]}) {
+        for (PairSet* up : {&ks, &s->kept_bra[x], &s->kept_tiled[x], &s->kept_tiled_bra[x]}) {
             rc = upload_set(*up);
             if (rc) return rc;
         }
@@ -1637,6 +1685,7 @@ int vlx_fock_autotune(vlx_context* ctx, vlx_screener* scr, const double* d_densi
     std::vector<double> g_ref(nn), g_var(nn);
     ctx->autotune_rejected = 0;
     for (int v = 0; v < NVARIANTS && rc == VLX_OK; v++) {
+        if (v == VARIANT_TILED_2SEG) continue;  // runs as VARIANT_TILED_WIDE
         ctx->force_variant = v;
         scr->schedules.clear();
         ctx->timing = false;
@@ -1780,7 +1829,7 @@ int vlx_fock_class_kernel(vlx_context* ctx, vlx_screener* scr, int ithreshold, i
         if (ce.la != la || ce.lb != lb || ce.lc != lc || ce.ld != ld) continue;
         if (sp->tiled) {
             const int L = la + lb + lc + ld;
-            const int wide = (L <= 2) ? 16 : (L == 3 ? 8 : 4);
+            const int wide = (L == la && la <= 2) ? 12 : (L <= 2 ? 16 : (L == 3 ? 8 : 4));
             // template arguments as the profiler prints them: <..., R, NW, RS, MULTI, DLDS>
             std::snprintf(name, len, "fock_kernel_tiled<%d,%d,%d,%d,double,%d,false,false,%s>", la, lb, lc, ld,
                           sp->tiled_waves == 4 ? 4 : wide, sp->dlds ? "true" : "false");
@@ -1881,6 +1930,9 @@ int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::
         a.grp_ao = scr->d_grp_ao.ptr;
         a.tile_lds_bytes = sch.tile_lds;
         a.tiled_waves = sch.tiled_waves;
+        a.ket_lanes = sch.singles ? ket.singles.d_lanes.ptr : ket.runs.d_lanes.ptr;
+        a.sc.ket_slots = sch.singles ? ket.singles.slots : ket.runs.slots;
+        a.sc.tile_doubles = sch.tile_lds / 8;
         a.sc.nitems = static_cast<long long>(sch.tiled ? sch.titems.size() : sch.items.size());
         a.sc.nket = ket.size();
         a.sc.ithreshold = ithreshold;
@@ -1941,7 +1993,7 @@ int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::
             } else if (sch.tiled) {
                 // one set of six tiles per density in LDS: as many densities per launch as fit
                 // beside the FP64 Boys table; the integrals are recomputed per group of densities
-                const int lds_max = 160 * 1024 - static_cast<int>(BOYS_TAB_SIZE * sizeof(double)) - 1024;
+                const int lds_max = TILED_LDS_ROOM;
                 const int chunk = std::max(1, std::min(ndens, lds_max / std::max(1, sch.tile_lds)));
                 for (int c0 = 0; c0 < ndens && !sch.titems.empty(); c0 += chunk) {
                     FockArgs am = a;
@@ -1950,6 +2002,7 @@ int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::
                     am.F = F + c0 * nn;
                     am.dfac = dfac + 2 * c0;
                     am.tile_lds_bytes = am.sc.ndens * sch.tile_lds;
+                    am.sc.tile_doubles = am.tile_lds_bytes / 8;
                     ce.tiled_multi(am, grid, st);
                 }
             } else if (sch.mmd) {
@@ -2205,6 +2258,17 @@ __global__ void batch_k32_kernel(const unsigned long long* __restrict__ dmax, in
     k32[m] = k;
 }
 
+// Appends one molecule's lane-transposed entry primitives to a concatenated set of `slots` slots.
+void append_lanes(const PairSet::Entries& src, PairSet::Entries& dst, int slots, int nf)
+{
+    dst.slots = slots;
+    const size_t from = (size_t)VLX_WAVE * src.slots * nf, to = (size_t)VLX_WAVE * slots * nf;
+    for (size_t at = 0; at < src.lanes.size(); at += from) {
+        dst.lanes.insert(dst.lanes.end(), src.lanes.begin() + at, src.lanes.begin() + at + from);
+        dst.lanes.resize(dst.lanes.size() + to - from, 0.0);
+    }
+}
+
 // Concatenated pair lists, moved items and packed layout of a batch (see BatchPlan).
 int build_batch_plan(vlx_context* ctx, BatchPlan& P)
 {
@@ -2213,7 +2277,7 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
     const bool unscreened = P.ithreshold < 0;
     std::vector<std::vector<std::unique_ptr<ClassSchedule>>*> lists(nmol, nullptr);
     for (int m = 0; m < nmol; m++) {
-        const int rc = get_schedules(P.scrs[m], P.ithreshold, NO_FP32, &lists[m]);
+        const int rc = get_schedules(P.scrs[m], P.ithreshold, NO_FP32, &lists[m], true, nmol);
         if (rc) return rc;
     }
     // the four orders of every pair class, and each molecule's offsets in them
@@ -2248,6 +2312,12 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
         goff[m] = ngroups;
         ngroups += P.scrs[m]->ngroups;
     }
+    // primitive slots per lane entry of the concatenated runs: the widest molecule's
+    std::vector<int> runs_slots(npc, 1);
+    for (int m = 0; m < nmol; m++) {
+        const std::vector<PairSet>& v = sets_of(P.scrs[m], TKET);
+        for (int c = 0; c < std::min(npc, static_cast<int>(v.size())); c++) runs_slots[c] = std::max(runs_slots[c], v[c].runs.slots);
+    }
     for (int c = 0; c < npc; c++)
         for (int k = 0; k < NKIND; k++) {
             PairSet& dst = (*dst_sets[k])[c];
@@ -2274,6 +2344,9 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
                     eoff_singles[m * npc + c] = static_cast<int>(dst.singles.kentries.size());
                     for (int2 e : src.runs.kentries) dst.runs.kentries.push_back(make_int2(e.x + pair0, e.y));
                     for (int2 e : src.singles.kentries) dst.singles.kentries.push_back(make_int2(e.x + pair0, e.y));
+                    // chunks of fewer slots than the widest molecule's keep their order, slots padded
+                    append_lanes(src.runs, dst.runs, runs_slots[c], vlx_ket_fields(src.la, src.lb));
+                    append_lanes(src.singles, dst.singles, 1, vlx_ket_fields(src.la, src.lb));
                 }
             }
             finalize_set(dst);
@@ -2347,8 +2420,6 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
                         ti.gb += goff[m];
                         ti.gc += goff[m];
                         ti.gd += goff[m];
-                        if (ti.gd2 >= 0) ti.gd2 += goff[m];
-                        ti.jm += eo;
                         ti.mol = m;
                         L->titems.push_back(ti);
                     }
@@ -2449,6 +2520,9 @@ int record_batch(vlx_context* ctx, BatchPlan& P)
         a.grp_ao = P.d_grp_ao.ptr;
         a.tile_lds_bytes = L.tile_lds;
         a.tiled_waves = L.tiled_waves;
+        a.ket_lanes = L.singles ? ket.singles.d_lanes.ptr : ket.runs.d_lanes.ptr;
+        a.sc.ket_slots = L.singles ? ket.singles.slots : ket.runs.slots;
+        a.sc.tile_doubles = L.tile_lds / 8;
         a.boys_tab = ctx->d_boys.ptr + (size_t)(ce.la + ce.lb + ce.lc + ce.ld) * BOYS_TAB_SIZE;
         a.boys_tab_f = ctx->d_boys_f.ptr + (size_t)(ce.la + ce.lb + ce.lc + ce.ld) * BOYS_TAB_SIZE;
         a.D = P.d_D.ptr;

@@ -43,16 +43,15 @@ struct alignas(16) PairInfo {
     double abx, aby, abz;  // A - B
 };
 
-// Tiled Fock work: bras [i0, i1) of atom groups (ga, gb) against ket
-// primitive entries [j0, j1) (at most 64, one per lane) of atom groups (gc, gd),
-// of molecule `mol` of the launch (MolDesc).  bin_lo is the smallest Schwarz
-// bin of the item's kets (the precision split on the device, FockArgs::k32).
-// A chunk may span two ket segments with the same C group: entries [jm, j1)
-// then belong to D group gd2 (gd2 = -1 and jm = j1 for one segment).
+// Tiled Fock work: bras [i0, i1) of atom groups (ga, gb) against the ket
+// primitive entries [j0, j1) of atom groups (gc, gd), one or more whole chunks of
+// 64 (one entry per lane), of molecule `mol` of the launch (MolDesc).  bin_lo is
+// the smallest Schwarz bin of the item's kets; every chunk meets the bras its own
+// smallest bin allows.
 struct TileItem {
     int i0, i1, j0, j1;
     int ga, gb, gc, gd;
-    int mol, bin_lo, gd2, jm;
+    int mol, bin_lo;
 };
 
 // One unit of Fock work: kets [j0, j0 + 64) of the ket list (one per lane,
@@ -85,6 +84,8 @@ struct FockScalars {
     int ndens;                     // densities digested per quartet (multi-density kernels; 0 or 1: one)
     int det;                       // 1: deterministic fixed-point accumulation (multi-density and MD kernels)
     int bs_layout;                 // multi-density kernel: 1 bra-stationary work items, 0 ket-stationary
+    int ket_slots;                 // tiled kernel: primitive slots per lane entry (longest run)
+    int tile_doubles;              // tiled kernel: doubles of the F' tiles in the dynamic LDS
     int pad_sc;
     long long dstride;             // elements between consecutive densities (and F' accumulators)
 };
@@ -97,6 +98,7 @@ struct FockArgs {
     const WorkItem* items;
     const TileItem* titems;        // tiled variant
     const int2* kentries;          // tiled variant: (ket pair, first primitive | count << 16) per lane
+    const double* ket_lanes;       // tiled variant: the entries' primitives, [chunk][slot][field][lane]
     const int* grp_off;            // (ngroups x 4): offset of the (group, l) AO list in grp_ao
     const int* grp_n;              // (ngroups x 4): number of AOs in the (group, l) block
     const int* grp_ao;             // global AO index of each local AO
@@ -117,6 +119,10 @@ struct FockArgs {
                                    // bin + bin_lo < k32, the FP32 kernel the others)
     FockScalars sc;
 };
+
+// Doubles per ket primitive in the tiled kernel's lane-transposed layout (P - A only where the
+// recursion uses it).
+__host__ __device__ constexpr int vlx_ket_fields(int lc, int ld) { return lc + ld > 0 ? 8 : 5; }
 
 // Hermite functions of total degree <= l, and the padded U array of a pair
 // class (la, lb) of the matrix-core MD kernel: rows = Hermite index, columns
