@@ -288,10 +288,13 @@ struct vlx_context {
     std::map<int, int> tuned_variant;  // class entry -> VARIANT_* of the last autotune (default for new screeners)
     int autotune_rejected = 0;      // bit v: variant v's G failed the last autotune's check (never chosen)
     // atoms per group of the tiled kernels (VLX_GROUP_ATOMS); 0: the largest of 12, 8, 6, 4, 3,
-    // 2, 1 whose (ps|ss) tiles fit max_tile_lds (12 for def2-SVP waters, 8 for def2-TZVP)
+    // 2, 1 whose (pp|pp) tiles fit max_tile_lds (waters: 12 for def2-SVP, 8 for def2-TZVP, 6 for
+    // def2-SVPD).  A class whose tiles do not fit runs untiled, several times slower: 13 waters,
+    // def2-SVPD, one stream: 127 ms in groups of 12 atoms, 58 of 8, 53 of 6, 61 of 4; the sparser
+    // def2-SVP (32 waters) wants large groups: 26 ms of 12, 37 of 8, 51 of 6
     int group_atoms = 0;
     int tiled_waves = 0;            // 4: 4-wave blocks for every tiled class; 0: per-class default (VLX_TILED_WAVES)
-    int max_tile_lds = 96 * 1024;   // larger tiles fall back to the untiled kernel
+    int max_tile_lds = TILED_LDS_ROOM;  // larger tiles fall back to the untiled kernel (VLX_MAX_TILE_LDS)
     // primitives of one ket pair per lane of the tiled kernels (VLX_KET_PRIMS, 1..16): a ket
     // pair of n primitives takes ceil(n / ket_prims) lanes with near-equal shares
     int ket_prims = 3;
@@ -1374,18 +1377,16 @@ int vlx_screener_create(vlx_context* ctx, int nshells, const int* l, const int* 
         }
         for (int g : {12, 8, 6, 4, 3, 2, 1}) {
             group_atoms = g;
-            int gm0 = 0, gm1 = 0;
+            long long most = 0;  // s or p functions of a group
             for (size_t a0 = 0; a0 < per_atom.size(); a0 += g) {
-                int n0 = 0, n1 = 0;
+                long long n0 = 0, n1 = 0;
                 for (size_t a = a0; a < std::min(per_atom.size(), a0 + g); a++) {
                     n0 += per_atom[a][0];
                     n1 += per_atom[a][1];
                 }
-                gm0 = std::max(gm0, n0);
-                gm1 = std::max(gm1, n1);
+                most = std::max(most, std::max(n0, n1));
             }
-            // tiles of (ps|ss): AB, AC, AD = p x s; CD, BC, BD = s x s
-            if (8LL * (3LL * gm1 * gm0 + 3LL * gm0 * gm0) <= ctx->max_tile_lds) break;
+            if (8 * 6 * most * most <= ctx->max_tile_lds) break;  // six tiles of (pp|pp)
         }
     }
     s->group_atoms = group_atoms;
