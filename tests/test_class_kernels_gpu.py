@@ -1,0 +1,67 @@
+"""Tiled kernels, both digestions of the matrix-core kernel and the default choice between them,
+against the untiled kernels, at the edges of their work items."""
+import numpy as np
+import pytest
+
+from veloxchem_amd import FockDriver, Matrices, MolecularBasis, T4CScreener, _native, make_matrix, mat_t
+from veloxchem_amd.workloads import pseudo_density, water_cluster
+
+pytestmark = pytest.mark.gpu
+
+EPS = np.finfo(float).eps
+
+
+@pytest.mark.parametrize('waters, basis, label, omega, ithreshold', [
+    (1, 'def2-svp', '2jk', 0.0, 12),      # one atom group, chunks of a few kets, one molecule's latency
+    (1, 'def2-tzvp', '2jkx', 0.0, -1),    # no screening, f shells, every rank of the same-class pairs
+    (3, 'def2-svpd', 'k', 0.0, 12),       # several groups of 6 atoms, the last one of 3
+    (5, 'def2-svp', 'j', 0.0, 10),        # 12 + 3 atoms, J tiles only
+    (5, 'def2-svp', 'kx_rs', 0.4, 12),    # attenuated exchange
+    (6, 'def2-tzvp', '2jk', 0.0, 12),     # (pp|pp) chunks past 64 entries, items of several chunks
+])
+def test_class_kernels_agree(waters, basis, label, omega, ithreshold):
+    mol = water_cluster(waters, 6.0, 3)
+    bas = MolecularBasis.read(mol, basis)
+    scr = T4CScreener()
+    scr.partition(bas, mol, 'eri')
+    n = bas.get_dimensions_of_basis()
+    D = pseudo_density(n, 5 * waters, seed=9)
+    mats = {}
+    drv, ctx, lib = FockDriver(), _native.context(), _native.lib()
+    # an element sums up to n^2 products I D in an order of each kernel's own; the rounding errors of
+    # n^2 terms are independent, so they grow as n eps on each side
+    try:
+        for v in (0, -1, 1, 2, 3, 4, 5):
+            _native.check(lib.vlx_context_set_variant(ctx, v))
+            mats[v] = np.asarray(drv.compute(scr, D, label, 0.5, omega, ithreshold))
+    finally:
+        _native.check(lib.vlx_context_set_variant(ctx, -1))
+    tol = 2 * n * EPS * max(1.0, np.max(np.abs(mats[0])))
+    for v, g in mats.items():
+        assert np.isfinite(g).all(), v
+        assert np.max(np.abs(g - mats[0])) <= tol, (v, np.max(np.abs(g - mats[0])), tol)
+
+
+def test_direct_digestion_of_matrix_core_classes():
+    """Two densities in one call digest directly; each is the single build (LDS tiles)."""
+    mol = water_cluster(2, 6.0, 3)
+    bas = MolecularBasis.read(mol, 'def2-tzvp')
+    scr = T4CScreener()
+    scr.partition(bas, mol, 'eri')
+    n = bas.get_dimensions_of_basis()
+    dens = [pseudo_density(n, 10, seed=s) for s in (1, 2)]
+    drv, ctx, lib = FockDriver(), _native.context(), _native.lib()
+    try:
+        _native.check(lib.vlx_context_set_variant(ctx, 3))
+        ms = Matrices()
+        for i, d in enumerate(dens):
+            m = make_matrix(bas, mat_t.symmetric)
+            m.set_values(d)
+            ms.add(m, str(i))
+        out = drv.compute(scr, ms, ['2jk', 'k'], 0.0, 0.0, 12)
+        for i, lab in enumerate(['2jk', 'k']):
+            one = np.asarray(drv.compute(scr, dens[i], lab, 0.0, 0.0, 12))
+            g = out.matrix(str(i)).to_numpy()
+            assert np.max(np.abs(g - one)) <= 2 * n * EPS * max(1.0, np.max(np.abs(one)))
+    finally:
+        _native.check(lib.vlx_context_set_variant(ctx, -1))

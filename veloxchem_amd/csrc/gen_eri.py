@@ -358,7 +358,8 @@ def main(outdir, lmax):
         variants[(la, lb, lc, ld)] = var
         if var == 'md':
             src = ['// generated by gen_eri.py -- do not edit', '#include "../md_kernels.h"', '',
-                   f'VLX_INSTANTIATE_MD_CLASS({la}, {lb}, {lc}, {ld})']
+                   f'VLX_INSTANTIATE_MD_CLASS({la}, {lb}, {lc}, {ld})',
+                   f'VLX_INSTANTIATE_MMD_TILED({la}, {lb}, {lc}, {ld})']
             if (la, lb) == (lc, ld):
                 src.append(f'VLX_INSTANTIATE_MD_DIAG({la}, {lb})')
         else:
@@ -371,6 +372,7 @@ def main(outdir, lmax):
                 src.append(f'VLX_INSTANTIATE_KSL({la}, {lb}, {lc}, {ld}, {ksl_waves(la, lb, lc, ld, var)})')
             if mmd_eligible(la, lb, lc, ld, var):
                 src.append(f'VLX_INSTANTIATE_MMD({la}, {lb}, {lc}, {ld})')
+                src.append(f'VLX_INSTANTIATE_MMD_TILED({la}, {lb}, {lc}, {ld})')
             if (la, lb) == (lc, ld):
                 src.append(f'VLX_INSTANTIATE_DIAG({la}, {lb})')
             if tiled_eligible(la, lb, lc, ld):
@@ -392,6 +394,8 @@ def main(outdir, lmax):
             d.append(f'VLX_DECLARE_TILED({la}, {lb}, {lc}, {ld})')
         if mmd_eligible(la, lb, lc, ld, variants[(la, lb, lc, ld)]) and variants[(la, lb, lc, ld)] != 'md':
             d.append(f'VLX_DECLARE_MMD({la}, {lb}, {lc}, {ld})')
+        if mmd_eligible(la, lb, lc, ld, variants[(la, lb, lc, ld)]):
+            d.append(f'VLX_DECLARE_MMD_TILED({la}, {lb}, {lc}, {ld})')
         if (la, lb) == (lc, ld):
             d.append(f'VLX_DECLARE_DIAG({la}, {lb})')
     d.append('static const ClassLaunchers g_class_table[] = {')
@@ -411,8 +415,10 @@ def main(outdir, lmax):
         tlm = f'&launch_tiled_multi_{la}{lb}{lc}{ld}' if has_tiled else 'nullptr'
         ksl = f'&launch_ksl_{la}{lb}{lc}{ld}' if ksl_waves(la, lb, lc, ld, var) else 'nullptr'
         tld = f'&launch_tiled_dlds_{la}{lb}{lc}{ld}' if has_tiled else 'nullptr'
+        mmt = (f'&launch_mmd_tiled_{la}{lb}{lc}{ld}, &mmd_scratch_{la}{lb}{lc}{ld}'
+               if mmd_eligible(la, lb, lc, ld, var) else 'nullptr, nullptr')
         d.append(f'    {{{x}, {y}, {la}, {lb}, {lc}, {ld}, {nv}, {nh}, {ks}, &launch_fock_{la}{lb}{lc}{ld}, '
-                 f'&launch_eri_{la}{lb}{lc}{ld}, {tl}, {tl32}, {mm}, {fm}, {tlm}, {ksl}, {tld}}},')
+                 f'&launch_eri_{la}{lb}{lc}{ld}, {tl}, {tl32}, {mm}, {fm}, {tlm}, {ksl}, {tld}, {mmt}}},')
     d.append('};')
     d.append('static const DiagLauncher g_diag_table[] = {')
     for (la, lb) in pcs:

@@ -275,68 +275,6 @@ __device__ void quartet(const PrimPair* __restrict__ bra_prims, int bra_np, cons
     __syncthreads();
 }
 
-// Fock digestion of one block in LDS (factor s included), lanes over outputs.
-template <int la, int lb, int lc, int ld, bool DET = false>
-__device__ void digest(const PairInfo& bp, const PairInfo& kp, double s, const double* __restrict__ out,
-                       const double* __restrict__ D, double* __restrict__ F, const int n, const double fj,
-                       const double fk)
-{
-    using S = Sizes<la, lb, lc, ld>;
-    constexpr int na = S::nsa, nb = S::nsb, nc = S::nsc, nd = S::nsd;
-    auto I = [&](int i, int j, int k, int l) { return out[(i * nb + j) * S::nscd + k * nd + l]; };
-    auto P = [&](int i) { return bp.ao_a + i * bp.str_a; };
-    auto Q = [&](int j) { return bp.ao_b + j * bp.str_b; };
-    auto R = [&](int k) { return kp.ao_a + k * kp.str_a; };
-    auto T = [&](int l) { return kp.ao_b + l * kp.str_b; };
-    const int lane = threadIdx.x;
-    if (fj != 0.0) {
-        for (int e = lane; e < na * nb; e += blockDim.x) {
-            const int i = e / nb, j = e % nb;
-            double v = 0.0;
-            for (int k = 0; k < nc; k++)
-                for (int l = 0; l < nd; l++) v = fma(I(i, j, k, l), D[(size_t)R(k) * n + T(l)], v);
-            acc_add<DET>(F, (size_t)P(i) * n + Q(j), fj * s * v);
-        }
-        for (int e = lane; e < nc * nd; e += blockDim.x) {
-            const int k = e / nd, l = e % nd;
-            double v = 0.0;
-            for (int i = 0; i < na; i++)
-                for (int j = 0; j < nb; j++) v = fma(I(i, j, k, l), D[(size_t)P(i) * n + Q(j)], v);
-            acc_add<DET>(F, (size_t)R(k) * n + T(l), fj * s * v);
-        }
-    }
-    if (fk != 0.0) {
-        for (int e = lane; e < na * nc; e += blockDim.x) {  // F'_ac += I D_bd
-            const int i = e / nc, k = e % nc;
-            double v = 0.0;
-            for (int j = 0; j < nb; j++)
-                for (int l = 0; l < nd; l++) v = fma(I(i, j, k, l), D[(size_t)Q(j) * n + T(l)], v);
-            acc_add<DET>(F, (size_t)P(i) * n + R(k), fk * s * v);
-        }
-        for (int e = lane; e < na * nd; e += blockDim.x) {  // F'_ad += I D_bc
-            const int i = e / nd, l = e % nd;
-            double v = 0.0;
-            for (int j = 0; j < nb; j++)
-                for (int k = 0; k < nc; k++) v = fma(I(i, j, k, l), D[(size_t)Q(j) * n + R(k)], v);
-            acc_add<DET>(F, (size_t)P(i) * n + T(l), fk * s * v);
-        }
-        for (int e = lane; e < nb * nc; e += blockDim.x) {  // F'_bc += I D_ad
-            const int j = e / nc, k = e % nc;
-            double v = 0.0;
-            for (int i = 0; i < na; i++)
-                for (int l = 0; l < nd; l++) v = fma(I(i, j, k, l), D[(size_t)P(i) * n + T(l)], v);
-            acc_add<DET>(F, (size_t)Q(j) * n + R(k), fk * s * v);
-        }
-        for (int e = lane; e < nb * nd; e += blockDim.x) {  // F'_bd += I D_ac
-            const int j = e / nd, l = e % nd;
-            double v = 0.0;
-            for (int i = 0; i < na; i++)
-                for (int k = 0; k < nc; k++) v = fma(I(i, j, k, l), D[(size_t)P(i) * n + R(k)], v);
-            acc_add<DET>(F, (size_t)Q(j) * n + T(l), fk * s * v);
-        }
-    }
-}
-
 }  // namespace md
 
 // ------------------------------------------------------------------------
@@ -346,15 +284,23 @@ __device__ void digest(const PairInfo& bp, const PairInfo& kp, double s, const d
 // per screener (u_build_kernel) and stored in HBM as
 //   U[prim][h][s] = k sum_{cart a, b} S_a S_b E^x E^y E^z
 // (h < nherm(la + lb) Hermite index, s < (2la+1)(2lb+1) spherical index, both
-// padded to multiples of 16 with zeros).  One wavefront takes one shell
-// quartet at a time; per primitive quartet it builds R^0[tuv] (scaled by
-// 1/sqrt(zeta + eta)) in LDS and runs two FP64 matrix-core products
-//   X[p][cd]    = sum_q (-1)^{|q|} R^0[p + q] U_CD[q][cd]       (v_mfma_f64_16x16x4)
+// padded to multiples of 16 with zeros; a ket's U carries the sign (-1)^|h|).  One
+// wavefront takes one shell quartet at a time; per primitive quartet it builds
+// R^0[tuv] (scaled by 1/sqrt(zeta + eta)) in LDS and runs two FP64 matrix-core products
+//   X[p][cd]    = sum_q R^0[p + q] U_CD[q][cd]                   (v_mfma_f64_16x16x4)
 //   out[ab][cd] += sum_p U_AB[p][ab] X[p][cd]
-// one 16-wide cd tile at a time; out stays in the matrix-core accumulators
-// over all primitive quartets of the shell quartet.  Operand layouts of
-// v_mfma_f64_16x16x4f64 (wave64): A[i][k] in lane i + 16k, B[k][j] in lane
-// j + 16k, D[i][j] in register i / 4 of lane j + 16 (i % 4).
+// Operand layouts of v_mfma_f64_16x16x4f64 (wave64): A[i][k] in lane i + 16k, B[k][j] in lane
+// j + 16k, D[i][j] in register i / 4 of lane j + 16 (i % 4).  So register r of X's row tile m is, in
+// every lane, the B operand of the second product's step 4m + r: X never leaves the registers.  The
+// byte offset of R^0[p + q] of every step of the first product is a constant of the lane, computed
+// once per wavefront and kept packed in registers, as are the steps of the R recursion and the
+// operands of the digestion.
+//
+// Digestion: the six F' blocks' elements, each with the D block it contracts, are dealt to the lanes
+// in order of their number of terms (146 elements in three rounds of 35, 21 and 15 terms for (fd|dp)),
+// instead of one block after another with 15 to 35 of 64 lanes at work.  An element's F' address is
+// also the address of the D element that the lane fetches, at the quartet's start, behind the
+// integrals.
 
 using md::hidx;
 using md::nherm;
@@ -424,24 +370,301 @@ template <int la, int lb, int lc, int ld>
 struct MmdSizes {
     static constexpr int L = la + lb + lc + ld;
     static constexpr int nhab = nherm(la + lb), nhcd = nherm(lc + ld), nr = nherm(L);
-    static constexpr int nsab = (2 * la + 1) * (2 * lb + 1), nscd = (2 * lc + 1) * (2 * ld + 1);
+    static constexpr int na = 2 * la + 1, nb = 2 * lb + 1, nc = 2 * lc + 1, nd = 2 * ld + 1;
+    static constexpr int nsab = na * nb, nscd = nc * nd;
     static constexpr int HA = vlx_u_rows(la, lb), SA = vlx_u_cols(la, lb);  // bra U: HA x SA
     static constexpr int HC = vlx_u_rows(lc, ld), SC = vlx_u_cols(lc, ld);  // ket U: HC x SC
-    static constexpr int MT = SA / 16, NT = SC / 16, MX = HA / 16;
+    static constexpr int MT = SA / 16, NT = SC / 16, MX = (nhab + 15) / 16;
     static constexpr int KX = (nhcd + 3) / 4, KO = (nhab + 3) / 4;
-    static constexpr int XC = MX < 2 ? MX : 2;  // X row tiles per chunk
-    // operands preloaded into registers: the X product's U_CD column when its K loop is short,
-    // and the whole U_AB operand of the out product when one chunk covers all its K steps
-    static constexpr bool PRE_X = KX <= 8;
-    static constexpr bool PRE_O = MX <= XC && KO * MT <= 16;
+    static constexpr int KR = (nr + VLX_WAVE - 1) / VLX_WAVE;  // entries of R^0 per lane
+    // X summed over the ket primitives before the second product, where its tiles fit in registers
+    static constexpr bool XSUM = MX * NT <= 6;
+    // U_CD operands of a primitive quartet fetched ahead of the R recursion
+    static constexpr bool PRE_X = KX * NT <= 12;
+    // elements of the six blocks AB, CD, AC, AD, BC, BD and rounds of the digestion
+    static constexpr int nout = nsab + nscd + (na + nb) * (nc + nd);
+    static constexpr int NR = (nout + VLX_WAVE - 1) / VLX_WAVE;
+    // estimated VGPRs, for the occupancy the registers are held to
+    static constexpr int regs = 8 * MT * NT + 8 * MX * (XSUM ? NT : 1) + MX * KX / 2 + 5 * KR + 2 * (L + 1) + 8 * NR +
+                                (PRE_X ? 2 * KX * NT : 8) + 40;
+    static constexpr int occupancy = regs <= 128 ? 4 : regs <= 170 ? 3 : regs <= 256 ? 2 : 1;
 };
 
-// Work item {j0, i0, i1}: bra i0 with kets [j0, i1), one shell quartet at a time.  With
-// a.ndens > 1 each block is digested into every density (density d at D0 + d * dstride, its F' at
+// Digestion of one shell quartet over the lanes: element o (in order of decreasing term count) of the
+// six blocks.  Element (x, y) of block X sums I[..] over the elements (u, v) of its partner block
+// (AB with CD, AC with BD, AD with BC): I offset x sx + y sy + u su + v sv, partner element u nv + v.
+template <int la, int lb, int lc, int ld>
+struct MmdDigest {
+    using S = MmdSizes<la, lb, lc, ld>;
+    struct Tab {
+        int ib[S::nout];     // byte offset of the first integral | of the partner block in LDS << 16
+        int step[S::nout];   // byte step of v | steps of v per u << 16 | terms << 24
+        int wrap[S::nout];   // extra byte step after nv steps | LDS slot of the element's D << 16
+        int addr[S::nout];   // row shell | row component << 2 | column shell << 5 | column component << 7 | Coulomb << 10
+        int terms[S::NR];    // most terms of a round
+    };
+    static constexpr Tab make()
+    {
+        Tab t{};
+        constexpr int n[4] = {S::na, S::nb, S::nc, S::nd};
+        constexpr int st[4] = {S::nb * S::nc * S::nd, S::nc * S::nd, S::nd, 1};
+        constexpr int blk[6][2] = {{0, 1}, {2, 3}, {0, 2}, {0, 3}, {1, 2}, {1, 3}};
+        constexpr int partner[6] = {1, 0, 5, 4, 3, 2};
+        int base[6] = {}, used[6] = {};
+        for (int b = 1; b < 6; b++) base[b] = base[b - 1] + n[blk[b - 1][0]] * n[blk[b - 1][1]];
+        int o = 0;
+        for (int k = 0; k < 6; k++) {
+            int best = -1, most = -1;
+            for (int b = 0; b < 6; b++) {
+                const int terms = n[blk[partner[b]][0]] * n[blk[partner[b]][1]];
+                if (!used[b] && terms > most) best = b, most = terms;
+            }
+            used[best] = 1;
+            const int x = blk[best][0], y = blk[best][1], u = blk[partner[best]][0], v = blk[partner[best]][1];
+            for (int i = 0; i < n[x]; i++)
+                for (int j = 0; j < n[y]; j++, o++) {
+                    t.ib[o] = 8 * (i * st[x] + j * st[y]) | (8 * base[partner[best]]) << 16;
+                    t.step[o] = 8 * st[v] | n[v] << 16 | most << 24;
+                    t.wrap[o] = 8 * (st[u] - n[v] * st[v]) | (base[best] + i * n[y] + j) << 16;
+                    t.addr[o] = x | i << 2 | y << 5 | j << 7 | (best < 2 ? 1 << 10 : 0);
+                    if (most > t.terms[o / VLX_WAVE]) t.terms[o / VLX_WAVE] = most;
+                }
+        }
+        return t;
+    }
+};
+template <int la, int lb, int lc, int ld>
+static __device__ constexpr typename MmdDigest<la, lb, lc, ld>::Tab g_mmd_digest = MmdDigest<la, lb, lc, ld>::make();
+
+// Orders the LDS accesses of the one wavefront of a block for the compiler; the hardware executes
+// the LDS instructions of a wavefront in order.
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ double lds_at(const double* __restrict__ base, const int byte)
+{
+    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + byte);
+}
+
+constexpr int VLX_DIGEST_UNROLL = 5;  // terms of the digestion loaded together (term counts are odd)
+
+// What a lane of the MD kernels keeps for the whole launch.
+template <int la, int lb, int lc, int ld>
+struct MmdLane {
+    using S = MmdSizes<la, lb, lc, ld>;
+    // byte offsets of R^0[p + q], two steps (row tile, column group) a register; masked rows and
+    // columns read R^0[0] against zero rows of U
+    unsigned ridx[(S::MX * S::KX + 1) / 2];
+    // the lane's entries of the R recursion: byte offsets of the two sources, factor and axis
+    unsigned rsrc[S::KR];
+    double rfac[S::KR];
+    int raxis[S::KR];
+    // the lane's elements of the digestion
+    int gib[S::NR], gstep[S::NR], gwrap[S::NR], gaddr[S::NR];
+
+    __device__ __forceinline__ void init(const int lane)
+    {
+        static_assert(8 * S::nr < 65536 && 8 * S::nsab * S::nscd < 65536, "LDS byte offsets pack into 16 bits");
+        const int lr = lane & 15, lk = lane >> 4;
+#pragma unroll
+        for (int e = 0; e < (S::MX * S::KX + 1) / 2; e++) ridx[e] = 0;
+#pragma unroll
+        for (int e = 0; e < S::MX * S::KX; e++) {
+            const int p = 16 * (e / S::KX) + lr, q = 4 * (e % S::KX) + lk;
+            const int tuv = g_herm.e[min(p, S::nhab - 1)] + g_herm.e[min(q, S::nhcd - 1)];
+            const unsigned off = (p < S::nhab && q < S::nhcd) ? 8u * hidx_packed(tuv) : 0u;
+            ridx[e / 2] |= off << (16 * (e & 1));
+        }
+#pragma unroll
+        for (int k = 0; k < S::KR; k++) {
+            const int rr = g_hrec.e[min(lane + VLX_WAVE * k, S::nr - 1)];
+            rsrc[k] = 8u * (rr & 511) | 8u * ((rr >> 9) & 511) << 16;
+            raxis[k] = (rr >> 18) & 3;
+            rfac[k] = static_cast<double>(rr >> 20);
+        }
+#pragma unroll
+        for (int k = 0; k < S::NR; k++) {
+            const int o = lane + VLX_WAVE * k;
+            const bool ok = o < S::nout;
+            gib[k] = ok ? g_mmd_digest<la, lb, lc, ld>.ib[o] : 0;
+            gstep[k] = ok ? g_mmd_digest<la, lb, lc, ld>.step[o] : 0;
+            gwrap[k] = ok ? g_mmd_digest<la, lb, lc, ld>.wrap[o] : 0;
+            gaddr[k] = ok ? g_mmd_digest<la, lb, lc, ld>.addr[o] : 0;
+        }
+    }
+    // element k of the digestion in D and F' (elements past the last: 0)
+    __device__ __forceinline__ size_t place(const int k, const int lane, const PairInfo& bp, const PairInfo& kp,
+                                            const int nao) const
+    {
+        const int x = gaddr[k] & 3, i = (gaddr[k] >> 2) & 7, y = (gaddr[k] >> 5) & 3, j = (gaddr[k] >> 7) & 7;
+        const int row = x == 0 ? bp.ao_a + i * bp.str_a : x == 1 ? bp.ao_b + i * bp.str_b : kp.ao_a + i * kp.str_a;
+        const int col = y == 1 ? bp.ao_b + j * bp.str_b : y == 2 ? kp.ao_a + j * kp.str_a : kp.ao_b + j * kp.str_b;
+        return lane + VLX_WAVE * k < S::nout ? (size_t)row * nao + col : 0;
+    }
+    // element k's sum over its terms: integrals in outs, the six D blocks in dblk
+    __device__ __forceinline__ double sum(const int k, const int terms, const double* __restrict__ outs,
+                                          const double* __restrict__ dblk) const
+    {
+        const int step = gstep[k] & 0xffff, nv = (gstep[k] >> 16) & 0xff, wrap = gwrap[k] & 0xffff;
+        int io = gib[k] & 0xffff, dof = gib[k] >> 16, c = 0;
+        double v = 0.0;
+        for (int t = 0; t < terms; t += VLX_DIGEST_UNROLL) {
+            double x[VLX_DIGEST_UNROLL], d[VLX_DIGEST_UNROLL];
+            // loads of several terms in flight; past the last one they repeat it
+#pragma unroll
+            for (int q = 0; q < VLX_DIGEST_UNROLL; q++) {
+                x[q] = lds_at(outs, io);
+                d[q] = lds_at(dblk, dof);
+                const bool more = t + q + 1 < terms, end = c + 1 == nv;
+                dof += more ? 8 : 0;
+                io += more ? step + (end ? wrap : 0) : 0;
+                c = end ? 0 : c + 1;
+            }
+#pragma unroll
+            for (int q = 0; q < VLX_DIGEST_UNROLL; q++) v = t + q < terms ? fma(x[q], d[q], v) : v;
+        }
+        return v;
+    }
+};
+
+// Contracted spherical block (ab|cd) of one shell quartet by one wavefront, into outs[ab][cd] (LDS).
+// rbuf: R^n for even n in the first nr doubles, odd n in the second.
+template <int la, int lb, int lc, int ld, bool RS>
+__device__ __forceinline__ void mmd_block(const MmdLane<la, lb, lc, ld>& ln, const int lane, const PairInfo& bp,
+                                          const PairInfo& kp, const PrimPair* __restrict__ bra_prims,
+                                          const double* __restrict__ bra_u, const PrimPair* __restrict__ ket_prims,
+                                          const double* __restrict__ ket_u, const double* __restrict__ boys_tab,
+                                          const double omega2, double* __restrict__ rbuf, double* __restrict__ outs)
+{
+    using S = MmdSizes<la, lb, lc, ld>;
+    constexpr int L = S::L, MX = S::MX, KX = S::KX, MT = S::MT, NT = S::NT, KR = S::KR;
+    const int lr = lane & 15, lk = lane >> 4;
+    vlx_d4 acc[NT][MT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int m = 0; m < MT; m++) acc[nt][m] = vlx_d4{0.0, 0.0, 0.0, 0.0};
+    for (int ib = 0; ib < bp.nprim; ib++) {
+        const PrimPair pb = bra_prims[bp.prim_start + ib];
+        const double* ua = bra_u + (size_t)(bp.prim_start + ib) * (S::HA * S::SA) + lk * S::SA + lr;
+        vlx_d4 x[S::XSUM ? NT : 1][MX];
+        auto clear_x = [&](vlx_d4 (&t)[MX]) {
+#pragma unroll
+            for (int m = 0; m < MX; m++) t[m] = vlx_d4{0.0, 0.0, 0.0, 0.0};
+        };
+        // out[ab][cd] += sum_p U_AB[p][ab] X[p][cd] of column tile nt
+        auto out_product = [&](const vlx_d4 (&t)[MX], vlx_d4 (&o)[MT]) {
+#pragma unroll
+            for (int kp2 = 0; kp2 < S::KO; kp2++) {
+#pragma unroll
+                for (int ms = 0; ms < MT; ms++)
+                    o[ms] = __builtin_amdgcn_mfma_f64_16x16x4f64(ua[4 * kp2 * S::SA + 16 * ms], t[kp2 / 4][kp2 % 4],
+                                                                o[ms], 0, 0, 0);
+            }
+        };
+        if constexpr (S::XSUM) {
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) clear_x(x[nt]);
+        }
+        for (int ik = 0; ik < kp.nprim; ik++) {
+            const PrimPair pk = ket_prims[kp.prim_start + ik];
+            const double* uc = ket_u + (size_t)(kp.prim_start + ik) * (S::HC * S::SC) + lk * S::SC + lr;
+            double ucv[S::PRE_X ? NT : 1][S::PRE_X ? KX : 1];
+            if constexpr (S::PRE_X) {
+#pragma unroll
+                for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+                    for (int kq = 0; kq < KX; kq++) ucv[nt][kq] = uc[4 * kq * S::SC + 16 * nt];
+            }
+            const double sz = pb.zeta + pk.zeta;
+            const double rho_c = pb.zeta * pk.zeta * vrcp<double>(sz);
+            double rho = rho_c, w = vrsqrt<double>(sz);
+            if constexpr (RS) {
+                const double sfac = omega2 / (omega2 + rho_c);
+                rho = rho_c * sfac;
+                w *= sqrt(sfac);
+            }
+            const double pqx = pb.px - pk.px, pqy = pb.py - pk.py, pqz = pb.pz - pk.pz;
+            double seed[L + 1];
+            boys_eval<L, double, true>(rho * (pqx * pqx + pqy * pqy + pqz * pqz), boys_tab, seed);
+            // R^n_000 = w (-2 rho)^n F_n
+            {
+                double f = w;
+#pragma unroll
+                for (int n = 0; n <= L; n++) {
+                    seed[n] *= f;
+                    f *= -2.0 * rho;
+                }
+            }
+            double pq[KR];
+#pragma unroll
+            for (int k = 0; k < KR; k++) pq[k] = ln.raxis[k] == 0 ? pqx : (ln.raxis[k] == 1 ? pqy : pqz);
+            // R levels n = L .. 0, one FMA and one product per entry
+            if (lane == 0) rbuf[(L & 1) * S::nr] = seed[L];
+#pragma unroll
+            for (int n = L - 1; n >= 0; n--) {
+                wave_lds_fence();
+                const double* prev = rbuf + ((n + 1) & 1) * S::nr;
+                double* cur = rbuf + (n & 1) * S::nr;
+#pragma unroll
+                for (int k = 0; VLX_WAVE * k < nherm(L - n); k++) {
+                    const int idx = lane + VLX_WAVE * k;
+                    if (idx < nherm(L - n)) {
+                        const double v1 = lds_at(prev, ln.rsrc[k] & 0xffff), v2 = lds_at(prev, ln.rsrc[k] >> 16);
+                        const double val = fma(ln.rfac[k], v2, pq[k] * v1);
+                        cur[idx] = idx == 0 ? seed[n] : val;
+                    }
+                }
+            }
+            wave_lds_fence();
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) {
+                vlx_d4 (&t)[MX] = x[S::XSUM ? nt : 0];
+                if constexpr (!S::XSUM) clear_x(t);
+#pragma unroll
+                for (int kq = 0; kq < KX; kq++) {
+                    double bv;
+                    if constexpr (S::PRE_X) bv = ucv[nt][kq];
+                    else bv = uc[4 * kq * S::SC + 16 * nt];
+#pragma unroll
+                    for (int m = 0; m < MX; m++) {
+                        const int e = m * KX + kq;
+                        const double av = lds_at(rbuf, (e & 1) ? ln.ridx[e / 2] >> 16 : ln.ridx[e / 2] & 0xffff);
+                        t[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, t[m], 0, 0, 0);
+                    }
+                }
+                if constexpr (!S::XSUM) out_product(t, acc[nt]);
+            }
+            wave_lds_fence();
+        }
+        if constexpr (S::XSUM) {
+#pragma unroll
+            for (int nt = 0; nt < NT; nt++) out_product(x[nt], acc[nt]);
+        }
+    }
+    // contracted block -> LDS [ab][cd]
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++)
+#pragma unroll
+        for (int ms = 0; ms < MT; ms++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int ab = 16 * ms + lk + 4 * r, cd = 16 * nt + lr;
+                if (ab < S::nsab && cd < S::nscd) outs[ab * S::nscd + cd] = acc[nt][ms][r];
+            }
+}
+
+// Direct digestion (several densities, deterministic builds, tiles that do not fit in LDS): work item
+// {j0, i0, i1}, bra i0 with kets [j0, i1), one shell quartet at a time, F' through global atomics.
+// With a.ndens > 1 each block is digested into every density (density d at D0 + d * dstride, its F' at
 // F0 + d * dstride, factors dfac[2 d], dfac[2 d + 1]).  a.det: F0 holds fixed-point accumulators
 // (fx_add, two words per element) and the factors come from dfac also for one density.
 template <int la, int lb, int lc, int ld, bool RS>
-__global__ void __launch_bounds__(VLX_WAVE) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(VLX_WAVE) __attribute__((amdgpu_waves_per_eu(MmdSizes<la, lb, lc, ld>::occupancy)))
     fock_kernel_mmd(const PairInfo* __restrict__ bra, const PrimPair* __restrict__ bra_prims,
                     const double* __restrict__ bra_u, const PairInfo* __restrict__ ket,
                     const PrimPair* __restrict__ ket_prims, const double* __restrict__ ket_u,
@@ -450,28 +673,16 @@ __global__ void __launch_bounds__(VLX_WAVE) __attribute__((amdgpu_waves_per_eu(4
                     const int* __restrict__ glim, const double* __restrict__ dfac, const FockScalars a)
 {
     using S = MmdSizes<la, lb, lc, ld>;
-    constexpr int L = S::L;
+    constexpr int NR = S::NR;
     __shared__ double rbuf[2 * S::nr];
-    __shared__ double seeds[L + 1];
-    __shared__ double xt[S::XC * 16 * 16];
     __shared__ double outs[S::nsab * S::nscd];
+    __shared__ double dblk[S::nout];
     const int lane = threadIdx.x;
-    const int lr = lane & 15, lk = lane >> 4;
-    static_assert(16 * (S::MX + S::XC) <= nherm(VLX_MAX_LTOT) && 4 * S::KX <= nherm(VLX_MAX_LTOT),
-                  "X-product rows and columns index the Hermite decode table");
-    // packed Hermite (t, u, v) of this lane's X-product columns q = 4 kq + lk (0 beyond nhcd): the
-    // same for every quartet, kept in registers when the column loop is unrolled
-    int tqv[S::PRE_X ? S::KX : 1];
-#pragma unroll
-    for (int kq = 0; kq < (S::PRE_X ? S::KX : 1); kq++) {
-        const int q = 4 * kq + lk;
-        tqv[kq] = (S::PRE_X && q < S::nhcd) ? g_herm.e[q] : 0;
-    }
+    MmdLane<la, lb, lc, ld> ln;
+    ln.init(lane);
     for (long long it = blockIdx.x; it < a.nitems; it += gridDim.x) {
         const WorkItem wi = items[it];
         const MolDesc md = mols[wi.mol];
-        const double* __restrict__ D = D0 + md.base;
-        double* __restrict__ F = F0 + md.base;
         const PairInfo bp = bra[wi.i0];
         for (int j = wi.j0; j < wi.i1; j++) {
             const PairInfo kp = ket[j];
@@ -479,179 +690,171 @@ __global__ void __launch_bounds__(VLX_WAVE) __attribute__((amdgpu_waves_per_eu(4
             if (glim != nullptr &&
                 bp.bin + kp.bin > quartet_bin_limit(glim, a.ngroups, bp.grp_a, bp.grp_b, kp.grp_a, kp.grp_b))
                 continue;
-            // one 16-wide cd tile at a time: its accumulators persist over all primitive quartets
-            for (int nt = 0; nt < S::NT; nt++) {
-                vlx_d4 acc[S::MT];
+            // elements of the six blocks: their place in D and F', and the first density's D
+            size_t goff[NR];
+            double dval[NR];
 #pragma unroll
-                for (int m = 0; m < S::MT; m++) acc[m] = vlx_d4{0.0, 0.0, 0.0, 0.0};
-                for (int ib = 0; ib < bp.nprim; ib++) {
-                    const PrimPair pb = bra_prims[bp.prim_start + ib];
-                    const double* ua = bra_u + (size_t)(bp.prim_start + ib) * (S::HA * S::SA);
-                    for (int ik = 0; ik < kp.nprim; ik++) {
-                        const PrimPair pk = ket_prims[kp.prim_start + ik];
-                        const double* uc = ket_u + (size_t)(kp.prim_start + ik) * (S::HC * S::SC) + 16 * nt + lr;
-                        // short K loops: both products' U operands go to registers here, so that
-                        // their memory latency overlaps the Boys function and the R levels
-                        double ucv[S::PRE_X ? S::KX : 1], uav[S::PRE_O ? S::KO : 1][S::PRE_O ? S::MT : 1];
-                        if constexpr (S::PRE_X) {
-#pragma unroll
-                            for (int kq = 0; kq < S::KX; kq++) ucv[kq] = uc[(4 * kq + lk) * S::SC];
-                        }
-                        if constexpr (S::PRE_O) {
-#pragma unroll
-                            for (int kp2 = 0; kp2 < S::KO; kp2++)
-#pragma unroll
-                                for (int ms = 0; ms < S::MT; ms++) uav[kp2][ms] = ua[(4 * kp2 + lk) * S::SA + 16 * ms + lr];
-                        }
-                        const double sz = pb.zeta + pk.zeta;
-                        const double rho_c = pb.zeta * pk.zeta / sz;
-                        double rho = rho_c, w = vrsqrt<double>(sz);
-                        if constexpr (RS) {
-                            const double sfac = a.omega2 / (a.omega2 + rho_c);
-                            rho = rho_c * sfac;
-                            w *= sqrt(sfac);
-                        }
-                        const double pqx = pb.px - pk.px, pqy = pb.py - pk.py, pqz = pb.pz - pk.pz;
-                        double Fm[L + 1];
-                        boys_eval<L, double, true>(rho * (pqx * pqx + pqy * pqy + pqz * pqz), boys_tab, Fm);
-                        // R levels n = L .. 0, ping-pong in rbuf; R^n_000 = w (-2 rho)^n F_n, lane n
-                        // keeps level n's seed in LDS (the level loop then needs no register array)
-                        {
-                            double f = w, mine = 0.0;
-#pragma unroll
-                            for (int n = 0; n <= L; n++) {
-                                if (lane == n) mine = f * Fm[n];
-                                f *= -2.0 * rho;
-                            }
-                            if (lane <= L) seeds[lane] = mine;
-                            if (lane == L) rbuf[(L & 1) ? S::nr : 0] = mine;
-                        }
-                        double* cur = rbuf + ((L & 1) ? S::nr : 0);
-#pragma unroll 1
-                        for (int n = L - 1; n >= 0; n--) {
-                            double* prev = cur;
-                            cur = (cur == rbuf) ? rbuf + S::nr : rbuf;
-                            __syncthreads();
-                            const int nn = nherm(L - n);
-                            for (int idx = lane; idx < nn; idx += VLX_WAVE) {
-                                // one branch-free step from the packed table (idx 0: the seed)
-                                const int rr = g_hrec.e[idx];
-                                const int ax = (rr >> 18) & 3;
-                                const double pq = ax == 0 ? pqx : (ax == 1 ? pqy : pqz);
-                                const double val = fma(double(rr >> 20), prev[(rr >> 9) & 511], pq * prev[rr & 511]);
-                                cur[idx] = idx == 0 ? seeds[n] : val;
-                            }
-                        }
-                        __syncthreads();
-                        // X = sum_q (-1)^|q| R^0[p + q] U_CD[q][cd] for the 16 columns cd of tile nt, in
-                        // chunks of XC row tiles; each chunk feeds its K range of out += U_AB^T X at once
-#pragma unroll 1
-                        for (int pc = 0; pc < S::MX; pc += S::XC) {
-                            vlx_d4 x[S::XC];
-                            int prow[S::XC];
-                            bool prow_ok[S::XC];
-#pragma unroll
-                            for (int i = 0; i < S::XC; i++) {
-                                x[i] = vlx_d4{0.0, 0.0, 0.0, 0.0};
-                                const int p = 16 * (pc + i) + lr;  // < 16 (MX + XC) <= HA + 16, inside g_herm
-                                prow_ok[i] = p < S::nhab;
-                                const int tp = g_herm.e[p];
-                                prow[i] = prow_ok[i] ? tp : 0;
-                            }
-                            // branch-free steps: a masked row (p >= nhab) or column (q >= nhcd) has its
-                            // Hermite index zeroed, so it reads an in-range R entry, and selects an
-                            // exact zero; the LDS reads can then be issued ahead of the products
-#pragma unroll(S::PRE_X ? S::KX : 4)
-                            for (int kq = 0; kq < S::KX; kq++) {
-                                const int q = 4 * kq + lk;
-                                const bool qok = q < S::nhcd;
-                                int tq;
-                                if constexpr (S::PRE_X) {
-                                    tq = tqv[kq];
-                                } else {
-                                    const int t0 = g_herm.e[q];
-                                    tq = qok ? t0 : 0;
-                                }
-                                const bool neg = ((tq & 0xff) + ((tq >> 8) & 0xff) + (tq >> 16)) & 1;
-                                double bv;
-                                if constexpr (S::PRE_X) bv = ucv[kq];
-                                else bv = uc[q * S::SC];
-#pragma unroll
-                                for (int i = 0; i < S::XC; i++) {
-                                    // a last chunk past the MX row tiles (odd MX) has nothing to compute:
-                                    // wave-uniform skip; its X rows are never read by the next product
-                                    if (S::MX % S::XC != 0 && pc + i >= S::MX) continue;
-                                    const double r0 = cur[hidx_packed(prow[i] + tq)];
-                                    const double sr = neg ? -r0 : r0;
-                                    const double av = (qok && prow_ok[i]) ? sr : 0.0;
-                                    x[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, x[i], 0, 0, 0);
-                                }
-                            }
-#pragma unroll
-                            for (int i = 0; i < S::XC; i++)
-#pragma unroll
-                                for (int r = 0; r < 4; r++) xt[(16 * i + lk + 4 * r) * 16 + lr] = x[i][r];
-                            __syncthreads();
-                            // out[ab][cd] += sum_p U_AB[p][ab] X[p][cd] over this chunk's rows p
-                            const int k0 = 4 * pc, k1 = std::min(S::KO, 4 * (pc + S::XC));
-                            if constexpr (S::PRE_O) {
-                                // all K steps of the product are in registers (one chunk covers them)
-#pragma unroll
-                                for (int kp2 = 0; kp2 < S::KO; kp2++) {
-                                    const int pr = 4 * kp2 + lk;
-                                    const double bv = xt[(pr - 16 * pc) * 16 + lr];
-#pragma unroll
-                                    for (int ms = 0; ms < S::MT; ms++)
-                                        acc[ms] = __builtin_amdgcn_mfma_f64_16x16x4f64(uav[kp2][ms], bv, acc[ms], 0, 0, 0);
-                                }
-                            } else {
-                                // unrolled so that the U_AB loads of later steps issue ahead of the products
-#pragma unroll 4
-                                for (int kp2 = k0; kp2 < k1; kp2++) {
-                                    const int pr = 4 * kp2 + lk;
-                                    const double bv = xt[(pr - 16 * pc) * 16 + lr];
-#pragma unroll
-                                    for (int ms = 0; ms < S::MT; ms++) {
-                                        const double av = ua[pr * S::SA + 16 * ms + lr];
-                                        acc[ms] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[ms], 0, 0, 0);
-                                    }
-                                }
-                            }
-                            __syncthreads();
-                        }
-                    }
-                }
-                // contracted tile -> LDS [ab][cd]
-#pragma unroll
-                for (int ms = 0; ms < S::MT; ms++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int ab = 16 * ms + lk + 4 * r, cd = 16 * nt + lr;
-                        if (ab < S::nsab && cd < S::nscd) outs[ab * S::nscd + cd] = acc[ms][r];
-                    }
+            for (int k = 0; k < NR; k++) {
+                goff[k] = ln.place(k, lane, bp, kp, md.nao);
+                dval[k] = D0[md.base + goff[k]];
             }
-            __syncthreads();
+            mmd_block<la, lb, lc, ld, RS>(ln, lane, bp, kp, bra_prims, bra_u, ket_prims, ket_u, boys_tab, a.omega2, rbuf, outs);
             double sf = 1.0;
             if (bp.same) sf *= 0.5;
             if (kp.same) sf *= 0.5;
             if (a.same_class && bp.rank == j) sf *= 0.5;
-            if (a.det) {  // F0: fixed-point accumulators (two words per element), factors in dfac
-                for (int dd = 0; dd < max(a.ndens, 1); dd++)
-                    md::digest<la, lb, lc, ld, true>(bp, kp, sf, outs, D + dd * a.dstride,
-                                                     F0 + 2 * (md.base + dd * a.dstride), md.nao, dfac[2 * dd],
-                                                     dfac[2 * dd + 1]);
-            } else if (a.ndens > 1) {
-                for (int dd = 0; dd < a.ndens; dd++)
-                    md::digest<la, lb, lc, ld>(bp, kp, sf, outs, D + dd * a.dstride, F + dd * a.dstride, md.nao,
-                                               dfac[2 * dd], dfac[2 * dd + 1]);
-            } else {
-                md::digest<la, lb, lc, ld>(bp, kp, sf, outs, D, F, md.nao, a.fj, a.fk);
+            const int nds = a.ndens > 1 ? a.ndens : 1;
+            for (int dd = 0; dd < nds; dd++) {
+                if (dd > 0) {
+                    wave_lds_fence();
+#pragma unroll
+                    for (int k = 0; k < NR; k++) dval[k] = D0[md.base + dd * a.dstride + goff[k]];
+                }
+#pragma unroll
+                for (int k = 0; k < NR; k++)
+                    if (lane + VLX_WAVE * k < S::nout) dblk[ln.gwrap[k] >> 16] = dval[k];
+                wave_lds_fence();
+                const bool table = a.det || a.ndens > 1;
+                const double fj = sf * (table ? dfac[2 * dd] : a.fj), fk = sf * (table ? dfac[2 * dd + 1] : a.fk);
+#pragma unroll
+                for (int k = 0; k < NR; k++) {
+                    const double coef = (ln.gaddr[k] >> 10) & 1 ? fj : fk;
+                    const int terms = coef != 0.0 ? ln.gstep[k] >> 24 : 0;
+                    const double v = ln.sum(k, terms, outs, dblk);
+                    if (terms > 0) {
+                        const size_t at = md.base + dd * a.dstride + goff[k];
+                        if (a.det) fx_add(reinterpret_cast<unsigned long long*>(F0), at, coef * v);
+                        else unsafeAtomicAdd(F0 + at, coef * v);
+                    }
+                }
             }
-            __syncthreads();
+            wave_lds_fence();
         }
     }
 }
 
+// Tiled digestion: a block of NW wavefronts takes one TileItem (here [j0, j1) are ket pairs of the
+// tiled order), and the F' elements go into the six LDS tiles of the item's atom groups, flushed once
+// per item as in fock_kernel_tiled.  The direct form is bound by its global atomics: FP64 atomics of
+// eight L2s are carried out at the memory side, 13 to 17 billion a second over the whole chip in every
+// class, while the matrix cores are busy 17% and the vector units 26% of the time ((fp|dp), 116 atomics
+// a quartet).  Units of up to 8 kets of one bra go round the wavefronts.  One stream, 20 waters
+// def2-TZVP, direct / tiled: (fp|dp) 4.3 / 3.9 ms, (fp|fp) 1.5 / 1.8 ms (its tiles leave 8 wavefronts a
+// CU), (dd|dp) of one water 0.043 / 0.043 ms.
+template <int la, int lb, int lc, int ld>
+struct MmdTile {
+    using S = MmdSizes<la, lb, lc, ld>;
+    static constexpr int NW = 4 * S::occupancy;  // one block fills a CU's registers
+    static constexpr int scratch = 2 * S::nr + S::nsab * S::nscd + S::nout;  // doubles per wavefront
+    static constexpr int KETS = 8;
+};
+
+template <int la, int lb, int lc, int ld, bool RS>
+__global__ void __launch_bounds__((MmdTile<la, lb, lc, ld>::NW * VLX_WAVE))
+    __attribute__((amdgpu_waves_per_eu(MmdSizes<la, lb, lc, ld>::occupancy)))
+    fock_kernel_mmd_tiled(const PairInfo* __restrict__ pairs_bra, const PrimPair* __restrict__ bra_prims,
+                          const double* __restrict__ bra_u, const PairInfo* __restrict__ pairs_ket,
+                          const PrimPair* __restrict__ ket_prims, const double* __restrict__ ket_u,
+                          const TileItem* __restrict__ items, const double* __restrict__ boys_tab,
+                          const double* __restrict__ D0, double* __restrict__ F0, const MolDesc* __restrict__ mols,
+                          const int* __restrict__ glim, const int* __restrict__ grp_off, const int* __restrict__ grp_n,
+                          const int* __restrict__ grp_ao, const FockScalars a)
+{
+    using S = MmdSizes<la, lb, lc, ld>;
+    using T = MmdTile<la, lb, lc, ld>;
+    constexpr int NR = S::NR, NW = T::NW;
+    extern __shared__ double tiles[];
+    const int lane = threadIdx.x & (VLX_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / VLX_WAVE);
+    double* rbuf = tiles + a.tile_doubles + wave * T::scratch;
+    double* outs = rbuf + 2 * S::nr;
+    double* dblk = outs + S::nsab * S::nscd;
+    for (int e = threadIdx.x; e < a.tile_doubles; e += NW * VLX_WAVE) tiles[e] = 0.0;
+    MmdLane<la, lb, lc, ld> ln;
+    ln.init(lane);
+    __syncthreads();
+    for (long long it = blockIdx.x; it < a.nitems; it += gridDim.x) {
+        const TileItem ti = items[it];
+        const MolDesc md = mols[ti.mol];
+        const double* __restrict__ D = D0 + md.base;
+        double* __restrict__ F = F0 + md.base;
+        int ilim = a.ithreshold;
+        if (glim != nullptr) ilim = min(ilim, quartet_bin_limit(glim, a.ngroups, ti.ga, ti.gb, ti.gc, ti.gd));
+        // smallest bin sum of the item: past the limit it has no quartet (block-uniform skip)
+        if (a.ithreshold >= 0 && pairs_bra[ti.i0].bin + ti.bin_lo > ilim) continue;
+        const int nA = grp_n[ti.ga * 4 + la], nB = grp_n[ti.gb * 4 + lb];
+        const int nC = grp_n[ti.gc * 4 + lc], nD = grp_n[ti.gd * 4 + ld];
+        // tiles J_AB, K_AC, K_BC, J_CD, K_AD, K_BD
+        double* t_jab = tiles;
+        double* t_kac = t_jab + nA * nB;
+        double* t_kbc = t_kac + nA * nC;
+        double* t_jcd = t_kbc + nB * nC;
+        double* t_kad = t_jcd + nC * nD;
+        double* t_kbd = t_kad + nA * nD;
+        // the lane's elements in the tiles: place of component (i, j), row stride
+        int tbase[NR], tstride[NR];
+#pragma unroll
+        for (int k = 0; k < NR; k++) {
+            const int x = ln.gaddr[k] & 3, i = (ln.gaddr[k] >> 2) & 7, y = (ln.gaddr[k] >> 5) & 3, j = (ln.gaddr[k] >> 7) & 7;
+            tstride[k] = y == 1 ? nB : y == 2 ? nC : nD;
+            const double* t = y == 1 ? t_jab : y == 2 ? (x == 0 ? t_kac : t_kbc) : x == 0 ? t_kad : x == 1 ? t_kbd : t_jcd;
+            tbase[k] = static_cast<int>(t - tiles) + i * tstride[k] + j;
+        }
+        const int nunit = (ti.j1 - ti.j0 + T::KETS - 1) / T::KETS;
+        for (int u = wave; u < (ti.i1 - ti.i0) * nunit; u += NW) {
+            const int i = ti.i0 + u / nunit, j0 = ti.j0 + u % nunit * T::KETS;
+            const PairInfo bp = pairs_bra[i];
+            for (int j = j0; j < min(ti.j1, j0 + T::KETS); j++) {
+                const PairInfo kp = pairs_ket[j];
+                if (a.ithreshold >= 0 && bp.bin + kp.bin > ilim) break;  // kets go by bin
+                if (a.same_class && bp.rank < kp.rank) continue;
+                int toff[NR];
+                double dval[NR];
+#pragma unroll
+                for (int k = 0; k < NR; k++) {
+                    const int x = ln.gaddr[k] & 3, y = (ln.gaddr[k] >> 5) & 3;
+                    const int row = x == 0 ? bp.loc_a : x == 1 ? bp.loc_b : kp.loc_a;
+                    const int col = y == 1 ? bp.loc_b : y == 2 ? kp.loc_a : kp.loc_b;
+                    toff[k] = tbase[k] + row * tstride[k] + col;
+                    dval[k] = D[ln.place(k, lane, bp, kp, md.nao)];
+                }
+                mmd_block<la, lb, lc, ld, RS>(ln, lane, bp, kp, bra_prims, bra_u, ket_prims, ket_u, boys_tab, a.omega2, rbuf,
+                                              outs);
+                double sf = 1.0;
+                if (bp.same) sf *= 0.5;
+                if (kp.same) sf *= 0.5;
+                if (a.same_class && bp.rank == kp.rank) sf *= 0.5;
+#pragma unroll
+                for (int k = 0; k < NR; k++)
+                    if (lane + VLX_WAVE * k < S::nout) dblk[ln.gwrap[k] >> 16] = dval[k];
+                wave_lds_fence();
+#pragma unroll
+                for (int k = 0; k < NR; k++) {
+                    const int terms = ((ln.gaddr[k] >> 10) & 1 ? a.fj : a.fk) != 0.0 ? ln.gstep[k] >> 24 : 0;
+                    const double v = ln.sum(k, terms, outs, dblk);
+                    if (terms > 0) unsafeAtomicAdd(&tiles[toff[k]], sf * v);
+                }
+                wave_lds_fence();
+            }
+        }
+        __syncthreads();
+        const int* ra = grp_ao + grp_off[ti.ga * 4 + la];
+        const int* rb = grp_ao + grp_off[ti.gb * 4 + lb];
+        const int* rc = grp_ao + grp_off[ti.gc * 4 + lc];
+        const int* rd = grp_ao + grp_off[ti.gd * 4 + ld];
+        if (a.fj != 0.0) {
+            flush_tile<NW>(F, md.nao, t_jab, nA, nB, ra, rb, a.fj, wave, lane);
+            flush_tile<NW>(F, md.nao, t_jcd, nC, nD, rc, rd, a.fj, wave, lane);
+        }
+        if (a.fk != 0.0) {
+            flush_tile<NW>(F, md.nao, t_kac, nA, nC, ra, rc, a.fk, wave, lane);
+            flush_tile<NW>(F, md.nao, t_kbc, nB, nC, rb, rc, a.fk, wave, lane);
+            flush_tile<NW>(F, md.nao, t_kad, nA, nD, ra, rd, a.fk, wave, lane);
+            flush_tile<NW>(F, md.nao, t_kbd, nB, nD, rb, rd, a.fk, wave, lane);
+        }
+        __syncthreads();
+    }
+}
 
 template <int la, int lb, int lc, int ld>
 __global__ void __launch_bounds__(VLX_WAVE) eri_out_kernel_md(const EriArgs a)
@@ -706,6 +909,23 @@ __global__ void __launch_bounds__(VLX_WAVE) diag_kernel_md(const DiagArgs a)
     hipLaunchKernelGGL((fock_kernel_mmd<la, lb, lc, ld, RS>), dim3(g), dim3(VLX_WAVE), 0, s, a.bra,     \
                        a.bra_prims, a.bra_u, a.ket, a.ket_prims, a.ket_u, a.items, a.boys_tab, a.D, a.F, \
                        a.mols, a.glim, a.dfac, a.sc)
+// tiled digestion: TileItem list, dynamic LDS of the tiles (a.tile_lds_bytes) and the waves' scratch
+#define VLX_INSTANTIATE_MMD_TILED(la, lb, lc, ld)                                                       \
+    void launch_mmd_tiled_##la##lb##lc##ld(const FockArgs& a, int grid, hipStream_t s)                  \
+    {                                                                                                   \
+        using T = MmdTile<la, lb, lc, ld>;                                                              \
+        const int lds = a.tile_lds_bytes + 8 * T::NW * T::scratch;                                      \
+        if (a.sc.omega2 > 0.0)                                                                          \
+            hipLaunchKernelGGL((fock_kernel_mmd_tiled<la, lb, lc, ld, true>), dim3(grid), dim3(T::NW * VLX_WAVE), \
+                               lds, s, a.bra, a.bra_prims, a.bra_u, a.ket, a.ket_prims, a.ket_u, a.titems, \
+                               a.boys_tab, a.D, a.F, a.mols, a.glim, a.grp_off, a.grp_n, a.grp_ao, a.sc); \
+        else                                                                                            \
+            hipLaunchKernelGGL((fock_kernel_mmd_tiled<la, lb, lc, ld, false>), dim3(grid),              \
+                               dim3(T::NW * VLX_WAVE), lds, s, a.bra, a.bra_prims, a.bra_u, a.ket,      \
+                               a.ket_prims, a.ket_u, a.titems, a.boys_tab, a.D, a.F, a.mols, a.glim,    \
+                               a.grp_off, a.grp_n, a.grp_ao, a.sc);                                     \
+    }                                                                                                   \
+    int mmd_scratch_##la##lb##lc##ld() { return 8 * MmdTile<la, lb, lc, ld>::NW * MmdTile<la, lb, lc, ld>::scratch; }
 // launch_mmd_: the matrix-core kernel as an alternative variant of a class
 // whose default kernel is generated (same MD work items).
 #define VLX_INSTANTIATE_MMD(la, lb, lc, ld)                                                             \

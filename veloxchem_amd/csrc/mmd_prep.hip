@@ -1,14 +1,14 @@
 // Hermite-to-spherical matrices of the matrix-core MD Fock kernel, built once
 // per pair set: U[prim][h][s] = k sum_{cart a, b} S_a S_b E^x_t E^y_u E^z_v for
 // Hermite index h = (t, u, v) of degree <= la + lb and spherical index
-// s = (m_a, m_b) of the pair; zero in the padding rows and columns.
+// s = (m_a, m_b) of the pair; zero in the padding rows and columns.  Ket pairs carry (-1)^{t+u+v}.
 #include "md_kernels.h"
 
 namespace {
 
 __global__ void __launch_bounds__(VLX_WAVE)
     u_build_kernel(const PairInfo* __restrict__ pairs, const PrimPair* __restrict__ prims, int npairs, int la, int lb,
-                   double* __restrict__ U)
+                   bool ket, double* __restrict__ U)
 {
     __shared__ double e[3 * md::E3];
     const int nh = md::nherm(la + lb), nsb = 2 * lb + 1, ns = (2 * la + 1) * nsb;
@@ -45,7 +45,7 @@ __global__ void __launch_bounds__(VLX_WAVE)
                                    e[2 * md::E3 + (az * md::D1 + bz) * md::DT + v];
                         }
                     }
-                    acc *= pr.k;
+                    acc *= (ket && ((t + uu + v) & 1)) ? -pr.k : pr.k;
                 }
                 u[idx] = acc;
             }
@@ -55,10 +55,10 @@ __global__ void __launch_bounds__(VLX_WAVE)
 
 }  // namespace
 
-void vlx_launch_u_build(const PairInfo* pairs, const PrimPair* prims, int npairs, int la, int lb, double* u,
-                        hipStream_t s)
+void vlx_launch_u_build(const PairInfo* pairs, const PrimPair* prims, int npairs, int la, int lb, bool ket,
+                        double* u, hipStream_t s)
 {
     if (npairs <= 0) return;
     const int g = std::min(npairs, 16384);
-    hipLaunchKernelGGL(u_build_kernel, dim3(g), dim3(VLX_WAVE), 0, s, pairs, prims, npairs, la, lb, u);
+    hipLaunchKernelGGL(u_build_kernel, dim3(g), dim3(VLX_WAVE), 0, s, pairs, prims, npairs, la, lb, ket, u);
 }

@@ -173,7 +173,8 @@ struct ClassSchedule {
     int variant = 0;      // VARIANT_* the schedule runs
     bool tiled = false;
     bool singles = false; // tiled over single-primitive ket entries
-    bool mmd = false;     // matrix-core MD kernel (MD work items)
+    bool mmd = false;     // matrix-core MD kernel (MD work items, or tiled items when mmd_tiled)
+    bool mmd_tiled = false;  // matrix-core MD kernel with LDS tiles (TileItem over ket pairs)
     bool ksl = false;     // ket-stationary kernel with LDS accumulators (ket-stationary work items)
     bool dlds = false;    // tiled, the item's D blocks staged in LDS (twice the tile LDS)
     int tiled_waves = 0;  // 4: 4-wave blocks; 0: the class's wide block
@@ -195,7 +196,7 @@ struct vlx_screener;
 struct BatchLaunch {
     int entry = -1;       // index into g_class_table
     int variant = 0, tiled_waves = 0, tile_lds = 0, stream = 0;
-    bool tiled = false, singles = false, mmd = false, ksl = false;
+    bool tiled = false, singles = false, mmd = false, mmd_tiled = false, ksl = false;
     std::vector<TileItem> titems;
     std::vector<WorkItem> items;
     DevBuf<TileItem> d_titems;
@@ -248,6 +249,8 @@ constexpr int BRA_CHUNK = 128;  // default upper bound of bras per work item
 
 // largest tiled item, in (bra, 64-entry ket chunk) units: its tiles' flush is then a small share
 constexpr long long TILE_ITEM_UNITS = 1024;
+// largest tiled item of the matrix-core MD kernel, in shell quartets
+constexpr long long MMD_ITEM_UNITS = 2048;
 
 constexpr int NSIDE = 4;  // side streams that run class kernels concurrently
 
@@ -312,6 +315,7 @@ struct vlx_context {
     // largest grid (one wavefront per block) of a matrix-core MD launch (VLX_MMD_GRID): on the 64-water
     // def2-TZVP build 16384 / 32768 / 65536 measured 0.775 / 0.786 / 0.793 builds/s
     int mmd_grid = 65536;
+    bool u_pending = false;         // U arrays still being built on the stream (ensure_u, finish_u)
     // kets per matrix-core MD work item (VLX_MMD_KETS): on the 64-water def2-TZVP build the MD classes
     // took 333.2 / 327.1 / 332.1 / 342.9 ms with 1 / 2 / 4 / 8 kets
     int mmd_kets = 2;
@@ -628,16 +632,24 @@ void build_tiled(const vlx_screener& s, const PairSet& src, PairSet& ket, PairSe
     make_entries(1, ket.singles);
 }
 
-// U arrays of a pair set for the matrix-core MD Fock kernel (once per set).
-int ensure_u(vlx_context* ctx, PairSet& ps)
+// U arrays of a pair set for the matrix-core MD Fock kernel (once per set), left running on the
+// context's stream: the caller waits once, after its last set (finish_u).
+int ensure_u(vlx_context* ctx, PairSet& ps, bool ket)
 {
     if (ps.u_ready || ps.size() == 0) return VLX_OK;
     const size_t per = (size_t)vlx_u_rows(ps.la, ps.lb) * vlx_u_cols(ps.la, ps.lb);
     HIP_TRY(ps.d_u.alloc(per * ps.prims.size()));
-    vlx_launch_u_build(ps.d_pairs.ptr, ps.d_prims.ptr, ps.size(), ps.la, ps.lb, ps.d_u.ptr, ctx->stream);
+    vlx_launch_u_build(ps.d_pairs.ptr, ps.d_prims.ptr, ps.size(), ps.la, ps.lb, ket, ps.d_u.ptr, ctx->stream);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
     ps.u_ready = true;
+    ctx->u_pending = true;
+    return VLX_OK;
+}
+
+int finish_u(vlx_context* ctx)
+{
+    if (ctx->u_pending) HIP_TRY(hipStreamSynchronize(ctx->stream));
+    ctx->u_pending = false;
     return VLX_OK;
 }
 
@@ -820,12 +832,14 @@ int ensure_unscreened(vlx_screener* s)
 // create = false: only a schedule built earlier is returned (no host or device allocation);
 // without one the call fails.
 // share: the builds that run side by side in one launch (a batch's molecules), each aiming at its
-// share of the tiled items.
+// share of the tiled items.  direct: the matrix-core MD classes with the work items of the direct
+// digestion (multi-density and deterministic builds).
 int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_ptr<ClassSchedule>>** out,
-                  bool create = true, int share = 1)
+                  bool create = true, int share = 1, bool direct = false)
 {
     const int tile_items = std::max(1, s->ctx->tile_items / share);
-    const std::pair<int, int> key{((ithr + 1) * 128 + k32) * (NVARIANTS + 1) + (s->ctx->force_variant + 1), tile_items};
+    const std::pair<int, int> key{((ithr + 1) * 128 + k32) * (NVARIANTS + 1) + (s->ctx->force_variant + 1),
+                                  2 * tile_items + (direct ? 1 : 0)};
     auto it = s->schedules.find(key);
     if (it != s->schedules.end()) {
         *out = &it->second;
@@ -874,6 +888,16 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         // allows it); the autotuner's choice, or the one being timed, overrides it
         int var = (can_tile && (L <= 4 || nsph <= 75)) ? (s->ctx->tiled_waves == 4 ? VARIANT_TILED4 : VARIANT_TILED_WIDE)
                                                       : VARIANT_UNTILED;
+        // The others: a lane of the generated kernels runs a quartet by itself and spills where the
+        // block is large, a wavefront of the matrix-core kernel shares it.  One stream, generated /
+        // matrix-core, 20 waters def2-TZVP: (fd|pp) 6.3 / 1.9 ms, (dd|dp) 5.2 / 1.2, (dp|dp) 4.1 / 2.5,
+        // (fd|ds) 2.5 / 2.4, (fp|pp) 4.4 / 4.8, but (fp|fs) 4.0 / 4.4, (dp|pp) 3.9 / 6.5 and
+        // (ff|ps) 1.9 / 2.7: the line is at 175 integrals.  Smaller blocks are matrix-core as well
+        // while a launch has too few quartets for a lane each: the generated kernels then take the
+        // time of one lane ((dp|pp) of one water, 144 primitive quartets, 0.18 / 0.08 ms; of two waters
+        // def2-TZVP, 6000, 0.39 / 0.16; (fp|fs) there 0.82 / 0.15), and lose it at about 2e5
+        // (of the whole launch: a batch's molecules share it)
+        if (var == VARIANT_UNTILED && ce.mmd && (nsph >= 175 || sch->prim_quartets * share < 200000)) var = VARIANT_MMD;
         if (s->ctx->force_variant >= 0) {
             var = s->ctx->force_variant;
         } else {
@@ -893,6 +917,8 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         if (ce.variant == VLX_WAVE_MD) var = VARIANT_MMD;  // no generated kernel
         sch->variant = var;
         sch->mmd = var == VARIANT_MMD;
+        sch->mmd_tiled = sch->mmd && !direct && s->ctx->use_tiled && ce.mmd_tiled &&
+                         tile_lds + ce.mmd_scratch() <= 160 * 1024 - 1024;
         sch->ksl = var == VARIANT_KSL;
         sch->dlds = var == VARIANT_TILED_DLDS;
         if (variant_tiled(var)) {
@@ -949,6 +975,42 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
             }
             // longest items first, so that the launch ends on short ones
             auto units_of = [](const TileItem& t) { return (long long)(t.i1 - t.i0) * ((t.j1 - t.j0) / VLX_WAVE); };
+            std::stable_sort(sch->titems.begin(), sch->titems.end(),
+                             [&](const TileItem& x, const TileItem& y) { return units_of(x) > units_of(y); });
+        } else if (sch->mmd_tiled) {
+            // tiled items of ket pairs: (bras of a bra segment) x (kets of a ket segment)
+            const PairSet& tb = unscreened ? s->all_tiled_bra[ce.x] : s->kept_tiled_bra[ce.x];
+            const PairSet& tk = unscreened ? s->all_tiled[ce.y] : s->kept_tiled[ce.y];
+            sch->tile_lds = tile_lds;
+            auto kets = [&](const PairSet::Segment& ks, int bin) {  // kets a bra of bin `bin` meets
+                if (unscreened) return ks.end - ks.start;
+                return ithr - bin < 0 ? 0 : ks.cnt_le[std::min(ithr - bin, NBINS - 1)];
+            };
+            long long units = 0;
+            for (size_t sk = 0; sk < tk.segs.size(); sk++)
+                for (size_t sb = same ? sk : 0; sb < tb.segs.size(); sb++)
+                    for (int i = tb.segs[sb].start; i < tb.segs[sb].end; i++) units += kets(tk.segs[sk], std::max(tb.pairs[i].bin, 0));
+            const long long target = std::max(16LL, std::min(MMD_ITEM_UNITS, units / tile_items));
+            for (size_t sk = 0; sk < tk.segs.size(); sk++) {
+                const auto& ks = tk.segs[sk];
+                const int bin_lo = std::max(tk.pairs[ks.start].bin, 0);
+                for (size_t sb = same ? sk : 0; sb < tb.segs.size(); sb++) {
+                    const auto& bs = tb.segs[sb];
+                    for (int i0 = bs.start, i1; i0 < bs.end; i0 = i1) {
+                        // kets of the item: those of its first bra, which has the smallest bin
+                        const int nk = kets(ks, std::max(tb.pairs[i0].bin, 0));
+                        if (nk == 0) break;
+                        long long u = 0;
+                        for (i1 = i0; i1 < bs.end && (i1 == i0 || u < target); i1++) {
+                            const int m = kets(ks, std::max(tb.pairs[i1].bin, 0));
+                            if (m == 0) break;
+                            u += m;
+                        }
+                        sch->titems.push_back({i0, i1, ks.start, ks.start + nk, bs.ga, bs.gb, ks.ga, ks.gb, 0, bin_lo});
+                    }
+                }
+            }
+            auto units_of = [](const TileItem& t) { return (long long)(t.i1 - t.i0) * (t.j1 - t.j0); };
             std::stable_sort(sch->titems.begin(), sch->titems.end(),
                              [&](const TileItem& x, const TileItem& y) { return units_of(x) > units_of(y); });
         } else if (!sch->mmd && (ce.variant == VLX_KET_STATIONARY || sch->ksl)) {
@@ -1021,6 +1083,9 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
             for (const auto& ti : sch->titems) count(ti, sch->prim_slots);
             for (const auto& ti : sch->titems32) count(ti, sch->prim_slots32);
             sch->prim_slots += sch->prim_slots32;
+        } else if (sch->mmd_tiled) {  // one quartet per wavefront pass
+            sch->lane_slots = sch->quartets;
+            sch->prim_slots = sch->prim_quartets;
         } else if (!sch->mmd) {
             // estimated cost of an item in FLOPs of one lane: primitive iterations times the
             // per-primitive work, plus the contracted work per quartet; the items are then
@@ -1053,12 +1118,16 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
             }
         }
         if (sch->items.empty() && sch->titems.empty() && sch->titems32.empty()) continue;
-        if (sch->mmd) {
-            int rc = ensure_u(s->ctx, unscreened ? s->all_bra[ce.x] : s->kept_bra[ce.x]);
-            if (!rc) rc = ensure_u(s->ctx, unscreened ? s->all[ce.y] : s->kept[ce.y]);
+        if (sch->mmd_tiled) {
+            int rc = ensure_u(s->ctx, unscreened ? s->all_tiled_bra[ce.x] : s->kept_tiled_bra[ce.x], false);
+            if (!rc) rc = ensure_u(s->ctx, unscreened ? s->all_tiled[ce.y] : s->kept_tiled[ce.y], true);
+            if (rc) return rc;
+        } else if (sch->mmd) {
+            int rc = ensure_u(s->ctx, unscreened ? s->all_bra[ce.x] : s->kept_bra[ce.x], false);
+            if (!rc) rc = ensure_u(s->ctx, unscreened ? s->all[ce.y] : s->kept[ce.y], true);
             if (rc) return rc;
         }
-        if (sch->tiled) {
+        if (sch->tiled || sch->mmd_tiled) {
             if (!sch->titems.empty()) HIP_TRY(sch->d_titems.upload(sch->titems));
             if (!sch->titems32.empty()) HIP_TRY(sch->d_titems32.upload(sch->titems32));
         } else {
@@ -1066,6 +1135,7 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         }
         list.push_back(std::move(sch));
     }
+    if (const int rc = finish_u(s->ctx)) return rc;
     // spread classes over the side streams, most expensive first: by the autotuner's measured
     // times when every class has one (the kernel families differ ~5x in FLOP rate), else by
     // estimated FLOPs
@@ -1835,7 +1905,8 @@ int vlx_fock_class_kernel(vlx_context* ctx, vlx_screener* scr, int ithreshold, i
             std::snprintf(name, len, "fock_kernel_tiled<%d,%d,%d,%d,double,%d,false,false,%s>", la, lb, lc, ld,
                           sp->tiled_waves == 4 ? 4 : wide, sp->dlds ? "true" : "false");
         } else {
-            const char* k = sp->mmd                             ? "fock_kernel_mmd"
+            const char* k = sp->mmd_tiled                       ? "fock_kernel_mmd_tiled"
+                            : sp->mmd                           ? "fock_kernel_mmd"
                             : sp->ksl                           ? "fock_kernel_ksl"
                             : (ce.variant == VLX_KET_STATIONARY) ? "fock_kernel"
                                                                 : "fock_kernel_bs";
@@ -1904,10 +1975,11 @@ int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::
         const ClassSchedule& sch = *schp;
         if (solo >= 0 && (sch.stream < 0) != (solo == 1)) continue;
         const auto& ce = g_class_table[sch.entry];
-        const PairSet& bra = sch.tiled ? (unscreened ? scr->all_tiled_bra[ce.x] : scr->kept_tiled_bra[ce.x])
-                                       : (unscreened ? scr->all_bra[ce.x] : scr->kept_bra[ce.x]);
-        const PairSet& ket = sch.tiled ? (unscreened ? scr->all_tiled[ce.y] : scr->kept_tiled[ce.y])
-                                       : (unscreened ? scr->all[ce.y] : scr->kept[ce.y]);
+        const bool titems = sch.tiled || sch.mmd_tiled;
+        const PairSet& bra = titems ? (unscreened ? scr->all_tiled_bra[ce.x] : scr->kept_tiled_bra[ce.x])
+                                    : (unscreened ? scr->all_bra[ce.x] : scr->kept_bra[ce.x]);
+        const PairSet& ket = titems ? (unscreened ? scr->all_tiled[ce.y] : scr->kept_tiled[ce.y])
+                                    : (unscreened ? scr->all[ce.y] : scr->kept[ce.y]);
         FockArgs a{};
         a.bra = bra.d_pairs.ptr;
         a.bra_prims = bra.d_prims.ptr;
@@ -1934,7 +2006,7 @@ int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::
         a.ket_lanes = sch.singles ? ket.singles.d_lanes.ptr : ket.runs.d_lanes.ptr;
         a.sc.ket_slots = sch.singles ? ket.singles.slots : ket.runs.slots;
         a.sc.tile_doubles = sch.tile_lds / 8;
-        a.sc.nitems = static_cast<long long>(sch.tiled ? sch.titems.size() : sch.items.size());
+        a.sc.nitems = static_cast<long long>(titems ? sch.titems.size() : sch.items.size());
         a.sc.nket = ket.size();
         a.sc.ithreshold = ithreshold;
         a.sc.same_class = (ce.x == ce.y) ? 1 : 0;
@@ -1947,7 +2019,7 @@ int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::
         a.sc.det = det ? 1 : 0;
         a.sc.bs_layout = (ce.variant == VLX_BRA_STATIONARY && !sch.ksl) ? 1 : 0;
         a.dfac = dfac;
-        const int grid = sch.tiled ? static_cast<int>(std::min<long long>(a.sc.nitems, ctx->tiled_grid))
+        const int grid = titems ? static_cast<int>(std::min<long long>(a.sc.nitems, ctx->tiled_grid))
                          : sch.mmd ? static_cast<int>(std::min<long long>(a.sc.nitems, ctx->mmd_grid))
                                    : static_cast<int>(untiled_waves(a.sc.nitems, ctx->untiled_wave_cap) / VLX_WAVES_PER_BLOCK);
         hipStream_t st = stream ? stream : (sch.stream < 0 ? ctx->stream : ctx->side[sch.stream % ctx->nstreams]);
@@ -1964,6 +2036,7 @@ int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::
             HIP_TRY(hipEventRecord(pend.start, st));
         }
         if (multi) {
+            if (sch.mmd_tiled) return fail(VLX_ERR_ARG, "multi-density builds digest directly");
             if (det && sch.tiled) return fail(VLX_ERR_ARG, "deterministic builds run the untiled kernels only");
             // Kernels whose single-density form keeps accumulators the multi-density form cannot
             // hold run once per density instead (the integrals are recomputed): ks-lds (one density
@@ -2028,6 +2101,8 @@ int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::
                 const int grid32 = static_cast<int>(std::min<long long>(a32.sc.nitems, ctx->tiled_grid));
                 ce.tiled32(a32, grid32, st);
             }
+        } else if (sch.mmd_tiled) {
+            ce.mmd_tiled(a, grid, st);
         } else if (sch.mmd) {
             ce.mmd(a, grid, st);
         } else if (sch.ksl) {
@@ -2079,7 +2154,7 @@ int multi_pass(vlx_context* ctx, vlx_screener* scr, const double* dens, int m, c
     std::vector<std::unique_ptr<ClassSchedule>>* list = nullptr;
     const int saved_variant = ctx->force_variant;
     if (det) ctx->force_variant = VARIANT_UNTILED;
-    int rc = get_schedules(scr, ithreshold, NO_FP32, &list, true);
+    int rc = get_schedules(scr, ithreshold, NO_FP32, &list, true, 1, true);
     ctx->force_variant = saved_variant;
     if (rc) return rc;
     const bool single = m == 1 && !det;
@@ -2393,7 +2468,7 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
         for (const auto& sp : *lists[m]) {
             const ClassSchedule& sch = *sp;
             const auto& ce = g_class_table[sch.entry];
-            const std::array<int, 4> key{sch.entry, sch.variant, sch.singles ? 1 : 0, sch.tiled_waves};
+            const std::array<int, 4> key{sch.entry, sch.variant, (sch.singles ? 1 : 0) + (sch.mmd_tiled ? 2 : 0), sch.tiled_waves};
             BatchLaunch*& L = by_key[key];
             if (!L) {
                 P.launches.push_back(std::make_unique<BatchLaunch>());
@@ -2403,14 +2478,16 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
                 L->tiled = sch.tiled;
                 L->singles = sch.singles;
                 L->mmd = sch.mmd;
+                L->mmd_tiled = sch.mmd_tiled;
                 L->ksl = sch.ksl;
                 L->tiled_waves = sch.tiled_waves;
             }
             L->tile_lds = std::max(L->tile_lds, sch.tile_lds);
             L->cost += (double)sch.prim_quartets * (ce.vrr_flops + 60) + (double)sch.quartets * ce.hrr_flops;
             const int x = m * npc + ce.x, y = m * npc + ce.y;
-            if (sch.tiled) {
-                const int eo = sch.singles ? eoff_singles[y] : eoff_runs[y];
+            if (sch.tiled || sch.mmd_tiled) {
+                // lane entries, or ket pairs of the matrix-core MD kernel
+                const int eo = sch.mmd_tiled ? poff[TKET][y] : sch.singles ? eoff_singles[y] : eoff_runs[y];
                 for (const auto* lst : {&sch.titems, &sch.titems32})
                     for (TileItem ti : *lst) {
                         ti.i0 += poff[TBRA][x];
@@ -2440,15 +2517,20 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
     for (auto& Lp : P.launches) {
         BatchLaunch& L = *Lp;
         const auto& ce = g_class_table[L.entry];
-        if (L.tiled) {
+        if (L.tiled || L.mmd_tiled) {
             HIP_TRY(L.d_titems.upload(L.titems));
+            if (L.mmd_tiled) {
+                int rc = ensure_u(ctx, P.tbra[ce.x], false);
+                if (!rc) rc = ensure_u(ctx, P.tket[ce.y], true);
+                if (rc) return rc;
+            }
             continue;
         }
         const PairSet& bra = P.bra[ce.x];
         const PairSet& ket = P.ket[ce.y];
         if (L.mmd) {
-            int rc = ensure_u(ctx, P.bra[ce.x]);
-            if (!rc) rc = ensure_u(ctx, P.ket[ce.y]);
+            int rc = ensure_u(ctx, P.bra[ce.x], false);
+            if (!rc) rc = ensure_u(ctx, P.ket[ce.y], true);
             if (rc) return rc;
         } else if (ctx->balance_items) {
             // the wavefronts' contiguous ranges of equal estimated cost, over the whole batch
@@ -2469,6 +2551,7 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
         }
         HIP_TRY(L.d_items.upload(L.items));
     }
+    if (const int rc = finish_u(ctx)) return rc;
     // side streams by estimated cost, most expensive launches first
     std::sort(P.launches.begin(), P.launches.end(),
               [](const std::unique_ptr<BatchLaunch>& a, const std::unique_ptr<BatchLaunch>& b) { return a->cost > b->cost; });
@@ -2504,8 +2587,9 @@ int record_batch(vlx_context* ctx, BatchPlan& P)
     for (auto& Lp : P.launches) {
         const BatchLaunch& L = *Lp;
         const auto& ce = g_class_table[L.entry];
-        const PairSet& bra = L.tiled ? P.tbra[ce.x] : P.bra[ce.x];
-        const PairSet& ket = L.tiled ? P.tket[ce.y] : P.ket[ce.y];
+        const bool titems = L.tiled || L.mmd_tiled;
+        const PairSet& bra = titems ? P.tbra[ce.x] : P.bra[ce.x];
+        const PairSet& ket = titems ? P.tket[ce.y] : P.ket[ce.y];
         FockArgs a{};
         a.bra = bra.d_pairs.ptr;
         a.bra_prims = bra.d_prims.ptr;
@@ -2532,7 +2616,7 @@ int record_batch(vlx_context* ctx, BatchPlan& P)
         a.k32 = nullptr;
         a.glim = nullptr;  // density-weighted screening: single-molecule builds only
         a.sc.ngroups = 0;
-        a.sc.nitems = static_cast<long long>(L.tiled ? L.titems.size() : L.items.size());
+        a.sc.nitems = static_cast<long long>(titems ? L.titems.size() : L.items.size());
         a.sc.nket = ket.size();
         a.sc.ithreshold = P.ithreshold;
         a.sc.same_class = (ce.x == ce.y) ? 1 : 0;
@@ -2552,6 +2636,8 @@ int record_batch(vlx_context* ctx, BatchPlan& P)
             } else {
                 ce.tiled(a, grid, s);
             }
+        } else if (L.mmd_tiled) {
+            ce.mmd_tiled(a, static_cast<int>(std::min<long long>(a.sc.nitems, ctx->tiled_grid)), s);
         } else if (L.mmd) {
             ce.mmd(a, static_cast<int>(std::min<long long>(a.sc.nitems, ctx->mmd_grid)), s);
         } else if (L.ksl) {

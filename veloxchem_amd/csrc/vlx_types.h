@@ -132,9 +132,10 @@ __host__ __device__ constexpr int vlx_pad16(int x) { return (x + 15) / 16 * 16; 
 __host__ __device__ constexpr int vlx_u_rows(int la, int lb) { return vlx_pad16(vlx_nherm(la + lb)); }
 __host__ __device__ constexpr int vlx_u_cols(int la, int lb) { return vlx_pad16((2 * la + 1) * (2 * lb + 1)); }
 
-// U arrays ([prim][vlx_u_rows][vlx_u_cols]) of the npairs pairs of one pair set.
-void vlx_launch_u_build(const PairInfo* pairs, const PrimPair* prims, int npairs, int la, int lb, double* u,
-                        hipStream_t s);
+// U arrays ([prim][vlx_u_rows][vlx_u_cols]) of the npairs pairs of one pair set, as bras or as
+// kets (signs of the ket Hermite functions).
+void vlx_launch_u_build(const PairInfo* pairs, const PrimPair* prims, int npairs, int la, int lb, bool ket,
+                        double* u, hipStream_t s);
 
 struct EriArgs {
     const PairInfo* bra;
@@ -176,6 +177,8 @@ struct ClassLaunchers {
     FockLaunchFn tiled_multi;  // multi-density form of `tiled` (FP64), or nullptr
     FockLaunchFn ksl;          // ket-stationary kernel with LDS accumulators (grid in wavefronts), or nullptr
     FockLaunchFn tiled_dlds;   // `tiled` (FP64, wide block) with the item's D blocks staged in LDS, or nullptr
+    FockLaunchFn mmd_tiled;    // `mmd` with LDS tiles (TileItem of ket pairs), or nullptr
+    int (*mmd_scratch)();      // bytes of LDS its wavefronts need beside the tiles
 };
 
 struct DiagLauncher {
@@ -197,3 +200,6 @@ struct DiagLauncher {
 #define VLX_DECLARE_KSL(la, lb, lc, ld) void launch_ksl_##la##lb##lc##ld(const FockArgs& a, int grid, hipStream_t s);
 #define VLX_DECLARE_DIAG(la, lb) void launch_diag_##la##lb(const DiagArgs& a, hipStream_t s);
 #define VLX_DECLARE_MMD(la, lb, lc, ld) void launch_mmd_##la##lb##lc##ld(const FockArgs& a, int grid, hipStream_t s);
+#define VLX_DECLARE_MMD_TILED(la, lb, lc, ld)                                              \
+    void launch_mmd_tiled_##la##lb##lc##ld(const FockArgs& a, int grid, hipStream_t s); \
+    int mmd_scratch_##la##lb##lc##ld();
