@@ -450,7 +450,10 @@ __device__ __forceinline__ double lds_at(const double* __restrict__ base, const 
     return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + byte);
 }
 
-constexpr int VLX_DIGEST_UNROLL = 5;  // terms of the digestion loaded together (term counts are odd)
+// terms of the digestion loaded together (term counts are odd): few wavefronts a SIMD wait for LDS
+// ((dd|dd) 0.336 -> 0.304 ms, (fd|dp) 1.57 -> 1.45), more of them are bound by the vector unit
+// ((dp|dp) 2.49 -> 2.64); 20 waters def2-TZVP, one stream
+constexpr int mmd_digest_unroll(int L) { return L >= 7 ? 5 : 1; }
 
 // What a lane of the MD kernels keeps for the whole launch.
 template <int la, int lb, int lc, int ld>
@@ -459,7 +462,8 @@ struct MmdLane {
     // byte offsets of R^0[p + q], two steps (row tile, column group) a register; masked rows and
     // columns read R^0[0] against zero rows of U
     unsigned ridx[(S::MX * S::KX + 1) / 2];
-    // the lane's entries of the R recursion: byte offsets of the two sources, factor and axis
+    // the lane's entries of the R recursion: byte offsets of the two sources, factor, byte offset of
+    // the component of P - Q in a row of seeds
     unsigned rsrc[S::KR];
     double rfac[S::KR];
     int raxis[S::KR];
@@ -483,7 +487,7 @@ struct MmdLane {
         for (int k = 0; k < S::KR; k++) {
             const int rr = g_hrec.e[min(lane + VLX_WAVE * k, S::nr - 1)];
             rsrc[k] = 8u * (rr & 511) | 8u * ((rr >> 9) & 511) << 16;
-            raxis[k] = (rr >> 18) & 3;
+            raxis[k] = 8 * ((rr >> 18) & 3);
             rfac[k] = static_cast<double>(rr >> 20);
         }
 #pragma unroll
@@ -512,11 +516,12 @@ struct MmdLane {
         const int step = gstep[k] & 0xffff, nv = (gstep[k] >> 16) & 0xff, wrap = gwrap[k] & 0xffff;
         int io = gib[k] & 0xffff, dof = gib[k] >> 16, c = 0;
         double v = 0.0;
-        for (int t = 0; t < terms; t += VLX_DIGEST_UNROLL) {
-            double x[VLX_DIGEST_UNROLL], d[VLX_DIGEST_UNROLL];
+        constexpr int UN = mmd_digest_unroll(S::L);
+        for (int t = 0; t < terms; t += UN) {
+            double x[UN], d[UN];
             // loads of several terms in flight; past the last one they repeat it
 #pragma unroll
-            for (int q = 0; q < VLX_DIGEST_UNROLL; q++) {
+            for (int q = 0; q < UN; q++) {
                 x[q] = lds_at(outs, io);
                 d[q] = lds_at(dblk, dof);
                 const bool more = t + q + 1 < terms, end = c + 1 == nv;
@@ -525,9 +530,86 @@ struct MmdLane {
                 c = end ? 0 : c + 1;
             }
 #pragma unroll
-            for (int q = 0; q < VLX_DIGEST_UNROLL; q++) v = t + q < terms ? fma(x[q], d[q], v) : v;
+            for (int q = 0; q < UN; q++) v = t + q < terms ? fma(x[q], d[q], v) : v;
         }
         return v;
+    }
+};
+
+// Per primitive quartet of up to 8 kets of one bra: P - Q and R^n_000 = w (-2 rho)^n F_n, n = 0..L, in
+// rows of an LDS table, one lane a primitive quartet.  All of it is the same for the 64 lanes that share
+// a quartet: computed there, a chain of two loads and the Boys function stood before every recursion
+// (20 waters def2-TZVP, one stream: (pp|pp) 5.1 -> 4.0 ms, (fp|dp) 3.94 -> 3.78).  The rows come in the
+// order in which mmd_block takes them (ket, bra primitive, ket primitive), CAP at a time.
+template <int L, bool RS>
+struct MmdSeeds {
+    static constexpr int CAP = 16, KETS = 8, stride = (L + 4) | 1;  // odd: rows start in different banks
+    static constexpr int size = CAP * stride;                      // doubles per wavefront
+    const PrimPair* __restrict__ bra_prims;
+    const PrimPair* __restrict__ ket_prims;
+    const double* __restrict__ boys_tab;
+    double omega2;
+    double* rows;
+    int lane, knp, kstart, before;  // lane t < KETS: primitives of ket t, first, primitive quartets before it
+    int total, next, filled;        // primitive quartets of the unit, the next to be taken, in the table up to
+
+    // kets of the unit: lane t's ket, taken or not
+    __device__ __forceinline__ void open(const PairInfo& bp, const PairInfo& kp, const bool take)
+    {
+        knp = kp.nprim;
+        kstart = kp.prim_start;
+        const int n = take ? bp.nprim * knp : 0;
+        int upto = n;
+#pragma unroll
+        for (int d = 1; d < KETS; d *= 2) {
+            const int o = __shfl_up(upto, d, VLX_WAVE);
+            upto += lane >= d ? o : 0;
+        }
+        before = upto - n;
+        total = __builtin_amdgcn_readlane(upto, KETS - 1);
+        next = filled = 0;
+    }
+    // row of the next primitive quartet
+    __device__ __forceinline__ const double* take(const PairInfo& bp)
+    {
+        if (next == filled) fill(bp);
+        return rows + (next++ - (filled - CAP)) * stride;
+    }
+    __device__ __forceinline__ void fill(const PairInfo& bp)
+    {
+        wave_lds_fence();
+        const int c = min(filled + lane, total - 1);
+        int t = 0;
+#pragma unroll
+        for (int k = 1; k < KETS; k++) t = c >= __builtin_amdgcn_readlane(before, k) ? k : t;
+        const int r = c - __shfl(before, t, VLX_WAVE), nk = __shfl(knp, t, VLX_WAVE), k0 = __shfl(kstart, t, VLX_WAVE);
+        const int ib = static_cast<int>((static_cast<float>(r) + 0.5f) / static_cast<float>(nk)), ik = r - ib * nk;
+        const PrimPair pb = bra_prims[bp.prim_start + ib];
+        const PrimPair pk = ket_prims[k0 + ik];
+        const double sz = pb.zeta + pk.zeta;
+        const double rho_c = pb.zeta * pk.zeta * vrcp<double>(sz);
+        double rho = rho_c, w = vrsqrt<double>(sz);
+        if constexpr (RS) {
+            const double sfac = omega2 / (omega2 + rho_c);
+            rho = rho_c * sfac;
+            w *= sqrt(sfac);
+        }
+        const double pqx = pb.px - pk.px, pqy = pb.py - pk.py, pqz = pb.pz - pk.pz;
+        double seed[L + 1];
+        boys_eval<L, double, true>(rho * (pqx * pqx + pqy * pqy + pqz * pqz), boys_tab, seed);
+        if (lane < CAP) {
+            double* row = rows + lane * stride;
+            row[0] = pqx;
+            row[1] = pqy;
+            row[2] = pqz;
+#pragma unroll
+            for (int n = 0; n <= L; n++) {
+                row[3 + n] = w * seed[n];
+                w *= -2.0 * rho;
+            }
+        }
+        filled += CAP;
+        wave_lds_fence();
     }
 };
 
@@ -535,10 +617,9 @@ struct MmdLane {
 // rbuf: R^n for even n in the first nr doubles, odd n in the second.
 template <int la, int lb, int lc, int ld, bool RS>
 __device__ __forceinline__ void mmd_block(const MmdLane<la, lb, lc, ld>& ln, const int lane, const PairInfo& bp,
-                                          const PairInfo& kp, const PrimPair* __restrict__ bra_prims,
-                                          const double* __restrict__ bra_u, const PrimPair* __restrict__ ket_prims,
-                                          const double* __restrict__ ket_u, const double* __restrict__ boys_tab,
-                                          const double omega2, double* __restrict__ rbuf, double* __restrict__ outs)
+                                          const PairInfo& kp, const double* __restrict__ bra_u,
+                                          const double* __restrict__ ket_u, MmdSeeds<la + lb + lc + ld, RS>& seeds,
+                                          double* __restrict__ rbuf, double* __restrict__ outs)
 {
     using S = MmdSizes<la, lb, lc, ld>;
     constexpr int L = S::L, MX = S::MX, KX = S::KX, MT = S::MT, NT = S::NT, KR = S::KR;
@@ -549,7 +630,6 @@ __device__ __forceinline__ void mmd_block(const MmdLane<la, lb, lc, ld>& ln, con
 #pragma unroll
         for (int m = 0; m < MT; m++) acc[nt][m] = vlx_d4{0.0, 0.0, 0.0, 0.0};
     for (int ib = 0; ib < bp.nprim; ib++) {
-        const PrimPair pb = bra_prims[bp.prim_start + ib];
         const double* ua = bra_u + (size_t)(bp.prim_start + ib) * (S::HA * S::SA) + lk * S::SA + lr;
         vlx_d4 x[S::XSUM ? NT : 1][MX];
         auto clear_x = [&](vlx_d4 (&t)[MX]) {
@@ -571,7 +651,6 @@ __device__ __forceinline__ void mmd_block(const MmdLane<la, lb, lc, ld>& ln, con
             for (int nt = 0; nt < NT; nt++) clear_x(x[nt]);
         }
         for (int ik = 0; ik < kp.nprim; ik++) {
-            const PrimPair pk = ket_prims[kp.prim_start + ik];
             const double* uc = ket_u + (size_t)(kp.prim_start + ik) * (S::HC * S::SC) + lk * S::SC + lr;
             double ucv[S::PRE_X ? NT : 1][S::PRE_X ? KX : 1];
             if constexpr (S::PRE_X) {
@@ -580,29 +659,12 @@ __device__ __forceinline__ void mmd_block(const MmdLane<la, lb, lc, ld>& ln, con
 #pragma unroll
                     for (int kq = 0; kq < KX; kq++) ucv[nt][kq] = uc[4 * kq * S::SC + 16 * nt];
             }
-            const double sz = pb.zeta + pk.zeta;
-            const double rho_c = pb.zeta * pk.zeta * vrcp<double>(sz);
-            double rho = rho_c, w = vrsqrt<double>(sz);
-            if constexpr (RS) {
-                const double sfac = omega2 / (omega2 + rho_c);
-                rho = rho_c * sfac;
-                w *= sqrt(sfac);
-            }
-            const double pqx = pb.px - pk.px, pqy = pb.py - pk.py, pqz = pb.pz - pk.pz;
-            double seed[L + 1];
-            boys_eval<L, double, true>(rho * (pqx * pqx + pqy * pqy + pqz * pqz), boys_tab, seed);
-            // R^n_000 = w (-2 rho)^n F_n
-            {
-                double f = w;
+            const double* row = seeds.take(bp);
+            double pq[KR], seed[L + 1];
 #pragma unroll
-                for (int n = 0; n <= L; n++) {
-                    seed[n] *= f;
-                    f *= -2.0 * rho;
-                }
-            }
-            double pq[KR];
+            for (int k = 0; k < KR; k++) pq[k] = lds_at(row, ln.raxis[k]);
 #pragma unroll
-            for (int k = 0; k < KR; k++) pq[k] = ln.raxis[k] == 0 ? pqx : (ln.raxis[k] == 1 ? pqy : pqz);
+            for (int n = 0; n <= L; n++) seed[n] = row[3 + n];
             // R levels n = L .. 0, one FMA and one product per entry
             if (lane == 0) rbuf[(L & 1) * S::nr] = seed[L];
 #pragma unroll
@@ -677,19 +739,28 @@ __global__ void __launch_bounds__(VLX_WAVE) __attribute__((amdgpu_waves_per_eu(M
     __shared__ double rbuf[2 * S::nr];
     __shared__ double outs[S::nsab * S::nscd];
     __shared__ double dblk[S::nout];
+    __shared__ double rows[MmdSeeds<S::L, RS>::size];
     const int lane = threadIdx.x;
     MmdLane<la, lb, lc, ld> ln;
     ln.init(lane);
+    MmdSeeds<S::L, RS> seeds{bra_prims, ket_prims, boys_tab, a.omega2, rows, lane};
+    unsigned long long taken = 0;
     for (long long it = blockIdx.x; it < a.nitems; it += gridDim.x) {
         const WorkItem wi = items[it];
         const MolDesc md = mols[wi.mol];
         const PairInfo bp = bra[wi.i0];
         for (int j = wi.j0; j < wi.i1; j++) {
+            // kets in units of up to 8; density-weighted screening (one quartet per wavefront)
+            if (((j - wi.j0) % MmdSeeds<S::L, RS>::KETS) == 0) {
+                const int n = min(wi.i1 - j, MmdSeeds<S::L, RS>::KETS);
+                const PairInfo kl = ket[j + min(lane, n - 1)];
+                const bool take = lane < n && (glim == nullptr || bp.bin + kl.bin <= quartet_bin_limit(glim, a.ngroups, bp.grp_a, bp.grp_b, kl.grp_a, kl.grp_b));
+                taken = __ballot(take);
+                seeds.open(bp, kl, take);
+            }
+            const int t = (j - wi.j0) % MmdSeeds<S::L, RS>::KETS;
+            if (!((taken >> t) & 1)) continue;
             const PairInfo kp = ket[j];
-            // density-weighted screening (wave-uniform: one quartet per wavefront)
-            if (glim != nullptr &&
-                bp.bin + kp.bin > quartet_bin_limit(glim, a.ngroups, bp.grp_a, bp.grp_b, kp.grp_a, kp.grp_b))
-                continue;
             // elements of the six blocks: their place in D and F', and the first density's D
             size_t goff[NR];
             double dval[NR];
@@ -698,7 +769,7 @@ __global__ void __launch_bounds__(VLX_WAVE) __attribute__((amdgpu_waves_per_eu(M
                 goff[k] = ln.place(k, lane, bp, kp, md.nao);
                 dval[k] = D0[md.base + goff[k]];
             }
-            mmd_block<la, lb, lc, ld, RS>(ln, lane, bp, kp, bra_prims, bra_u, ket_prims, ket_u, boys_tab, a.omega2, rbuf, outs);
+            mmd_block<la, lb, lc, ld, RS>(ln, lane, bp, kp, bra_u, ket_u, seeds, rbuf, outs);
             double sf = 1.0;
             if (bp.same) sf *= 0.5;
             if (kp.same) sf *= 0.5;
@@ -745,8 +816,8 @@ template <int la, int lb, int lc, int ld>
 struct MmdTile {
     using S = MmdSizes<la, lb, lc, ld>;
     static constexpr int NW = 4 * S::occupancy;  // one block fills a CU's registers
-    static constexpr int scratch = 2 * S::nr + S::nsab * S::nscd + S::nout;  // doubles per wavefront
-    static constexpr int KETS = 8;
+    static constexpr int scratch = 2 * S::nr + S::nsab * S::nscd + S::nout + MmdSeeds<S::L, false>::size;  // doubles per wavefront
+    static constexpr int KETS = MmdSeeds<S::L, false>::KETS;
 };
 
 template <int la, int lb, int lc, int ld, bool RS>
@@ -769,6 +840,7 @@ __global__ void __launch_bounds__((MmdTile<la, lb, lc, ld>::NW * VLX_WAVE))
     double* rbuf = tiles + a.tile_doubles + wave * T::scratch;
     double* outs = rbuf + 2 * S::nr;
     double* dblk = outs + S::nsab * S::nscd;
+    MmdSeeds<S::L, RS> seeds{bra_prims, ket_prims, boys_tab, a.omega2, dblk + S::nout, lane};
     for (int e = threadIdx.x; e < a.tile_doubles; e += NW * VLX_WAVE) tiles[e] = 0.0;
     MmdLane<la, lb, lc, ld> ln;
     ln.init(lane);
@@ -800,14 +872,24 @@ __global__ void __launch_bounds__((MmdTile<la, lb, lc, ld>::NW * VLX_WAVE))
             const double* t = y == 1 ? t_jab : y == 2 ? (x == 0 ? t_kac : t_kbc) : x == 0 ? t_kad : x == 1 ? t_kbd : t_jcd;
             tbase[k] = static_cast<int>(t - tiles) + i * tstride[k] + j;
         }
-        const int nunit = (ti.j1 - ti.j0 + T::KETS - 1) / T::KETS;
+        // kets of a unit: fewer where the item has few, for about 8 units a wavefront (8 kets always left
+        // wavefronts idle at the end of items: (dd|dd) 0.30 -> 0.18 ms, (fp|dp) 3.8 -> 3.35 ms, (fp|dp) of
+        // two waters 0.17 -> 0.10 ms)
+        const int ku = max(1, min(T::KETS, (ti.i1 - ti.i0) * (ti.j1 - ti.j0) / (8 * NW)));
+        const int nunit = (ti.j1 - ti.j0 + ku - 1) / ku;
         for (int u = wave; u < (ti.i1 - ti.i0) * nunit; u += NW) {
-            const int i = ti.i0 + u / nunit, j0 = ti.j0 + u % nunit * T::KETS;
+            const int i = ti.i0 + u / nunit, j0 = ti.j0 + u % nunit * ku;
             const PairInfo bp = pairs_bra[i];
-            for (int j = j0; j < min(ti.j1, j0 + T::KETS); j++) {
-                const PairInfo kp = pairs_ket[j];
-                if (a.ithreshold >= 0 && bp.bin + kp.bin > ilim) break;  // kets go by bin
-                if (a.same_class && bp.rank < kp.rank) continue;
+            const int n = min(ti.j1 - j0, ku);
+            const PairInfo kl = pairs_ket[j0 + min(lane, n - 1)];
+            const bool take = lane < n && !(a.ithreshold >= 0 && bp.bin + kl.bin > ilim) &&
+                              !(a.same_class && bp.rank < kl.rank);
+            const unsigned long long taken = __ballot(take);
+            if (taken == 0) continue;
+            seeds.open(bp, kl, take);
+            for (int t = 0; t < n; t++) {
+                if (!((taken >> t) & 1)) continue;
+                const PairInfo kp = pairs_ket[j0 + t];
                 int toff[NR];
                 double dval[NR];
 #pragma unroll
@@ -818,8 +900,7 @@ __global__ void __launch_bounds__((MmdTile<la, lb, lc, ld>::NW * VLX_WAVE))
                     toff[k] = tbase[k] + row * tstride[k] + col;
                     dval[k] = D[ln.place(k, lane, bp, kp, md.nao)];
                 }
-                mmd_block<la, lb, lc, ld, RS>(ln, lane, bp, kp, bra_prims, bra_u, ket_prims, ket_u, boys_tab, a.omega2, rbuf,
-                                              outs);
+                mmd_block<la, lb, lc, ld, RS>(ln, lane, bp, kp, bra_u, ket_u, seeds, rbuf, outs);
                 double sf = 1.0;
                 if (bp.same) sf *= 0.5;
                 if (kp.same) sf *= 0.5;
