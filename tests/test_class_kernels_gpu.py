@@ -18,6 +18,12 @@ EPS = np.finfo(float).eps
     (5, 'def2-svp', 'j', 0.0, 10),        # 12 + 3 atoms, J tiles only
     (5, 'def2-svp', 'kx_rs', 0.4, 12),    # attenuated exchange
     (6, 'def2-tzvp', '2jk', 0.0, 12),     # (pp|pp) chunks past 64 entries, items of several chunks
+    # Coulomb builds: the default choice goes through Hermite densities
+    (1, 'def2-svp', 'j', 0.0, 12),        # ranks of fewer entries than a block, one stage of kets
+    (2, 'def2-tzvp', 'j_rs', 0.5, 12),    # f shells: ranks 0 to 6, attenuated
+    (3, 'def2-svpd', 'j', 0.0, 6),        # bras that meet no ket of some ranks
+    (4, 'def2-tzvp', 'j', 0.0, 12),       # ragged last blocks and stages
+    (2, 'def2-svp', 'j', 0.0, -1),        # unscreened: the class kernels
 ])
 def test_class_kernels_agree(waters, basis, label, omega, ithreshold):
     mol = water_cluster(waters, 6.0, 3)

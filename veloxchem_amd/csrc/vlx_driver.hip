@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "../../include/vlxfock.h"
+#include "vlx_jtypes.h"
 #include "vlx_types.h"
 
 #include "gen/dispatch.inc"
@@ -252,6 +253,7 @@ constexpr long long TILE_ITEM_UNITS = 1024;
 // largest tiled item of the matrix-core MD kernel, in shell quartets
 constexpr long long MMD_ITEM_UNITS = 2048;
 
+constexpr int NPAIR_MAX = 10;  // pair classes of s, p, d and f shells
 constexpr int NSIDE = 4;  // side streams that run class kernels concurrently
 
 constexpr int NO_FP32 = 99;  // bin-sum threshold that sends no quartet to FP32
@@ -315,6 +317,7 @@ struct vlx_context {
     // largest grid (one wavefront per block) of a matrix-core MD launch (VLX_MMD_GRID): on the 64-water
     // def2-TZVP build 16384 / 32768 / 65536 measured 0.775 / 0.786 / 0.793 builds/s
     int mmd_grid = 65536;
+    bool use_jengine = true;        // Coulomb builds through Hermite densities (VLX_JENGINE)
     bool u_pending = false;         // U arrays still being built on the stream (ensure_u, finish_u)
     // kets per matrix-core MD work item (VLX_MMD_KETS): on the 64-water def2-TZVP build the MD classes
     // took 333.2 / 327.1 / 332.1 / 342.9 ms with 1 / 2 / 4 / 8 kets
@@ -365,8 +368,33 @@ struct vlx_context {
     std::vector<std::unique_ptr<BatchPlan>> plans;  // batched builds, most recently used last
 };
 
+// Coulomb build through Hermite densities (j_kernels.h): the primitives of a screener's binned pairs in
+// one list per Hermite rank la + lb, sorted by bin, and the work items per bin-sum limit.
+struct JEngine {
+    static constexpr int NRANK = 2 * VLX_GEN_LMAX + 1;
+    bool ready = false;
+    int n[NRANK] = {0};              // entries
+    int cnt[NRANK][NBINS] = {{0}};   // entries with bin <= b
+    std::vector<unsigned char> bins[NRANK];
+    DevBuf<char> arena;              // index lists, bins and counts
+    DevBuf<double> work;             // rows and J_p of every rank
+    DevView<int> pair_of[NPAIR_MAX], entry0[NPAIR_MAX], d_cnt[NRANK];
+    DevView<unsigned char> d_bins[NRANK];
+    DevView<double> rows[NRANK], jp[NRANK];
+    struct Launch {
+        int lab, lcd, first, count;
+        double cost;
+    };
+    struct Items {
+        std::vector<Launch> launches;  // most expensive first
+        DevBuf<JItem> d_items;
+    };
+    std::map<int, Items> items;      // by ithreshold
+};
+
 struct vlx_screener {
     vlx_context* ctx = nullptr;
+    JEngine jengine;
     int nshells = 0, nao = 0;
     std::vector<int> l, nprim, prim_offset, ao_base, ao_stride;
     std::vector<double> exps, norms, centers;
@@ -1219,6 +1247,7 @@ int vlx_context_create(int device, vlx_context** out)
     if (const char* e = std::getenv("VLX_LAUNCH_ORDER")) ctx->launch_by_cost = std::atoi(e) != 0;
     if (const char* e = std::getenv("VLX_TILED_GRID")) ctx->tiled_grid = std::max(1, std::atoi(e));
     if (const char* e = std::getenv("VLX_TILE_ITEMS")) ctx->tile_items = std::max(1, std::atoi(e));
+    if (const char* e = std::getenv("VLX_JENGINE")) ctx->use_jengine = std::atoi(e) != 0;
     if (const char* e = std::getenv("VLX_MMD_GRID")) ctx->mmd_grid = std::max(1, std::atoi(e));
     if (const char* e = std::getenv("VLX_MMD_KETS")) ctx->mmd_kets = std::max(1, std::min(64, std::atoi(e)));
     if (const char* e = std::getenv("VLX_MAX_TILE_LDS")) ctx->max_tile_lds = std::max(16 * 1024, std::atoi(e));
@@ -1960,11 +1989,11 @@ namespace {
 // density c at d_density + c nao^2 and F + c nao^2, factors (fj, fk) of density c at dfac[2 c]
 // (device, and on the host in ctx->h_dfac); fj and fk are then unused.  det: the same kernels with
 // fixed-point accumulation, F being the accumulator array (two words per element); the schedules
-// must be untiled.
+// must be untiled.  lmin: only the classes of total angular momentum lmin or more.
 int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::unique_ptr<ClassSchedule>>& list,
                     const double* d_density, double* F, double fj, double fk, double omega2, int ithreshold,
                     hipStream_t stream, int solo = -1, bool allow_timing = true, const int* glim = nullptr,
-                    int ndens = 1, const double* dfac = nullptr, bool det = false)
+                    int ndens = 1, const double* dfac = nullptr, bool det = false, int lmin = 0)
 {
     const bool multi = ndens > 1 || det;
     const bool timing = ctx->timing && allow_timing;
@@ -1975,6 +2004,7 @@ int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::
         const ClassSchedule& sch = *schp;
         if (solo >= 0 && (sch.stream < 0) != (solo == 1)) continue;
         const auto& ce = g_class_table[sch.entry];
+        if (ce.la + ce.lb + ce.lc + ce.ld < lmin) continue;
         const bool titems = sch.tiled || sch.mmd_tiled;
         const PairSet& bra = titems ? (unscreened ? scr->all_tiled_bra[ce.x] : scr->kept_tiled_bra[ce.x])
                                     : (unscreened ? scr->all_bra[ce.x] : scr->kept_bra[ce.x]);
@@ -2179,6 +2209,151 @@ int multi_pass(vlx_context* ctx, vlx_screener* scr, const double* dens, int m, c
     return VLX_OK;
 }
 
+// Lists of the Coulomb engine: the primitives of the binned pairs of each Hermite rank in order of bin
+// (the pairs of a class are already in that order, the classes of a rank are merged).
+int j_prepare(vlx_screener* s)
+{
+    JEngine& J = s->jengine;
+    if (J.ready) return VLX_OK;
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    std::vector<std::vector<int>> pair_of(s->kept.size()), entry0(s->kept.size());
+    size_t bytes = 0, doubles = 0;
+    for (int r = 0; r < JEngine::NRANK; r++) {
+        int count[NBINS] = {0}, at[NBINS];
+        for (const PairSet& ps : s->kept)
+            if (ps.size() > 0 && ps.la + ps.lb == r)
+                for (const PairInfo& p : ps.pairs) count[p.bin] += p.nprim;
+        int total = 0;
+        J.bins[r].clear();
+        for (int b = 0; b < NBINS; b++) {
+            at[b] = total;
+            total += count[b];
+            J.cnt[r][b] = total;
+            J.bins[r].insert(J.bins[r].end(), count[b], static_cast<unsigned char>(b));
+        }
+        J.n[r] = total;
+        for (size_t c = 0; c < s->kept.size(); c++) {
+            const PairSet& ps = s->kept[c];
+            if (ps.size() == 0 || ps.la + ps.lb != r) continue;
+            pair_of[c].resize(ps.prims.size());
+            for (int i = 0; i < ps.size(); i++) {
+                const PairInfo& p = ps.pairs[i];
+                entry0[c].push_back(at[p.bin]);
+                at[p.bin] += p.nprim;
+                for (int q = 0; q < p.nprim; q++) pair_of[c][p.prim_start + q] = i;
+            }
+            bytes += up(pair_of[c].size() * sizeof(int)) + up(entry0[c].size() * sizeof(int));
+        }
+        bytes += up(NBINS * sizeof(int)) + up(total);
+        doubles += (size_t)total * (j_row(r) + j_nherm(r));
+    }
+    std::vector<char> host(bytes);
+    HIP_TRY(J.arena.alloc(bytes));
+    HIP_TRY(J.work.alloc(doubles));
+    size_t off = 0;
+    auto put = [&](const void* src, size_t n, auto& view) {
+        if (n) std::memcpy(host.data() + off, src, n);
+        view.ptr = reinterpret_cast<decltype(view.ptr)>(J.arena.ptr + off);
+        off += up(n);
+    };
+    for (size_t c = 0; c < s->kept.size(); c++) {
+        if (s->kept[c].size() == 0) continue;
+        put(pair_of[c].data(), pair_of[c].size() * sizeof(int), J.pair_of[c]);
+        put(entry0[c].data(), entry0[c].size() * sizeof(int), J.entry0[c]);
+    }
+    double* w = J.work.ptr;
+    for (int r = 0; r < JEngine::NRANK; r++) {
+        put(J.cnt[r], NBINS * sizeof(int), J.d_cnt[r]);
+        put(J.bins[r].data(), J.bins[r].size(), J.d_bins[r]);
+        J.rows[r].ptr = w;
+        w += (size_t)J.n[r] * j_row(r);
+        J.jp[r].ptr = w;
+        w += (size_t)J.n[r] * j_nherm(r);
+    }
+    HIP_TRY(hipMemcpy(J.arena.ptr, host.data(), bytes, hipMemcpyHostToDevice));
+    J.ready = true;
+    return VLX_OK;
+}
+
+// Work items of every pair of ranks with LAB + LCD <= J_LMAX at one bin-sum limit: JBLOCK bras, with the
+// kets of the first (which has the smallest bin) split so that a launch has about 2048 blocks.
+int j_items(vlx_screener* s, int ithr, JEngine::Items** out)
+{
+    JEngine& J = s->jengine;
+    auto it = J.items.find(ithr);
+    if (it == J.items.end()) {
+        JEngine::Items I;
+        std::vector<JItem> all;
+        for (int x = 0; x < JEngine::NRANK; x++)
+            for (int y = 0; y < JEngine::NRANK && x + y <= J_LMAX; y++) {
+                auto kets = [&](int i0) {
+                    const int lim = ithr - J.bins[x][i0];
+                    return lim < 0 ? 0 : J.cnt[y][std::min(lim, NBINS - 1)];
+                };
+                long long visits = 0;
+                for (int i0 = 0; i0 < J.n[x]; i0 += JBLOCK) visits += kets(i0);
+                const int step = static_cast<int>(std::max(64LL, (visits / 2048 + 63) / 64 * 64));
+                const int first = static_cast<int>(all.size());
+                for (int i0 = 0; i0 < J.n[x]; i0 += JBLOCK)
+                    for (int k = 0, k1 = kets(i0); k < k1; k += step) all.push_back({i0, k, std::min(k1, k + step)});
+                if (all.size() == (size_t)first) continue;
+                std::stable_sort(all.begin() + first, all.end(),
+                                 [](const JItem& a, const JItem& b) { return a.k1 - a.k0 > b.k1 - b.k0; });
+                const double per = 70.0 + 2.0 * j_nherm(x + y) + j_nherm(x) * j_nherm(y);
+                I.launches.push_back({x, y, first, static_cast<int>(all.size()) - first, per * visits});
+            }
+        std::sort(I.launches.begin(), I.launches.end(),
+                  [](const JEngine::Launch& a, const JEngine::Launch& b) { return a.cost > b.cost; });
+        HIP_TRY(I.d_items.upload(all));
+        it = J.items.emplace(ithr, std::move(I)).first;
+    }
+    *out = &it->second;
+    return VLX_OK;
+}
+
+// The Hermite densities of D on the context stream, with the J_p cleared (before), or F' from the J_p
+// (after).
+int j_transform(vlx_context* ctx, vlx_screener* s, bool before, const double* D, double factor, double* F)
+{
+    JEngine& J = s->jengine;
+    for (size_t c = 0; c < s->kept.size(); c++) {
+        const PairSet& ps = s->kept[c];
+        if (ps.size() == 0) continue;
+        const int r = ps.la + ps.lb;
+        const JPrep a{ps.d_pairs.ptr, ps.d_prims.ptr, J.pair_of[c].ptr, J.entry0[c].ptr, static_cast<int>(ps.prims.size()),
+                      s->nao, D, J.rows[r].ptr, J.jp[r].ptr, factor, F};
+        if (before) vlx_launch_j_density(ps.la, ps.lb, a, ctx->stream);
+        else vlx_launch_j_fock(ps.la, ps.lb, a, ctx->stream);
+    }
+    HIP_TRY(hipGetLastError());
+    return VLX_OK;
+}
+
+int j_launch(vlx_context* ctx, vlx_screener* s, const JEngine::Items& I, double omega2, int ithr)
+{
+    JEngine& J = s->jengine;
+    double load[NSIDE] = {0.0};
+    for (const auto& l : I.launches) {
+        const int k = static_cast<int>(std::min_element(load, load + ctx->nstreams) - load);
+        load[k] += l.cost;
+        JArgs a{};
+        a.bra = J.rows[l.lab].ptr;
+        a.bra_bin = J.d_bins[l.lab].ptr;
+        a.ket = J.rows[l.lcd].ptr;
+        a.jp = J.jp[l.lab].ptr;
+        a.items = I.d_items.ptr + l.first;
+        a.boys_tab = ctx->d_boys.ptr + (size_t)(l.lab + l.lcd) * BOYS_TAB_SIZE;
+        a.ket_cnt = J.d_cnt[l.lcd].ptr;
+        a.omega2 = omega2;
+        a.nbra = J.n[l.lab];
+        a.nitems = l.count;
+        a.ithreshold = ithr;
+        vlx_launch_j(l.lab, l.lcd, a, ctx->side[k]);
+    }
+    HIP_TRY(hipGetLastError());
+    return VLX_OK;
+}
+
 // scratch = nullptr: F' and the max|D| slot live in context buffers (allocated on first use) and
 // missing schedules are built.  Otherwise F' is `scratch` (nao x nao doubles) and max|D| the
 // slot `scratch_dmax`, the schedules must exist already and nothing is allocated.
@@ -2249,16 +2424,38 @@ int fock_build(vlx_context* ctx, vlx_screener* scr, const double* d_density, dou
     std::vector<std::unique_ptr<ClassSchedule>>* list = nullptr;
     rc = get_schedules(scr, ithreshold, k32, &list, !no_alloc);
     if (rc) return rc;
-    rc = enqueue_classes(ctx, scr, *list, d_density, facc, fj, fk, omega2, ithreshold, nullptr, 1, !no_alloc, glim);
+    // Coulomb alone: through Hermite densities, the classes of higher angular momentum by their kernels.
+    // The lists and J_p are the screener's: a build without allocation, of which several may be in flight
+    // in captured graphs, keeps to the class kernels, as do forced variants, per-class timing and the
+    // modes that need quartets
+    const bool hermite = fk == 0.0 && fj != 0.0 && ithreshold >= 0 && k32 == NO_FP32 && glim == nullptr && !no_alloc &&
+                         !ctx->timing && ctx->force_variant < 0 && ctx->use_jengine;
+    const int lmin = hermite ? J_LMAX + 1 : 0;
+    JEngine::Items* ji = nullptr;
+    if (hermite) {
+        rc = j_prepare(scr);
+        if (!rc) rc = j_items(scr, ithreshold, &ji);
+        if (!rc) rc = j_transform(ctx, scr, true, d_density, fj, facc);
+        if (rc) return rc;
+    }
+    rc = enqueue_classes(ctx, scr, *list, d_density, facc, fj, fk, omega2, ithreshold, nullptr, 1, !no_alloc, glim, 1,
+                         nullptr, false, lmin);
     if (rc) return rc;
     HIP_TRY(hipEventRecord(ctx->ev_start, ctx->stream));
     for (int k = 0; k < NSIDE; k++) HIP_TRY(hipStreamWaitEvent(ctx->side[k], ctx->ev_start, 0));
     // the side streams join the context stream also when a launch fails part-way, so that
     // work ordered on the context stream (copies, frees) never overtakes a queued kernel
-    rc = enqueue_classes(ctx, scr, *list, d_density, facc, fj, fk, omega2, ithreshold, nullptr, 0, !no_alloc, glim);
+    if (hermite) rc = j_launch(ctx, scr, *ji, omega2, ithreshold);
+    if (!rc)
+        rc = enqueue_classes(ctx, scr, *list, d_density, facc, fj, fk, omega2, ithreshold, nullptr, 0, !no_alloc, glim, 1,
+                             nullptr, false, lmin);
     const int rj = join_side_streams(ctx);
     if (rc) return rc;
     if (rj) return rj;
+    if (hermite) {
+        rc = j_transform(ctx, scr, false, d_density, fj, facc);
+        if (rc) return rc;
+    }
     if (anti_coef == 0.0) symmetrize_kernel<<<sg, 256, 0, ctx->stream>>>(facc, d_fock_out, n);
     else antisym_add_kernel<<<sg, 256, 0, ctx->stream>>>(facc, d_fock_out, n, anti_coef);
     HIP_TRY(hipGetLastError());
