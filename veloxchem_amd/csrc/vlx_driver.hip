@@ -892,6 +892,7 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         auto sch = std::make_unique<ClassSchedule>();
         sch->entry = e;
         // exact quartet counts, from the ket side (ket order is sorted by bin)
+        long long ket_prims = 0;  // ket primitives over all quartets
         for (int j = 0; j < ket.size(); j++) {
             long long lo = 0, hi;
             if (unscreened) {
@@ -904,6 +905,7 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
             if (hi <= lo) continue;
             const PairSet& rk = same ? ket : bra;  // prefix sums in an order where [lo, hi) is contiguous
             sch->quartets += hi - lo;
+            ket_prims += (hi - lo) * ket.pairs[j].nprim;
             sch->prim_quartets += (long long)ket.pairs[j].nprim * (rk.nprim_prefix[hi] - rk.nprim_prefix[lo]);
         }
         const int* gm = s->grp_max;
@@ -912,20 +914,34 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         const int L = ce.la + ce.lb + ce.lc + ce.ld;
         const int nsph = (2 * ce.la + 1) * (2 * ce.lb + 1) * (2 * ce.lc + 1) * (2 * ce.ld + 1);
         const bool can_tile = s->ctx->use_tiled && ce.tiled && L <= s->ctx->tiled_lmax && tile_lds <= s->ctx->max_tile_lds;
-        // default: tiled for L <= 4 (and for L = 5 blocks of <= 75 integrals when tiled_lmax
-        // allows it); the autotuner's choice, or the one being timed, overrides it
-        int var = (can_tile && (L <= 4 || nsph <= 75)) ? (s->ctx->tiled_waves == 4 ? VARIANT_TILED4 : VARIANT_TILED_WIDE)
-                                                      : VARIANT_UNTILED;
+        // default: tiled for L <= 4 and for L = 5 blocks of <= 75 integrals; the autotuner's choice, or
+        // the one being timed, overrides it.  Lanes take single primitives instead of runs of up to 3 in
+        // classes of L >= 4 whose kets have few: a lane's loop is then the same length in every lane.
+        // One stream, runs / single primitives, at ket primitives a quartet: 1.3 (ds| def2-TZVP (dp|ds) 2.53 /
+        // 2.11 ms, (fs|ds) 1.70 / 1.49 (20 waters), 1.45 (pp| def2-SVPD (ds|pp) 1.48 / 1.23, (pp|pp) 1.71 /
+        // 1.48 (13 waters), 1.5 (ds| def2-SVP 1.31 / 1.09 (32 waters); but 1.7 (ds| def2-SVPD (ds|ds)
+        // 0.44 / 0.50, 1.9 (pp| def2-TZVP (ds|pp) 1.54 / 1.69.  (dp|pp), 135 integrals: untiled / tiled
+        // single primitives 11.3 / 7.5 ms at 1.45, 3.7 / 4.5 at 1.9
+        const bool few_prims = L >= 4 && ket_prims * 2 < sch->quartets * 3;
+        int var = VARIANT_UNTILED;
+        if (can_tile && (L <= 4 || nsph <= 75 || (L == 5 && few_prims))) {
+            if (s->ctx->tiled_waves == 4) var = few_prims ? VARIANT_TILED4_P1 : VARIANT_TILED4;
+            else var = few_prims ? VARIANT_TILED_WIDE_P1 : VARIANT_TILED_WIDE;
+        }
         // The others: a lane of the generated kernels runs a quartet by itself and spills where the
         // block is large, a wavefront of the matrix-core kernel shares it.  One stream, generated /
-        // matrix-core, 20 waters def2-TZVP: (fd|pp) 6.3 / 1.9 ms, (dd|dp) 5.2 / 1.2, (dp|dp) 4.1 / 2.5,
-        // (fd|ds) 2.5 / 2.4, (fp|pp) 4.4 / 4.8, but (fp|fs) 4.0 / 4.4, (dp|pp) 3.9 / 6.5 and
-        // (ff|ps) 1.9 / 2.7: the line is at 175 integrals.  Smaller blocks are matrix-core as well
-        // while a launch has too few quartets for a lane each: the generated kernels then take the
-        // time of one lane ((dp|pp) of one water, 144 primitive quartets, 0.18 / 0.08 ms; of two waters
-        // def2-TZVP, 6000, 0.39 / 0.16; (fp|fs) there 0.82 / 0.15), and lose it at about 2e5
-        // (of the whole launch: a batch's molecules share it)
-        if (var == VARIANT_UNTILED && ce.mmd && (nsph >= 175 || sch->prim_quartets * share < 200000)) var = VARIANT_MMD;
+        // matrix-core, 20 waters def2-TZVP: (fd|pp) 6.3 / 1.8 ms, (dd|dp) 5.2 / 1.1, (dp|dp) 4.1 / 2.6,
+        // (fd|ds) 2.5 / 1.9, (fp|pp) 4.4 / 4.2, but (fd|ps) 1.9 / 4.5 and (fp|ds) 3.0 / 5.6: blocks of 175
+        // integrals or more.  The generated kernels gain on it while a launch grows, since more lanes hide
+        // their latencies: 64 waters (fp|pp) 48 / 62, (fd|ds) 22 / 31, (dd|pp) 29 / 19, so blocks below 225
+        // integrals go back to them at 2e6 primitive quartets.  Smaller blocks are matrix-core while a launch
+        // has too few quartets for a lane each: the generated kernels then take the time of one lane
+        // ((dp|pp) of one water, 144 primitive quartets, 0.18 / 0.08 ms; of two waters def2-TZVP, 6000,
+        // 0.39 / 0.16; (fp|fs) there 0.82 / 0.15), and lose it at about 2e5
+        // (quartets of the whole launch: a batch's molecules share it)
+        const long long launch = sch->prim_quartets * share;
+        if (var == VARIANT_UNTILED && ce.mmd && (nsph >= 225 || launch < 200000 || (nsph >= 175 && launch < 2000000)))
+            var = VARIANT_MMD;
         if (s->ctx->force_variant >= 0) {
             var = s->ctx->force_variant;
         } else {
