@@ -860,14 +860,17 @@ int ensure_unscreened(vlx_screener* s)
 // create = false: only a schedule built earlier is returned (no host or device allocation);
 // without one the call fails.
 // share: the builds that run side by side in one launch (a batch's molecules), each aiming at its
-// share of the tiled items.  direct: the matrix-core MD classes with the work items of the direct
-// digestion (multi-density and deterministic builds).
+// share of the tiled items.  use: USE_DIRECT gives the matrix-core MD classes the work items of the
+// direct digestion (multi-density and deterministic builds); USE_BATCH leaves items and U arrays on
+// the host, for the batch's own concatenated lists (40 molecules: the uploads were 30 ms of the first
+// pass).
+enum ScheduleUse { USE_BUILD = 0, USE_DIRECT = 1, USE_BATCH = 2 };
 int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_ptr<ClassSchedule>>** out,
-                  bool create = true, int share = 1, bool direct = false)
+                  bool create = true, int share = 1, ScheduleUse use = USE_BUILD)
 {
     const int tile_items = std::max(1, s->ctx->tile_items / share);
     const std::pair<int, int> key{((ithr + 1) * 128 + k32) * (NVARIANTS + 1) + (s->ctx->force_variant + 1),
-                                  2 * tile_items + (direct ? 1 : 0)};
+                                  4 * tile_items + use};
     auto it = s->schedules.find(key);
     if (it != s->schedules.end()) {
         *out = &it->second;
@@ -961,7 +964,7 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         if (ce.variant == VLX_WAVE_MD) var = VARIANT_MMD;  // no generated kernel
         sch->variant = var;
         sch->mmd = var == VARIANT_MMD;
-        sch->mmd_tiled = sch->mmd && !direct && s->ctx->use_tiled && ce.mmd_tiled &&
+        sch->mmd_tiled = sch->mmd && use != USE_DIRECT && s->ctx->use_tiled && ce.mmd_tiled &&
                          tile_lds + ce.mmd_scratch() <= 160 * 1024 - 1024;
         sch->ksl = var == VARIANT_KSL;
         sch->dlds = var == VARIANT_TILED_DLDS;
@@ -1162,6 +1165,10 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
             }
         }
         if (sch->items.empty() && sch->titems.empty() && sch->titems32.empty()) continue;
+        if (use == USE_BATCH) {
+            list.push_back(std::move(sch));
+            continue;
+        }
         if (sch->mmd_tiled) {
             int rc = ensure_u(s->ctx, unscreened ? s->all_tiled_bra[ce.x] : s->kept_tiled_bra[ce.x], false);
             if (!rc) rc = ensure_u(s->ctx, unscreened ? s->all_tiled[ce.y] : s->kept_tiled[ce.y], true);
@@ -2200,7 +2207,7 @@ int multi_pass(vlx_context* ctx, vlx_screener* scr, const double* dens, int m, c
     std::vector<std::unique_ptr<ClassSchedule>>* list = nullptr;
     const int saved_variant = ctx->force_variant;
     if (det) ctx->force_variant = VARIANT_UNTILED;
-    int rc = get_schedules(scr, ithreshold, NO_FP32, &list, true, 1, true);
+    int rc = get_schedules(scr, ithreshold, NO_FP32, &list, true, 1, USE_DIRECT);
     ctx->force_variant = saved_variant;
     if (rc) return rc;
     const bool single = m == 1 && !det;
@@ -2566,7 +2573,7 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
     const bool unscreened = P.ithreshold < 0;
     std::vector<std::vector<std::unique_ptr<ClassSchedule>>*> lists(nmol, nullptr);
     for (int m = 0; m < nmol; m++) {
-        const int rc = get_schedules(P.scrs[m], P.ithreshold, NO_FP32, &lists[m], true, nmol);
+        const int rc = get_schedules(P.scrs[m], P.ithreshold, NO_FP32, &lists[m], true, nmol, USE_BATCH);
         if (rc) return rc;
     }
     // the four orders of every pair class, and each molecule's offsets in them
