@@ -37,7 +37,7 @@ def test_class_kernels_agree(waters, basis, label, omega, ithreshold):
     # an element sums up to n^2 products I D in an order of each kernel's own; the rounding errors of
     # n^2 terms are independent, so they grow as n eps on each side
     try:
-        for v in (0, -1, 1, 2, 3, 4, 5):
+        for v in (0, -1, 1, 2, 3, 4, 5, 6):
             _native.check(lib.vlx_context_set_variant(ctx, v))
             mats[v] = np.asarray(drv.compute(scr, D, label, 0.5, omega, ithreshold))
     finally:
@@ -71,3 +71,23 @@ def test_direct_digestion_of_matrix_core_classes():
             assert np.max(np.abs(g - one)) <= 2 * n * EPS * max(1.0, np.max(np.abs(one)))
     finally:
         _native.check(lib.vlx_context_set_variant(ctx, -1))
+
+
+def test_default_kernels_of_large_launches():
+    """2.5e6 quartets and more in several classes: the default there against the untiled kernels."""
+    mol = water_cluster(36, 2.7 * 36 ** (1.0 / 3.0), 3)
+    bas = MolecularBasis.read(mol, 'def2-tzvp')
+    scr = T4CScreener()
+    scr.partition(bas, mol, 'eri')
+    n = bas.get_dimensions_of_basis()
+    D = pseudo_density(n, 180, seed=9)
+    drv, ctx, lib = FockDriver(), _native.context(), _native.lib()
+    g = np.asarray(drv.compute(scr, D, '2jk', 0.0, 0.0, 12))
+    names = {c: _native.class_kernel(scr, 12, c) for c in ((2, 1, 1, 1), (3, 0, 3, 0), (3, 0, 2, 0))}
+    try:
+        _native.check(lib.vlx_context_set_variant(ctx, 0))
+        ref = np.asarray(drv.compute(scr, D, '2jk', 0.0, 0.0, 12))
+    finally:
+        _native.check(lib.vlx_context_set_variant(ctx, -1))
+    assert any('ksl' in k for k in names.values()), names
+    assert np.max(np.abs(g - ref)) <= 2 * n * EPS * max(1.0, np.max(np.abs(ref)))

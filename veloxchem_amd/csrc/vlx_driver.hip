@@ -945,6 +945,20 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         const long long launch = sch->prim_quartets * share;
         if (var == VARIANT_UNTILED && ce.mmd && (nsph >= 225 || launch < 200000 || (nsph >= 175 && launch < 2000000)))
             var = VARIANT_MMD;
+        // Ket-stationary items with LDS accumulators, in large launches: their bra walks are then long, and
+        // keep three of the six blocks from the global atomics that the bra-stationary form sends all six
+        // to; the tiled form's chunks, of one group pair each, hold fewer kets the larger the system.  One
+        // stream, default before / these, by quartets: bra-stationary (dp|pp) 2.0e6 3.7 / 4.2 ms, 4.0e6 7.5 /
+        // 5.5, 3.2e7 57 / 32; (fs|fs) 1.7e6 4.97 / 4.95, 1.3e7 33 / 8; (dd|ds) 1.9e6 4.7 / 5.0, 7.2e6 17.7 /
+        // 15.0; but (fp|pp) 1.4e7 44 / 51, (fp|fs) 39 / 48.  Tiled (dp|ds) 6.0e6 4.8 / 5.7, 1.2e7 11.6 / 10.4,
+        // 4.8e7 64 / 36; (fs|pp) 4.8e6 3.0 / 3.5, 9.8e6 6.8 / 4.8; (fs|ds) 7.2e6 3.5 / 4.0, 1.5e7 8.3 / 6.3
+        // (def2-TZVP); def2-SVPD (dp|ds) 2.6e7 20.7 / 16.6, tiled (dp|pp) 6.1e6 7.5 / 6.6; but (pp|pp)
+        // 5.1e7 12 / 28
+        const long long launch_q = sch->quartets * share;
+        if (ce.ksl && nsph <= 135 &&
+            ((var == VARIANT_UNTILED && launch_q >= 2500000) ||
+             (variant_tiled(var) && L == 5 && ce.lc + ce.ld >= 2 && launch_q >= (nsph > 75 ? 2500000 : 10000000))))
+            var = VARIANT_KSL;
         if (s->ctx->force_variant >= 0) {
             var = s->ctx->force_variant;
         } else {
