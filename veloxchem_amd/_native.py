@@ -93,6 +93,9 @@ def lib():
                                             _c_double_p]
         L.vlx_fock_class_kernel.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                             ctypes.c_int, ctypes.c_int, ctypes.c_char_p, ctypes.c_int]
+        L.vlx_fock_batch_class_kernel.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_void_p),
+                                                  ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                                  ctypes.c_char_p, ctypes.c_int]
         L.vlx_set_precision.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_double]
         L.vlx_set_density_screening.argtypes = [ctypes.c_void_p, ctypes.c_double]
         L.vlx_set_deterministic.argtypes = [ctypes.c_void_p, ctypes.c_int]
@@ -173,6 +176,15 @@ def class_kernel(screener, ithreshold, cls, device=0):
     buf = ctypes.create_string_buffer(128)
     check(lib().vlx_fock_class_kernel(context(device), screener.handle, int(ithreshold), *[int(x) for x in cls],
                                       buf, len(buf)))
+    return buf.value.decode()
+
+
+def batch_class_kernel(screeners, ithreshold, cls, device=0):
+    """Name of the kernel that class cls runs with in one batched build of the screeners."""
+    handles = (ctypes.c_void_p * len(screeners))(*[s.handle.value for s in screeners])
+    buf = ctypes.create_string_buffer(512)
+    check(lib().vlx_fock_batch_class_kernel(context(device), len(screeners), handles, int(ithreshold),
+                                            *[int(x) for x in cls], buf, len(buf)))
     return buf.value.decode()
 
 

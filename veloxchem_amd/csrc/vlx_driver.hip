@@ -417,7 +417,7 @@ struct vlx_screener {
         int cls = -1, idx = -1, swapped = 0;
     };
     std::vector<PairRef> pair_ref;  // nshells x nshells -> position in all[]
-    // by (ithreshold, FP32 bin-sum threshold, forced variant) and the tiled items aimed at
+    // by (ithreshold, FP32 bin-sum threshold, forced variant) and what uses them
     std::map<std::pair<int, int>, std::vector<std::unique_ptr<ClassSchedule>>> schedules;
     bool unscreened_ready = false;  // all_bra, all_tiled and all_tiled_bra are built on first use
     std::map<int, int> variant;  // class entry -> VARIANT_* chosen by vlx_fock_autotune
@@ -853,33 +853,51 @@ int ensure_unscreened(vlx_screener* s)
     return VLX_OK;
 }
 
+// Quartets of one class: exact counts, from the ket side (ket order is sorted by bin).
+struct ClassCounts {
+    long long quartets = 0, prim_quartets = 0;
+    long long ket_prims = 0;  // ket primitives over all quartets
+};
+ClassCounts class_counts(const vlx_screener& s, int entry, int ithr)
+{
+    const auto& ce = g_class_table[entry];
+    const bool unscreened = ithr < 0, same = ce.x == ce.y;
+    const PairSet& bra = unscreened ? s.all_bra[ce.x] : s.kept_bra[ce.x];
+    const PairSet& ket = unscreened ? s.all[ce.y] : s.kept[ce.y];
+    ClassCounts n;
+    for (int j = 0; j < ket.size(); j++) {
+        long long lo = 0, hi;
+        if (unscreened) {
+            hi = bra.size();
+        } else {
+            const int lim = ithr - ket.pairs[j].bin;
+            hi = (lim < 0) ? 0 : bra.cnt_le[std::min(lim, NBINS - 1)];
+        }
+        if (same) lo = j;  // ranks of the same-class bras run over the ket order
+        if (hi <= lo) continue;
+        const PairSet& rk = same ? ket : bra;  // prefix sums in an order where [lo, hi) is contiguous
+        n.quartets += hi - lo;
+        n.ket_prims += (hi - lo) * ket.pairs[j].nprim;
+        n.prim_quartets += (long long)ket.pairs[j].nprim * (rk.nprim_prefix[hi] - rk.nprim_prefix[lo]);
+    }
+    return n;
+}
+
 // Work items of every class at ithreshold.  k32 < NO_FP32 also splits the
 // tiled items: the bras of an item whose bin plus the smallest ket bin of
 // its chunk reaches k32 form an FP32 item (every quartet in it has
 // Schwarz bound < 10^(2 - k32)); the rest stay FP64.
-// create = false: only a schedule built earlier is returned (no host or device allocation);
-// without one the call fails.
+// use: USE_DIRECT gives the matrix-core MD classes the work items of the direct digestion (multi-density
+// and deterministic builds); USE_BATCH leaves items and U arrays on the host, for the batch's own
+// concatenated lists (40 molecules: the uploads were 30 ms of the first pass).
 // share: the builds that run side by side in one launch (a batch's molecules), each aiming at its
-// share of the tiled items.  use: USE_DIRECT gives the matrix-core MD classes the work items of the
-// direct digestion (multi-density and deterministic builds); USE_BATCH leaves items and U arrays on
-// the host, for the batch's own concatenated lists (40 molecules: the uploads were 30 ms of the first
-// pass).
+// share of the tiled items.  launch: each class's quartets over all of them, which choose its kernel
+// (nullptr: this build's own).
 enum ScheduleUse { USE_BUILD = 0, USE_DIRECT = 1, USE_BATCH = 2 };
-int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_ptr<ClassSchedule>>** out,
-                  bool create = true, int share = 1, ScheduleUse use = USE_BUILD)
+int make_schedules(vlx_screener* s, int ithr, int k32, ScheduleUse use, int share,
+                   const std::vector<ClassCounts>* launch, std::vector<std::unique_ptr<ClassSchedule>>& list)
 {
     const int tile_items = std::max(1, s->ctx->tile_items / share);
-    const std::pair<int, int> key{((ithr + 1) * 128 + k32) * (NVARIANTS + 1) + (s->ctx->force_variant + 1),
-                                  4 * tile_items + use};
-    auto it = s->schedules.find(key);
-    if (it != s->schedules.end()) {
-        *out = &it->second;
-        return VLX_OK;
-    }
-    if (!create)
-        return fail(VLX_ERR_ARG, "no work schedule of this screener for ithreshold %d and FP32 bin sum %d: one "
-                                 "allocating build of the screener at these settings must come first", ithr, k32);
-    std::vector<std::unique_ptr<ClassSchedule>> list;
     const int nentries = static_cast<int>(sizeof(g_class_table) / sizeof(g_class_table[0]));
     const bool unscreened = ithr < 0;
     if (unscreened) {
@@ -894,23 +912,9 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         const bool same = ce.x == ce.y;
         auto sch = std::make_unique<ClassSchedule>();
         sch->entry = e;
-        // exact quartet counts, from the ket side (ket order is sorted by bin)
-        long long ket_prims = 0;  // ket primitives over all quartets
-        for (int j = 0; j < ket.size(); j++) {
-            long long lo = 0, hi;
-            if (unscreened) {
-                hi = bra.size();
-            } else {
-                const int lim = ithr - ket.pairs[j].bin;
-                hi = (lim < 0) ? 0 : bra.cnt_le[std::min(lim, NBINS - 1)];
-            }
-            if (same) lo = j;  // ranks of the same-class bras run over the ket order
-            if (hi <= lo) continue;
-            const PairSet& rk = same ? ket : bra;  // prefix sums in an order where [lo, hi) is contiguous
-            sch->quartets += hi - lo;
-            ket_prims += (hi - lo) * ket.pairs[j].nprim;
-            sch->prim_quartets += (long long)ket.pairs[j].nprim * (rk.nprim_prefix[hi] - rk.nprim_prefix[lo]);
-        }
+        const ClassCounts own = class_counts(*s, e, ithr), &all = launch ? (*launch)[e] : own;
+        sch->quartets = own.quartets;
+        sch->prim_quartets = own.prim_quartets;
         const int* gm = s->grp_max;
         const int tile_lds = 8 * (gm[ce.la] * gm[ce.lb] + gm[ce.lc] * gm[ce.ld] + gm[ce.la] * gm[ce.lc] +
                                    gm[ce.la] * gm[ce.ld] + gm[ce.lb] * gm[ce.lc] + gm[ce.lb] * gm[ce.ld]);
@@ -925,7 +929,7 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         // 1.48 (13 waters), 1.5 (ds| def2-SVP 1.31 / 1.09 (32 waters); but 1.7 (ds| def2-SVPD (ds|ds)
         // 0.44 / 0.50, 1.9 (pp| def2-TZVP (ds|pp) 1.54 / 1.69.  (dp|pp), 135 integrals: untiled / tiled
         // single primitives 11.3 / 7.5 ms at 1.45, 3.7 / 4.5 at 1.9
-        const bool few_prims = L >= 4 && ket_prims * 2 < sch->quartets * 3;
+        const bool few_prims = L >= 4 && all.ket_prims * 2 < all.quartets * 3;
         int var = VARIANT_UNTILED;
         if (can_tile && (L <= 4 || nsph <= 75 || (L == 5 && few_prims))) {
             if (s->ctx->tiled_waves == 4) var = few_prims ? VARIANT_TILED4_P1 : VARIANT_TILED4;
@@ -942,8 +946,8 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         // ((dp|pp) of one water, 144 primitive quartets, 0.18 / 0.08 ms; of two waters def2-TZVP, 6000,
         // 0.39 / 0.16; (fp|fs) there 0.82 / 0.15), and lose it at about 2e5
         // (quartets of the whole launch: a batch's molecules share it)
-        const long long launch = sch->prim_quartets * share;
-        if (var == VARIANT_UNTILED && ce.mmd && (nsph >= 225 || launch < 200000 || (nsph >= 175 && launch < 2000000)))
+        if (var == VARIANT_UNTILED && ce.mmd &&
+            (nsph >= 225 || all.prim_quartets < 200000 || (nsph >= 175 && all.prim_quartets < 2000000)))
             var = VARIANT_MMD;
         // Ket-stationary items with LDS accumulators, in large launches: their bra walks are then long, and
         // keep three of the six blocks from the global atomics that the bra-stationary form sends all six
@@ -954,10 +958,9 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
         // 4.8e7 64 / 36; (fs|pp) 4.8e6 3.0 / 3.5, 9.8e6 6.8 / 4.8; (fs|ds) 7.2e6 3.5 / 4.0, 1.5e7 8.3 / 6.3
         // (def2-TZVP); def2-SVPD (dp|ds) 2.6e7 20.7 / 16.6, tiled (dp|pp) 6.1e6 7.5 / 6.6; but (pp|pp)
         // 5.1e7 12 / 28
-        const long long launch_q = sch->quartets * share;
         if (ce.ksl && nsph <= 135 &&
-            ((var == VARIANT_UNTILED && launch_q >= 2500000) ||
-             (variant_tiled(var) && L == 5 && ce.lc + ce.ld >= 2 && launch_q >= (nsph > 75 ? 2500000 : 10000000))))
+            ((var == VARIANT_UNTILED && all.quartets >= 2500000) ||
+             (variant_tiled(var) && L == 5 && ce.lc + ce.ld >= 2 && all.quartets >= (nsph > 75 ? 2500000 : 10000000))))
             var = VARIANT_KSL;
         if (s->ctx->force_variant >= 0) {
             var = s->ctx->force_variant;
@@ -1237,9 +1240,78 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
                 if (sp.get() == c.second) sorted.push_back(std::move(sp));
         list.swap(sorted);
     }
-    auto res = s->schedules.emplace(key, std::move(list));
-    *out = &res.first->second;
     return VLX_OK;
+}
+
+// The screener's schedule at these settings, built on the first call.
+// create = false: only a schedule built earlier is returned (no host or device allocation);
+// without one the call fails.
+int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_ptr<ClassSchedule>>** out,
+                  bool create = true, ScheduleUse use = USE_BUILD)
+{
+    const std::pair<int, int> key{((ithr + 1) * 128 + k32) * (NVARIANTS + 1) + (s->ctx->force_variant + 1), use};
+    auto it = s->schedules.find(key);
+    if (it == s->schedules.end()) {
+        if (!create)
+            return fail(VLX_ERR_ARG, "no work schedule of this screener for ithreshold %d and FP32 bin sum %d: one "
+                                     "allocating build of the screener at these settings must come first", ithr, k32);
+        std::vector<std::unique_ptr<ClassSchedule>> list;
+        const int rc = make_schedules(s, ithr, k32, use, 1, nullptr, list);
+        if (rc) return rc;
+        it = s->schedules.emplace(key, std::move(list)).first;
+    }
+    *out = &it->second;
+    return VLX_OK;
+}
+
+// The schedules of a batch's molecules, each distinct screener's once.  One kernel per class for the
+// whole batch, chosen by its quartets together; nothing of it stays in the screeners, whose other
+// batches may be of other sizes.
+using ScheduleList = std::vector<std::unique_ptr<ClassSchedule>>;
+int make_batch_schedules(const std::vector<vlx_screener*>& scrs, int ithr, std::map<vlx_screener*, ScheduleList>& made)
+{
+    const int nentries = static_cast<int>(sizeof(g_class_table) / sizeof(g_class_table[0]));
+    std::map<vlx_screener*, int> times;
+    for (vlx_screener* s : scrs) times[s]++;
+    std::vector<ClassCounts> launch(nentries);
+    for (const auto& [s, n] : times) {
+        const int rc = ithr < 0 ? ensure_unscreened(s) : VLX_OK;
+        if (rc) return rc;
+        for (int e = 0; e < nentries; e++) {
+            const ClassCounts c = class_counts(*s, e, ithr);
+            launch[e].quartets += n * c.quartets;
+            launch[e].prim_quartets += n * c.prim_quartets;
+            launch[e].ket_prims += n * c.ket_prims;
+        }
+    }
+    for (const auto& [s, n] : times) {
+        const int rc = make_schedules(s, ithr, NO_FP32, USE_BATCH, static_cast<int>(scrs.size()), &launch, made[s]);
+        if (rc) return rc;
+    }
+    return VLX_OK;
+}
+
+// The kernel of a schedule, if it is of class (la lb|lc ld), as profilers print it (single density).
+bool class_kernel_name(const ClassSchedule& sch, int la, int lb, int lc, int ld, char* name, int len)
+{
+    const auto& ce = g_class_table[sch.entry];
+    if (ce.la != la || ce.lb != lb || ce.lc != lc || ce.ld != ld) return false;
+    if (sch.tiled) {
+        const int L = la + lb + lc + ld;
+        const int wide = (L == la && la <= 2) ? 12 : (L <= 2 ? 16 : (L == 3 ? 8 : 4));
+        // template arguments <..., R, NW, RS, MULTI, DLDS>
+        std::snprintf(name, len, "fock_kernel_tiled<%d,%d,%d,%d,double,%d,false,false,%s>", la, lb, lc, ld,
+                      sch.tiled_waves == 4 ? 4 : wide, sch.dlds ? "true" : "false");
+    } else {
+        const char* k = sch.mmd_tiled                       ? "fock_kernel_mmd_tiled"
+                        : sch.mmd                           ? "fock_kernel_mmd"
+                        : sch.ksl                           ? "fock_kernel_ksl"
+                        : (ce.variant == VLX_KET_STATIONARY) ? "fock_kernel"
+                                                            : "fock_kernel_bs";
+        if (sch.ksl) std::snprintf(name, len, "%s<%d,%d,%d,%d,false,4>", k, la, lb, lc, ld);
+        else std::snprintf(name, len, "%s<%d,%d,%d,%d,false>", k, la, lb, lc, ld);
+    }
+    return true;
 }
 
 int check_symmetric_host(const double* d, int n)
@@ -1961,27 +2033,31 @@ int vlx_fock_class_kernel(vlx_context* ctx, vlx_screener* scr, int ithreshold, i
     std::vector<std::unique_ptr<ClassSchedule>>* list = nullptr;
     int rc = get_schedules(scr, ithreshold, NO_FP32, &list);
     if (rc) return rc;
-    for (const auto& sp : *list) {
-        const auto& ce = g_class_table[sp->entry];
-        if (ce.la != la || ce.lb != lb || ce.lc != lc || ce.ld != ld) continue;
-        if (sp->tiled) {
-            const int L = la + lb + lc + ld;
-            const int wide = (L == la && la <= 2) ? 12 : (L <= 2 ? 16 : (L == 3 ? 8 : 4));
-            // template arguments as the profiler prints them: <..., R, NW, RS, MULTI, DLDS>
-            std::snprintf(name, len, "fock_kernel_tiled<%d,%d,%d,%d,double,%d,false,false,%s>", la, lb, lc, ld,
-                          sp->tiled_waves == 4 ? 4 : wide, sp->dlds ? "true" : "false");
-        } else {
-            const char* k = sp->mmd_tiled                       ? "fock_kernel_mmd_tiled"
-                            : sp->mmd                           ? "fock_kernel_mmd"
-                            : sp->ksl                           ? "fock_kernel_ksl"
-                            : (ce.variant == VLX_KET_STATIONARY) ? "fock_kernel"
-                                                                : "fock_kernel_bs";
-            if (sp->ksl) std::snprintf(name, len, "%s<%d,%d,%d,%d,false,4>", k, la, lb, lc, ld);
-            else std::snprintf(name, len, "%s<%d,%d,%d,%d,false>", k, la, lb, lc, ld);
-        }
-        return VLX_OK;
-    }
+    for (const auto& sp : *list)
+        if (class_kernel_name(*sp, la, lb, lc, ld, name, len)) return VLX_OK;
     return fail(VLX_ERR_ARG, "class (%d%d|%d%d) has no work at this threshold", la, lb, lc, ld);
+}
+
+int vlx_fock_batch_class_kernel(vlx_context* ctx, int nmol, vlx_screener* const* scrs, int ithreshold, int la, int lb,
+                                int lc, int ld, char* name, int len)
+{
+    if (!ctx || nmol < 1 || !scrs || !name || len < 1) return fail(VLX_ERR_ARG, "NULL argument");
+    for (int m = 0; m < nmol; m++)
+        if (!scrs[m] || scrs[m]->ctx != ctx) return fail(VLX_ERR_ARG, "screener %d is not of this context", m);
+    HIP_TRY(hipSetDevice(ctx->device));
+    std::map<vlx_screener*, ScheduleList> made;
+    const int rc = make_batch_schedules(std::vector<vlx_screener*>(scrs, scrs + nmol), ithreshold, made);
+    if (rc) return rc;
+    std::string names;
+    for (const auto& kv : made)
+        for (const auto& sp : kv.second) {
+            char one[128];
+            if (!class_kernel_name(*sp, la, lb, lc, ld, one, sizeof(one))) continue;
+            if (names.find(one) == std::string::npos) names += (names.empty() ? "" : " ") + std::string(one);
+        }
+    if (names.empty()) return fail(VLX_ERR_ARG, "class (%d%d|%d%d) has no work at this threshold", la, lb, lc, ld);
+    std::snprintf(name, len, "%s", names.c_str());
+    return VLX_OK;
 }
 
 int vlx_fock_work(vlx_screener* scr, int ithreshold, int max_records, int* nrecords, int* classes,
@@ -2221,7 +2297,7 @@ int multi_pass(vlx_context* ctx, vlx_screener* scr, const double* dens, int m, c
     std::vector<std::unique_ptr<ClassSchedule>>* list = nullptr;
     const int saved_variant = ctx->force_variant;
     if (det) ctx->force_variant = VARIANT_UNTILED;
-    int rc = get_schedules(scr, ithreshold, NO_FP32, &list, true, 1, USE_DIRECT);
+    int rc = get_schedules(scr, ithreshold, NO_FP32, &list, true, USE_DIRECT);
     ctx->force_variant = saved_variant;
     if (rc) return rc;
     const bool single = m == 1 && !det;
@@ -2585,11 +2661,8 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
     const int nmol = static_cast<int>(P.scrs.size());
     const int npc = npair_classes();
     const bool unscreened = P.ithreshold < 0;
-    std::vector<std::vector<std::unique_ptr<ClassSchedule>>*> lists(nmol, nullptr);
-    for (int m = 0; m < nmol; m++) {
-        const int rc = get_schedules(P.scrs[m], P.ithreshold, NO_FP32, &lists[m], true, nmol, USE_BATCH);
-        if (rc) return rc;
-    }
+    std::map<vlx_screener*, ScheduleList> made;
+    if (const int rc = make_batch_schedules(P.scrs, P.ithreshold, made)) return rc;
     // the four orders of every pair class, and each molecule's offsets in them
     enum { KET = 0, BRA = 1, TKET = 2, TBRA = 3, NKIND = 4 };
     auto sets_of = [&](vlx_screener* sc, int kind) -> std::vector<PairSet>& {
@@ -2699,7 +2772,7 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
     // launches: every molecule's class schedules, grouped by (class, variant, lane entries, block)
     std::map<std::array<int, 4>, BatchLaunch*> by_key;
     for (int m = 0; m < nmol; m++) {
-        for (const auto& sp : *lists[m]) {
+        for (const auto& sp : made[P.scrs[m]]) {
             const ClassSchedule& sch = *sp;
             const auto& ce = g_class_table[sch.entry];
             const std::array<int, 4> key{sch.entry, sch.variant, (sch.singles ? 1 : 0) + (sch.mmd_tiled ? 2 : 0), sch.tiled_waves};
