@@ -302,6 +302,9 @@ int vlx_fock_autotune_rejected(vlx_context* ctx, int* mask);
  * runs with at ithreshold, written to name[0..len). */
 int vlx_fock_class_kernel(vlx_context* ctx, vlx_screener* scr, int ithreshold, int la, int lb, int lc, int ld,
                           char* name, int len);
+/* The same for a build of several densities (vlx_fock_compute_multi). */
+int vlx_fock_multi_class_kernel(vlx_context* ctx, vlx_screener* scr, int ithreshold, int la, int lb, int lc, int ld,
+                                char* name, int len);
 /* The same for a batched build of these screeners in FP64 (several names, separated by spaces, where
  * molecules differ in what they can run or were tuned to). */
 int vlx_fock_batch_class_kernel(vlx_context* ctx, int nmol, vlx_screener* const* scrs, int ithreshold, int la, int lb,

@@ -141,6 +141,57 @@ def test_multi_many_densities_match_single_builds():
     assert np.max(np.abs(one.matrix('0').to_numpy() - single)) < 1e-12 * max(1.0, np.max(np.abs(single)))
 
 
+def _against_single_builds(scr, bas, n, nocc):
+    """Two densities in one call against a build each: an element sums up to n^2 products of independent
+    rounding errors in an order of each kernel's own, n eps on either side."""
+    dens = [pseudo_density(n, nocc, seed=s) for s in (1, 2)]
+    drv = FockDriver()
+    out = drv.compute(scr, _matrices(bas, dens, [False] * 2), ['2jk', 'k'], 0.0, 0.0, 12)
+    for i, lab in enumerate(['2jk', 'k']):
+        one = np.asarray(drv.compute(scr, dens[i], lab, 0.0, 0.0, 12))
+        err = np.max(np.abs(out.matrix(str(i)).to_numpy() - one))
+        assert err <= 2 * n * np.finfo(float).eps * max(1.0, np.max(np.abs(one))), (lab, err)
+
+
+@pytest.mark.parametrize('tuned', [False, True])
+def test_middle_launches_of_several_densities_share_integrals(tuned):
+    """From 3e4 primitive quartets on, blocks of fewer than 189 integrals run the generated kernels in
+    builds of several densities (the direct digestion of the matrix-core kernel is up to five times
+    slower there), also where single builds were tuned to the matrix-core kernel."""
+    from veloxchem_amd import _native
+    mol = water_cluster(8, 6.3, 3)
+    bas = MolecularBasis.read(mol, 'def2-tzvp')
+    scr = _screened(mol, bas)
+    work = [(tuple(c), pq) for c, _, pq, _ in scr.work(12)]
+    if tuned:
+        ctx, lib = _native.context(), _native.lib()
+        cls, cp = _native.as_int(np.array([c for c, _ in work]).ravel())
+        var, vp = _native.as_int(np.full(len(work), 3))
+        _native.check(lib.vlx_fock_set_variants(ctx, scr.handle, len(work), cp, vp, None))
+    seen = {'mmd': 0, 'generated': 0}
+    for c, pq in work:
+        block = int(np.prod([2 * x + 1 for x in c]))
+        if sum(c) < 6:
+            continue
+        direct = block >= 245 or pq < (600000 if block >= 189 else 30000)
+        name = _native.class_kernel(scr, 12, c, multi=True)
+        assert ('mmd' in name) == direct, (c, pq, name)
+        seen['mmd' if direct else 'generated'] += 1
+    assert min(seen.values()) >= 3, seen
+    _against_single_builds(scr, bas, bas.get_dimensions_of_basis(), 40)
+
+
+def test_large_launches_of_several_densities():
+    """Launches of 2.5e6 quartets and more: ket-stationary items with LDS accumulators, once per density."""
+    from veloxchem_amd import _native
+    mol = water_cluster(36, 2.7 * 36 ** (1.0 / 3.0), 3)
+    bas = MolecularBasis.read(mol, 'def2-tzvp')
+    scr = _screened(mol, bas)
+    names = [_native.class_kernel(scr, 12, c, multi=True) for c in ((2, 1, 1, 1), (3, 0, 3, 0), (3, 0, 2, 0))]
+    assert any('ksl' in k for k in names), names
+    _against_single_builds(scr, bas, bas.get_dimensions_of_basis(), 180)
+
+
 def test_multi_argument_errors():
     from veloxchem_amd import _native
     mol, bas = dimer('def2-svpd')

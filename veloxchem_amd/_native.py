@@ -93,6 +93,7 @@ def lib():
                                             _c_double_p]
         L.vlx_fock_class_kernel.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                             ctypes.c_int, ctypes.c_int, ctypes.c_char_p, ctypes.c_int]
+        L.vlx_fock_multi_class_kernel.argtypes = L.vlx_fock_class_kernel.argtypes
         L.vlx_fock_batch_class_kernel.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_void_p),
                                                   ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                                   ctypes.c_char_p, ctypes.c_int]
@@ -171,11 +172,12 @@ def last_fp32_bin_sum(device=0):
     return k.value
 
 
-def class_kernel(screener, ithreshold, cls, device=0):
-    """Name of the kernel that class cls = (la, lb, lc, ld) runs with, as profilers report it."""
+def class_kernel(screener, ithreshold, cls, device=0, multi=False):
+    """Name of the kernel that class cls = (la, lb, lc, ld) runs with, as profilers report it; ``multi``:
+    in a build of several densities."""
     buf = ctypes.create_string_buffer(128)
-    check(lib().vlx_fock_class_kernel(context(device), screener.handle, int(ithreshold), *[int(x) for x in cls],
-                                      buf, len(buf)))
+    name = lib().vlx_fock_multi_class_kernel if multi else lib().vlx_fock_class_kernel
+    check(name(context(device), screener.handle, int(ithreshold), *[int(x) for x in cls], buf, len(buf)))
     return buf.value.decode()
 
 

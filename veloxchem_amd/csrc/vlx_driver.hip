@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <array>
 #include <cctype>
+#include <climits>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -945,10 +946,18 @@ int make_schedules(vlx_screener* s, int ithr, int k32, ScheduleUse use, int shar
         // has too few quartets for a lane each: the generated kernels then take the time of one lane
         // ((dp|pp) of one water, 144 primitive quartets, 0.18 / 0.08 ms; of two waters def2-TZVP, 6000,
         // 0.39 / 0.16; (fp|fs) there 0.82 / 0.15), and lose it at about 2e5
-        // (quartets of the whole launch: a batch's molecules share it)
-        if (var == VARIANT_UNTILED && ce.mmd &&
-            (nsph >= 225 || all.prim_quartets < 200000 || (nsph >= 175 && all.prim_quartets < 2000000)))
-            var = VARIANT_MMD;
+        // (quartets of the whole launch: a batch's molecules share it).
+        // Several densities: the matrix-core kernel digests directly, all six blocks of every density by
+        // global atomics, and loses the LDS tiles that the lines above rest on, while the generated kernels
+        // share a quartet's integrals and its loads of pairs.  One stream, generated / matrix-core, four
+        // densities: 49 to 175 integrals (fs|dp) at 3.8e3 primitive quartets 0.32 / 0.09 ms, (fs|dd) 2.7e4
+        // 0.87 / 0.70, but (fd|ds) 4.6e4 0.91 / 1.26, (ff|ss) 9.1e4 0.28 / 1.34, (fs|dd) 2.5e5 3.0 / 4.5;
+        // (fp|pp), 189, 2.1e5 2.6 / 1.9, 2.0e6 9.8 / 15; (dd|pp), 225, 5.5e5 5.9 / 5.5, 1.1e6 13.6 / 17.4;
+        // (dp|dp), 225, 8.7e5 9.0 / 9.4; (fd|fs), 245, 8.0e5 22.8 / 20.8, 2.9e6 67 / 68; (fp|dp), 315, 3.5e6
+        // 68 / 52 (2 to 64 waters def2-TZVP, 13 waters def2-SVPD)
+        const long long generated_from = use == USE_DIRECT ? (nsph >= 245 ? LLONG_MAX : nsph >= 189 ? 600000 : 30000)
+                                                           : (nsph >= 225 ? LLONG_MAX : nsph >= 175 ? 2000000 : 200000);
+        if (var == VARIANT_UNTILED && ce.mmd && all.prim_quartets < generated_from) var = VARIANT_MMD;
         // Ket-stationary items with LDS accumulators, in large launches: their bra walks are then long, and
         // keep three of the six blocks from the global atomics that the bra-stationary form sends all six
         // to; the tiled form's chunks, of one group pair each, hold fewer kets the larger the system.  One
@@ -957,7 +966,12 @@ int make_schedules(vlx_screener* s, int ithr, int k32, ScheduleUse use, int shar
         // 15.0; but (fp|pp) 1.4e7 44 / 51, (fp|fs) 39 / 48.  Tiled (dp|ds) 6.0e6 4.8 / 5.7, 1.2e7 11.6 / 10.4,
         // 4.8e7 64 / 36; (fs|pp) 4.8e6 3.0 / 3.5, 9.8e6 6.8 / 4.8; (fs|ds) 7.2e6 3.5 / 4.0, 1.5e7 8.3 / 6.3
         // (def2-TZVP); def2-SVPD (dp|ds) 2.6e7 20.7 / 16.6, tiled (dp|pp) 6.1e6 7.5 / 6.6; but (pp|pp)
-        // 5.1e7 12 / 28
+        // 5.1e7 12 / 28.  Several densities: these items run once per density, and still take less than the
+        // forms that share the integrals, whose atomics grow with the densities too: four densities, 36
+        // waters (dp|pp) 57 / 38, (fp|ds) 46 / 32, (fs|fs) 36 / 18, (fd|ps) 27.7 / 25.6; 64 waters (fp|ds)
+        // 164 / 106, but (dd|ds) 59 / 63, (ff|ss) 29 / 32 of 4953.  Mixed precision: the FP32 form of a tiled
+        // class / these items in FP64, 36 waters (dp|ds) 13.7 / 10.8, (fs|pp) 8.6 / 4.8, (fs|ds) 8.4 / 6.3, 24
+        // waters def2-SVPD (dp|ds) 17.2 / 13.4
         if (ce.ksl && nsph <= 135 &&
             ((var == VARIANT_UNTILED && all.quartets >= 2500000) ||
              (variant_tiled(var) && L == 5 && ce.lc + ce.ld >= 2 && all.quartets >= (nsph > 75 ? 2500000 : 10000000))))
@@ -967,8 +981,11 @@ int make_schedules(vlx_screener* s, int ithr, int k32, ScheduleUse use, int shar
         } else {
             const auto vit = s->variant.find(e);
             const auto cit = s->ctx->tuned_variant.find(e);
-            if (vit != s->variant.end()) var = vit->second;
-            else if (cit != s->ctx->tuned_variant.end()) var = cit->second;
+            int tuned = -1;
+            if (vit != s->variant.end()) tuned = vit->second;
+            else if (cit != s->ctx->tuned_variant.end()) tuned = cit->second;
+            // a matrix-core choice was timed with LDS tiles, which the direct digestion has not
+            if (tuned >= 0 && !(tuned == VARIANT_MMD && use == USE_DIRECT)) var = tuned;
         }
         if (variant_tiled(var) && !can_tile) var = VARIANT_UNTILED;
         if (var == VARIANT_MMD && !ce.mmd) var = VARIANT_UNTILED;
@@ -1291,21 +1308,38 @@ int make_batch_schedules(const std::vector<vlx_screener*>& scrs, int ithr, std::
     return VLX_OK;
 }
 
-// The kernel of a schedule, if it is of class (la lb|lc ld), as profilers print it (single density).
-bool class_kernel_name(const ClassSchedule& sch, int la, int lb, int lc, int ld, char* name, int len)
+// Kernels whose single-density form keeps accumulators the multi-density form cannot
+// hold run once per density instead (the integrals are recomputed): ks-lds (one density
+// of LDS slots), the ket-stationary register accumulators (the multi-density direct
+// digestion measured 4.8x slower than four launches) and the tiled classes above L = 2
+// or over single primitives (k tile sets cut the occupancy: 1.1-1.9x slower).  MD,
+// bra-stationary and L <= 2 tiled classes share the integrals (0.5-0.95x of k launches,
+// def2-SVP and def2-TZVP water clusters).
+bool runs_per_density(const ClassSchedule& sch)
+{
+    const auto& ce = g_class_table[sch.entry];
+    return sch.ksl || (!sch.tiled && !sch.mmd && ce.variant == VLX_KET_STATIONARY) ||
+           (sch.tiled && (sch.singles || ce.la + ce.lb + ce.lc + ce.ld > 2));
+}
+
+// The kernel of a schedule, if it is of class (la lb|lc ld), as profilers print it; multi: in a build of
+// several densities.
+bool class_kernel_name(const ClassSchedule& sch, int la, int lb, int lc, int ld, char* name, int len, bool multi = false)
 {
     const auto& ce = g_class_table[sch.entry];
     if (ce.la != la || ce.lb != lb || ce.lc != lc || ce.ld != ld) return false;
+    multi = multi && !runs_per_density(sch);
     if (sch.tiled) {
         const int L = la + lb + lc + ld;
         const int wide = (L == la && la <= 2) ? 12 : (L <= 2 ? 16 : (L == 3 ? 8 : 4));
         // template arguments <..., R, NW, RS, MULTI, DLDS>
-        std::snprintf(name, len, "fock_kernel_tiled<%d,%d,%d,%d,double,%d,false,false,%s>", la, lb, lc, ld,
-                      sch.tiled_waves == 4 ? 4 : wide, sch.dlds ? "true" : "false");
+        std::snprintf(name, len, "fock_kernel_tiled<%d,%d,%d,%d,double,%d,false,%s,%s>", la, lb, lc, ld,
+                      sch.tiled_waves == 4 ? 4 : wide, multi ? "true" : "false", sch.dlds && !multi ? "true" : "false");
     } else {
         const char* k = sch.mmd_tiled                       ? "fock_kernel_mmd_tiled"
                         : sch.mmd                           ? "fock_kernel_mmd"
                         : sch.ksl                           ? "fock_kernel_ksl"
+                        : multi                             ? "fock_kernel_multi"
                         : (ce.variant == VLX_KET_STATIONARY) ? "fock_kernel"
                                                             : "fock_kernel_bs";
         if (sch.ksl) std::snprintf(name, len, "%s<%d,%d,%d,%d,false,4>", k, la, lb, lc, ld);
@@ -2038,6 +2072,18 @@ int vlx_fock_class_kernel(vlx_context* ctx, vlx_screener* scr, int ithreshold, i
     return fail(VLX_ERR_ARG, "class (%d%d|%d%d) has no work at this threshold", la, lb, lc, ld);
 }
 
+int vlx_fock_multi_class_kernel(vlx_context* ctx, vlx_screener* scr, int ithreshold, int la, int lb, int lc, int ld,
+                                char* name, int len)
+{
+    if (!ctx || !scr || !name || len < 1) return fail(VLX_ERR_ARG, "NULL argument");
+    std::vector<std::unique_ptr<ClassSchedule>>* list = nullptr;
+    int rc = get_schedules(scr, ithreshold, NO_FP32, &list, true, USE_DIRECT);
+    if (rc) return rc;
+    for (const auto& sp : *list)
+        if (class_kernel_name(*sp, la, lb, lc, ld, name, len, true)) return VLX_OK;
+    return fail(VLX_ERR_ARG, "class (%d%d|%d%d) has no work at this threshold", la, lb, lc, ld);
+}
+
 int vlx_fock_batch_class_kernel(vlx_context* ctx, int nmol, vlx_screener* const* scrs, int ithreshold, int la, int lb,
                                 int lc, int ld, char* name, int len)
 {
@@ -2181,17 +2227,7 @@ int enqueue_classes(vlx_context* ctx, vlx_screener* scr, const std::vector<std::
         if (multi) {
             if (sch.mmd_tiled) return fail(VLX_ERR_ARG, "multi-density builds digest directly");
             if (det && sch.tiled) return fail(VLX_ERR_ARG, "deterministic builds run the untiled kernels only");
-            // Kernels whose single-density form keeps accumulators the multi-density form cannot
-            // hold run once per density instead (the integrals are recomputed): ks-lds (one density
-            // of LDS slots), the ket-stationary register accumulators (the multi-density direct
-            // digestion measured 4.8x slower than four launches) and the tiled classes above L = 2
-            // or over single primitives (k tile sets cut the occupancy: 1.1-1.9x slower).  MD,
-            // bra-stationary and L <= 2 tiled classes share the integrals (0.5-0.95x of k launches,
-            // def2-SVP and def2-TZVP water clusters).
-            const int L = ce.la + ce.lb + ce.lc + ce.ld;
-            const bool per_density =
-                !det && (sch.ksl || (!sch.tiled && !sch.mmd && ce.variant == VLX_KET_STATIONARY) ||
-                         (sch.tiled && (sch.singles || L > 2)));
+            const bool per_density = !det && runs_per_density(sch);
             if (per_density) {
                 const int waves = static_cast<int>(untiled_waves(a.sc.nitems, ctx->untiled_wave_cap));
                 for (int c = 0; c < ndens; c++) {
