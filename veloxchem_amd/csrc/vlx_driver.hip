@@ -957,7 +957,12 @@ int make_schedules(vlx_screener* s, int ithr, int k32, ScheduleUse use, int shar
         // 68 / 52 (2 to 64 waters def2-TZVP, 13 waters def2-SVPD)
         const long long generated_from = use == USE_DIRECT ? (nsph >= 245 ? LLONG_MAX : nsph >= 189 ? 600000 : 30000)
                                                            : (nsph >= 225 ? LLONG_MAX : nsph >= 175 ? 2000000 : 200000);
-        if (var == VARIANT_UNTILED && ce.mmd && all.prim_quartets < generated_from) var = VARIANT_MMD;
+        // A molecule of a large batch stays with the matrix-core kernel below a hundredth of the line: it
+        // fills few of the 64 lanes of the generated kernels' items, however large the launch ((dp|pp) of one
+        // to three waters; 40 uneven def2-SVP clusters 8.45 / 8.2 ms; a fortieth: 20 uneven def2-TZVP clusters
+        // 31.8 / 32.7)
+        const bool small = use == USE_BATCH && own.prim_quartets < generated_from / 100;
+        if (var == VARIANT_UNTILED && ce.mmd && (all.prim_quartets < generated_from || small)) var = VARIANT_MMD;
         // Ket-stationary items with LDS accumulators, in large launches: their bra walks are then long, and
         // keep three of the six blocks from the global atomics that the bra-stationary form sends all six
         // to; the tiled form's chunks, of one group pair each, hold fewer kets the larger the system.  One
@@ -1281,9 +1286,9 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
     return VLX_OK;
 }
 
-// The schedules of a batch's molecules, each distinct screener's once.  One kernel per class for the
-// whole batch, chosen by its quartets together; nothing of it stays in the screeners, whose other
-// batches may be of other sizes.
+// The schedules of a batch's molecules, each distinct screener's once.  The kernel of a class goes by
+// the whole batch's quartets (small molecules aside: see make_schedules); nothing of it stays in the
+// screeners, whose other batches may be of other sizes.
 using ScheduleList = std::vector<std::unique_ptr<ClassSchedule>>;
 int make_batch_schedules(const std::vector<vlx_screener*>& scrs, int ithr, std::map<vlx_screener*, ScheduleList>& made)
 {
