@@ -148,7 +148,10 @@ int vlx_fock_compute_device(vlx_context* ctx, vlx_screener* scr, const double* d
  * (VLX_ERR_ARG otherwise).  The work schedule of (screener, ithreshold,
  * precision split) must exist: one vlx_fock_compute_device call with the
  * same screener and settings (and, in mixed mode, a density of the same
- * max|D| decade) comes first, else VLX_ERR_ARG.  Per-class timing is not
+ * max|D| decade) or, in FP64, one build of several densities comes first,
+ * else VLX_ERR_ARG (a batched build leaves no schedule of its molecules).
+ * A Coulomb build (labels j, j_rs) runs the class kernels here, not the
+ * Hermite densities of vlx_fock_compute_device.  Per-class timing is not
  * recorded.  Every call on one device shares the array: calls that overlap
  * on one device (two contexts, or two host threads) race and must be
  * serialised by the caller.  Same arguments, results and stream behaviour

@@ -62,6 +62,26 @@ def test_noalloc_mixed_precision_matches():
     assert float(np.max(np.abs(ga - gb))) < 1e-10
 
 
+def test_noalloc_after_a_build_of_several_densities():
+    """The schedule of a build of several densities serves the no-allocation build too."""
+    lib, ctx = _native.lib(), _native.context(0)
+    scr, D, n = _case(2, 4.0, 57, 'def2-tzvp')
+    d_dm, d_two, d_g = _native.DeviceArray((2, n, n)), _native.DeviceArray((2, n, n)), _native.DeviceArray((n, n))
+    try:
+        d_dm.upload(np.stack([D, 2.0 * D]))
+        labels = (ctypes.c_char_p * 2)(b'2jk', b'k')
+        _native.check(lib.vlx_fock_compute_multi_device(ctx, scr.handle, 2, d_dm.ptr, None, labels, 0.0, 0.0, 12,
+                                                        d_two.ptr))
+        _native.check(lib.vlx_fock_compute_device_noalloc(ctx, scr.handle, d_dm.ptr, b'2jk', 0.0, 0.0, 12, d_g.ptr))
+        _native.check(lib.vlx_context_synchronize(ctx))
+        two, g = d_two.download(), d_g.download()
+    finally:
+        for a in (d_dm, d_two, d_g):
+            a.free()
+    # sums of up to n^2 products in orders of their own: n eps on either side
+    assert np.max(np.abs(g - two[0])) <= 2 * n * np.finfo(float).eps * np.max(np.abs(two[0]))
+
+
 def test_noalloc_refuses_unprepared_schedule_and_large_basis():
     lib, ctx = _native.lib(), _native.context(0)
     scr, D, n = _case(1, 3.0, 51)

@@ -1273,6 +1273,8 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
 {
     const std::pair<int, int> key{((ithr + 1) * 128 + k32) * (NVARIANTS + 1) + (s->ctx->force_variant + 1), use};
     auto it = s->schedules.find(key);
+    // a build of several densities leaves the direct digestion's schedule, complete on the device
+    if (it == s->schedules.end() && !create && use == USE_BUILD) it = s->schedules.find({key.first, USE_DIRECT});
     if (it == s->schedules.end()) {
         if (!create)
             return fail(VLX_ERR_ARG, "no work schedule of this screener for ithreshold %d and FP32 bin sum %d: one "
