@@ -657,6 +657,13 @@ void build_tiled(const vlx_screener& s, const PairSet& src, PairSet& ket, PairSe
     // runs of up to ket_prims primitives (they share a pair's contracted work: HRR,
     // digestion), and single primitives (chunks of pairs with mixed primitive counts, such
     // as the 1-, 3- and 5-primitive d-s pairs of def2 bases, then fill every lane)
+    // only for the pair classes that are kets of a tiled class
+    const auto& table = g_class_table;
+    if (std::none_of(std::begin(table), std::end(table), [&](const auto& ce) {
+            return ce.tiled && ce.lc == ket.la && ce.ld == ket.lb &&
+                   ce.la + ce.lb + ce.lc + ce.ld <= s.ctx->tiled_lmax;
+        }))
+        return;
     make_entries(s.ctx->ket_prims, ket.runs);
     make_entries(1, ket.singles);
 }
