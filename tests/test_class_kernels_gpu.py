@@ -1,8 +1,10 @@
 """Tiled kernels, both digestions of the matrix-core kernel and the default choice between them,
-against the untiled kernels, at the edges of their work items."""
+against the untiled kernels, at the edges of their work items.  The 13 largest classes have no other
+kernel than the matrix-core one: its two digestions are checked against the oracle."""
 import numpy as np
 import pytest
 
+from oracle import oracle as orc
 from veloxchem_amd import FockDriver, Matrices, MolecularBasis, T4CScreener, _native, make_matrix, mat_t
 from veloxchem_amd.workloads import pseudo_density, water_cluster
 
@@ -46,6 +48,41 @@ def test_class_kernels_agree(waters, basis, label, omega, ithreshold):
     for v, g in mats.items():
         assert np.isfinite(g).all(), v
         assert np.max(np.abs(g - mats[0])) <= tol, (v, np.max(np.abs(g - mats[0])), tol)
+
+
+@pytest.mark.parametrize('digestion', ['tiles', 'direct'])
+@pytest.mark.parametrize('label, omega', [('2jk', 0.0), ('k', 0.4)])
+def test_matrix_core_kernel_against_oracle(digestion, label, omega):
+    """Every class from la + lb + lc + ld = 4 on, three waters def2-TZVP: 8 + 1 atoms in two groups, so
+    that the tiles' items are ragged; direct: as a build of two densities."""
+    mol = water_cluster(3, 6.0, 3)
+    bas = MolecularBasis.read(mol, 'def2-tzvp')
+    scr = T4CScreener()
+    scr.partition(bas, mol, 'eri')
+    n = bas.get_dimensions_of_basis()
+    D = pseudo_density(n, 15, seed=9)
+    drv, ctx, lib = FockDriver(), _native.context(), _native.lib()
+    name = label + '_rs' if omega else label
+    try:
+        _native.check(lib.vlx_context_set_variant(ctx, 3))
+        if digestion == 'tiles':
+            g = np.asarray(drv.compute(scr, D, name, 0.0, omega, 12))
+        else:
+            ms = Matrices()
+            for i in range(2):
+                m = make_matrix(bas, mat_t.symmetric)
+                m.set_values((i + 1) * D)
+                ms.add(m, str(i))
+            out = drv.compute(scr, ms, [name] * 2, 0.0, omega, 12)
+            g = out.matrix('0').to_numpy()
+            assert np.max(np.abs(out.matrix('1').to_numpy() - 2 * g)) <= 2 * n * EPS * np.max(np.abs(2 * g))
+    finally:
+        _native.check(lib.vlx_context_set_variant(ctx, -1))
+    ob = orc.basis_from(bas, mol)
+    ref = orc.fock_erf(ob, D, label, 0.0, omega, 12)[0] if omega else orc.fock(ob, D, label, 0.0, 12)[0]
+    # n^2 products in orders of their own (n eps on either side), each integral off by some 32 eps
+    err = np.max(np.abs(g - ref))
+    assert err <= (2 * n + 32) * EPS * max(1.0, np.max(np.abs(ref))), err
 
 
 def test_direct_digestion_of_matrix_core_classes():
