@@ -46,6 +46,32 @@ def log(msg):
     print(f'bench: {msg}', file=sys.stderr, flush=True)
 
 
+# per-class tables: on stderr, since the JSON line has to stay short enough to be read whole
+CLASS_TABLES = ('class_ms', 'class_tflops', 'class_ms_one_stream', 'class_tflops_one_stream', 'class_flops', 'autotune')
+
+
+def split_class_tables(result):
+    """(result without its per-class tables, the tables), nested dictionaries included."""
+    line, tables = {}, {}
+    for k, v in result.items():
+        if k in CLASS_TABLES or k.startswith('classes_one_stream'):
+            tables[k] = v
+        elif isinstance(v, dict):
+            line[k], inner = split_class_tables(v)
+            if inner:
+                tables[k] = inner
+        else:
+            line[k] = v
+    return line, tables
+
+
+def report(result):
+    """The JSON line on stdout, the per-class tables on stderr."""
+    line, tables = split_class_tables(result)
+    log('per-class tables ' + json.dumps(tables, default=_plain))
+    print(json.dumps(line, default=_plain))
+
+
 def kernel_traffic(workload, name):
     try:
         with open(TRAFFIC_FILES[workload]) as fh:
@@ -612,7 +638,7 @@ def main():
         svp, _ = workload_builds(32, 10.0, 32, 'def2-svp', args.ithreshold, args.steps, args.warmup, [],
                                  0 if args.no_autotune else 2, 'water32_svp', args.save_tune, args.load_tune,
                                  not args.no_single_stream)
-        print(json.dumps({'svp32': svp}, default=_plain))
+        report({'svp32': svp})
         return
     head, (mol, bas, scr, dm, g) = workload_builds(64, 12.8, 64, 'def2-tzvp', args.ithreshold, args.steps,
                                                    args.warmup, taus, atr, 'water64_tzvp', args.save_tune,
@@ -686,7 +712,7 @@ def main():
             log('reference CPU build of the headline workload')
             result['cpu_baseline'] = cpu_baseline(mol, bas, dm, args.ithreshold, args.cpu_seconds, 'def2-tzvp', g,
                                                   repeats=args.cpu_repeats)
-    print(json.dumps(result, default=_plain))
+    report(result)
 
 
 def _plain(o):

@@ -128,3 +128,27 @@ def test_default_kernels_of_large_launches():
         _native.check(lib.vlx_context_set_variant(ctx, -1))
     assert any('ksl' in k for k in names.values()), names
     assert np.max(np.abs(g - ref)) <= 2 * n * EPS * max(1.0, np.max(np.abs(ref)))
+
+
+@pytest.mark.parametrize('mode', ['mixed', 'screened'])
+def test_fast_modes_of_large_launches(mode):
+    """The same launches in mixed precision (FP32 quartets add 1e-3 tau at most, as in the small
+    molecules' test) and with density-weighted screening (1e4 tau)."""
+    mol = water_cluster(36, 2.7 * 36 ** (1.0 / 3.0), 3)
+    bas = MolecularBasis.read(mol, 'def2-tzvp')
+    scr = T4CScreener()
+    scr.partition(bas, mol, 'eri')
+    D = pseudo_density(bas.get_dimensions_of_basis(), 180, seed=9)
+    drv = FockDriver()
+    ref = np.asarray(drv.compute(scr, D, '2jk', 0.0, 0.0, 12))
+    try:
+        if mode == 'mixed':
+            _native.set_precision('mixed', 1e-6)
+        else:
+            _native.set_density_screening(1e-10)
+        g = np.asarray(drv.compute(scr, D, '2jk', 0.0, 0.0, 12))
+    finally:
+        _native.set_precision('fp64')
+        _native.set_density_screening(0.0)
+    assert np.isfinite(g).all()
+    assert np.max(np.abs(g - ref)) <= (1e-9 if mode == 'mixed' else 1e-6)
