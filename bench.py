@@ -46,18 +46,21 @@ def log(msg):
     print(f'bench: {msg}', file=sys.stderr, flush=True)
 
 
-# per-class tables: on stderr, since the JSON line has to stay short enough to be read whole
-CLASS_TABLES = ('class_ms', 'class_tflops', 'class_ms_one_stream', 'class_tflops_one_stream', 'class_flops', 'autotune')
+# tables per class, molecule or SCF stage: on stderr, since the JSON line has to stay short enough to be
+# read whole
+TABLES = ('class_ms', 'class_tflops', 'class_ms_one_stream', 'class_tflops_one_stream', 'class_flops', 'autotune',
+          'clusters', 'one_electron_s', 'linear_algebra_s', 'screener_s', 'guess_s', 'conv_thresh', 'precision',
+          'incremental_fock', 'fock_builds')
 
 
-def split_class_tables(result):
-    """(result without its per-class tables, the tables), nested dictionaries included."""
+def split_tables(result):
+    """(result without its tables, the tables), nested dictionaries included."""
     line, tables = {}, {}
     for k, v in result.items():
-        if k in CLASS_TABLES or k.startswith('classes_one_stream'):
+        if k in TABLES or k.startswith('classes_one_stream'):
             tables[k] = v
         elif isinstance(v, dict):
-            line[k], inner = split_class_tables(v)
+            line[k], inner = split_tables(v)
             if inner:
                 tables[k] = inner
         else:
@@ -65,10 +68,20 @@ def split_class_tables(result):
     return line, tables
 
 
+def rounded(o):
+    """Floats of nested values to 6 significant digits (energies keep theirs)."""
+    if isinstance(o, dict):
+        return {k: v if k == 'energy' else rounded(v) for k, v in o.items()}
+    if isinstance(o, (list, tuple)):
+        return [rounded(v) for v in o]
+    return float(f'{o:.6g}') if isinstance(o, (float, np.floating)) else o
+
+
 def report(result):
-    """The JSON line on stdout, the per-class tables on stderr."""
-    line, tables = split_class_tables(result)
-    log('per-class tables ' + json.dumps(tables, default=_plain))
+    """The JSON line on stdout (its own values in full, nested ones rounded), the tables on stderr."""
+    line, tables = split_tables(result)
+    log('tables ' + json.dumps(tables, default=_plain))
+    line = {k: rounded(v) if isinstance(v, (dict, list)) else v for k, v in line.items()}
     print(json.dumps(line, default=_plain))
 
 
