@@ -192,6 +192,7 @@ struct ClassSchedule {
 };
 
 struct vlx_screener;
+using ScheduleList = std::vector<std::unique_ptr<ClassSchedule>>;
 
 // One launch of a batched build: the work items of one (class, kernel variant) of every
 // molecule of the batch, their indices moved into the batch's concatenated pair lists.
@@ -216,6 +217,8 @@ struct BatchLaunch {
 // later calls with the same screeners and settings.
 struct BatchPlan {
     std::vector<vlx_screener*> scrs;
+    // the molecules' schedules, shared by the plans of the same molecules
+    std::shared_ptr<const std::map<vlx_screener*, ScheduleList>> schedules;
     std::vector<int> epochs;                 // the screeners' variant epochs the plan was built at
     int ithreshold = 0, force_variant = -1, nstreams = 0;
     double fj = 0.0, fk = 0.0, omega2 = 0.0; // label factors (kernel arguments of the graph)
@@ -1298,7 +1301,6 @@ int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_pt
 // The schedules of a batch's molecules, each distinct screener's once.  The kernel of a class goes by
 // the whole batch's quartets (small molecules aside: see make_schedules); nothing of it stays in the
 // screeners, whose other batches may be of other sizes.
-using ScheduleList = std::vector<std::unique_ptr<ClassSchedule>>;
 int make_batch_schedules(const std::vector<vlx_screener*>& scrs, int ithr, std::map<vlx_screener*, ScheduleList>& made)
 {
     const int nentries = static_cast<int>(sizeof(g_class_table) / sizeof(g_class_table[0]));
@@ -2711,8 +2713,16 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
     const int nmol = static_cast<int>(P.scrs.size());
     const int npc = npair_classes();
     const bool unscreened = P.ithreshold < 0;
-    std::map<vlx_screener*, ScheduleList> made;
-    if (const int rc = make_batch_schedules(P.scrs, P.ithreshold, made)) return rc;
+    // another plan of these molecules, for another label or precision, has the same schedules
+    // (a second plan of 8 16-water def2-TZVP clusters: 631 ms without, 526 with)
+    for (const auto& q : ctx->plans)
+        if (q->scrs == P.scrs && q->epochs == P.epochs && q->ithreshold == P.ithreshold && q->force_variant == P.force_variant)
+            P.schedules = q->schedules;
+    if (!P.schedules) {
+        auto made = std::make_shared<std::map<vlx_screener*, ScheduleList>>();
+        if (const int rc = make_batch_schedules(P.scrs, P.ithreshold, *made)) return rc;
+        P.schedules = made;
+    }
     // the four orders of every pair class, and each molecule's offsets in them
     enum { KET = 0, BRA = 1, TKET = 2, TBRA = 3, NKIND = 4 };
     auto sets_of = [&](vlx_screener* sc, int kind) -> std::vector<PairSet>& {
@@ -2822,7 +2832,7 @@ int build_batch_plan(vlx_context* ctx, BatchPlan& P)
     // launches: every molecule's class schedules, grouped by (class, variant, lane entries, block)
     std::map<std::array<int, 4>, BatchLaunch*> by_key;
     for (int m = 0; m < nmol; m++) {
-        for (const auto& sp : made[P.scrs[m]]) {
+        for (const auto& sp : P.schedules->at(P.scrs[m])) {
             const ClassSchedule& sch = *sp;
             const auto& ce = g_class_table[sch.entry];
             const std::array<int, 4> key{sch.entry, sch.variant, (sch.singles ? 1 : 0) + (sch.mmd_tiled ? 2 : 0), sch.tiled_waves};
