@@ -52,8 +52,11 @@ int vlx_set_block_size_factor(vlx_context* ctx, int factor);
  * quartet in FP32 when its Schwarz bound times max|D| of the build is below
  * `threshold` (decided per tile of kets at the screener's decimal bins:
  * bin_ab + bin_cd >= ceil(2 + log10(max|D| / threshold))), for the classes
- * with the LDS-tiled kernel (la+lb+lc+ld <= 4); J/K accumulation stays FP64.
- * Range-separated labels (*_rs) always run in FP64.
+ * that run the LDS-tiled kernel (la+lb+lc+ld <= 5, see vlx_fock_class_kernel);
+ * the others, and J/K accumulation, stay FP64.
+ * Range-separated labels (*_rs) always run in FP64.  A mixed Coulomb build
+ * (label j) runs the class kernels, which takes longer than its FP64 build:
+ * that one needs no integral blocks.
  */
 enum { VLX_PRECISION_FP64 = 0, VLX_PRECISION_MIXED = 1 };
 int vlx_set_precision(vlx_context* ctx, int mode, double threshold);
@@ -314,7 +317,9 @@ int vlx_fock_batch_class_kernel(vlx_context* ctx, int nmol, vlx_screener* const*
                                 int lc, int ld, char* name, int len);
 
 /* Per-class kernel timing with HIP events on the context's stream
- * (off by default).  vlx_context_class_times synchronises the stream and
+ * (off by default).  While it is on, a Coulomb build (labels j, j_rs) runs the
+ * class kernels, so that every class has a time; without it that build goes
+ * through Hermite densities and takes a fraction of their sum.  vlx_context_class_times synchronises the stream and
  * returns, per class (la, lb, lc, ld), the summed kernel time in ms and the
  * number of launches since the last reset. */
 int vlx_context_set_timing(vlx_context* ctx, int enable);

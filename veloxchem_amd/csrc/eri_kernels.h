@@ -959,7 +959,8 @@ __global__ void __launch_bounds__(NW * VLX_WAVE) __attribute__((amdgpu_waves_per
             stage(d_bd, rb, nB, rd, nD);
             __syncthreads();
         }
-        // wavefronts per chunk: as few as leave each some eight bras, but no group without a chunk
+        // wavefronts per chunk: halved while they have fewer than eight bras each and the groups of
+        // wavefronts are fewer than the chunks (the last halving can leave groups without a chunk)
         const int nch = (ti.j1 - ti.j0) / VLX_WAVE;
         int S = NW;
         while (S > 1 && NW / S < nch && ti.i1 - ti.i0 < 8 * S) S >>= 1;

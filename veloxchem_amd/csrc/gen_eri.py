@@ -316,7 +316,7 @@ def ksl_waves(la, lb, lc, ld, var):
 
 
 # lane-private accumulator slots of fock_kernel_ksl with 4-wave blocks: 64 x 256 threads x 8 B =
-# 128 KiB, plus the 25.5 KB Boys table, within the 160 KB of LDS
+# 128 KiB, plus the 20.3 KB Boys table, within the 160 KB of LDS
 KSL_MAX_SLOTS = 64
 
 

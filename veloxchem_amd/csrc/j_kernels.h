@@ -4,7 +4,7 @@
 //   H_q = (-1)^q sum_cd U_cd[q] D_cd
 //
 // with U the Hermite-to-spherical matrix of a primitive pair.  H is made once per primitive of every
-// pair (j_prep.hip) and U_ab is applied once at the end, so a primitive quartet costs its Boys function,
+// pair (j_engine.hip) and U_ab is applied once at the end, so a primitive quartet costs its Boys function,
 // the recursion to R^0 and one product per (p, q): no horizontal recursion, no integrals, no digestion.
 // The class kernels spend 70-90% of a Coulomb build on those.  Every primitive of one Hermite rank
 // (la + lb) is in one list, whatever its pair class, sorted by the pair's Schwarz bin, so that the pair
@@ -12,10 +12,11 @@
 // Both orders of a quartet are visited: half the recursions could be saved by adding to the ket's J_q as
 // well, but every lane would then reduce or scatter that sum for each ket.
 //
-// Bound by the FP64 vector units: a lane keeps one bra primitive, its J_p and R^0 in registers, the kets
-// pass through LDS as broadcasts.  27 waters def2-TZVP, label j: 116 ms with the class kernels, 32 ms so;
-// the largest launches are those of the lowest ranks, (0,1) 6.7 ms and (2,1) 5.6 ms of 103 ms run one
-// after another.
+// Bound by the FP64 vector units, busy 84 to 94% of the time in the launches of ranks up to 3: a lane
+// keeps one bra primitive, its J_p and R^0 in registers, the kets pass through LDS as broadcasts.  The
+// ranks above it are held to 4 waves a CU by their registers, at 36 to 67%.  27 waters def2-TZVP, label
+// j: 116 ms with the class kernels, 32 ms so; run one after another the largest launches are those of the
+// lowest ranks, (1,0), (0,1), (1,1) and (0,0) at 2.0 to 2.4 ms of 29, beside 9 ms of class kernels.
 #pragma once
 
 #include "eri_kernels.h"

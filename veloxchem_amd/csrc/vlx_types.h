@@ -115,8 +115,9 @@ struct FockArgs {
                                    // pair of atom groups (from max|D| of the block), or nullptr (off)
     const double* dfac;            // multi-density kernels: (fj, fk) of each density, 2 x ndens doubles
     const int* k32;                // per molecule: FP32 bin-sum threshold on the device, or nullptr
-                                   // (tiled items: the FP64 kernel runs the item's bras with
-                                   // bin + bin_lo < k32, the FP32 kernel the others)
+                                   // (tiled items: of every 64-entry chunk the FP64 kernel runs the
+                                   // bras with bin + the chunk's smallest bin < k32, the FP32 kernel
+                                   // the others)
     FockScalars sc;
 };
 
