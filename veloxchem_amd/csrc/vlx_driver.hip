@@ -318,8 +318,9 @@ struct vlx_context {
     // 120.6 / 122.6 / 125.8 ms for a 20-water def2-TZVP build, 27.9 / 28.5 / 28.8 / 30.2 / 32.6 ms for 32-water def2-SVP
     int tile_items = 1024;
     int untiled_wave_cap = 8192;  // largest wavefront count of an untiled launch (VLX_UNTILED_WAVES)
-    // largest grid (one wavefront per block) of a matrix-core MD launch (VLX_MMD_GRID): on the 64-water
-    // def2-TZVP build 16384 / 32768 / 65536 measured 0.775 / 0.786 / 0.793 builds/s
+    // largest grid (one wavefront per block) of a matrix-core MD launch with direct digestion
+    // (VLX_MMD_GRID): two densities of 20 / 36 / 64 waters def2-TZVP at 65536 128.2 / 577 / 2411 ms, at 16384
+    // 129.2 / 579 / 2411
     int mmd_grid = 65536;
     bool use_jengine = true;        // Coulomb builds through Hermite densities (VLX_JENGINE)
     bool u_pending = false;         // U arrays still being built on the stream (ensure_u, finish_u)
@@ -935,11 +936,12 @@ int make_schedules(vlx_screener* s, int ithr, int k32, ScheduleUse use, int shar
         // default: tiled for L <= 4 and for L = 5 blocks of <= 75 integrals; the autotuner's choice, or
         // the one being timed, overrides it.  Lanes take single primitives instead of runs of up to 3 in
         // classes of L >= 4 whose kets have few: a lane's loop is then the same length in every lane.
-        // One stream, runs / single primitives, at ket primitives a quartet: 1.3 (ds| def2-TZVP (dp|ds) 2.53 /
-        // 2.11 ms, (fs|ds) 1.70 / 1.49 (20 waters), 1.45 (pp| def2-SVPD (ds|pp) 1.48 / 1.23, (pp|pp) 1.71 /
-        // 1.48 (13 waters), 1.5 (ds| def2-SVP 1.31 / 1.09 (32 waters); but 1.7 (ds| def2-SVPD (ds|ds)
-        // 0.44 / 0.50, 1.9 (pp| def2-TZVP (ds|pp) 1.54 / 1.69.  (dp|pp), 135 integrals: untiled / tiled
-        // single primitives 11.3 / 7.5 ms at 1.45, 3.7 / 4.5 at 1.9
+        // One stream, runs / single primitives, at ket primitives a quartet: 1.32 (ds| def2-TZVP (dp|ds) 2.17 /
+        // 1.94 ms, (fs|ds) 1.55 / 1.38 (20 waters), 1.45 (pp| def2-SVPD (ds|pp) 1.37 / 1.17, (pp|pp) 1.59 /
+        // 1.39 (13 waters), 1.49 (ds| def2-SVP (dp|ds) 1.37 / 1.07 (32 waters); from there on neither for
+        // all: 1.67 (ds| def2-SVPD (dp|ds) 2.15 / 2.07, (ds|ds) 0.45 / 0.44, 1.91 (pp| def2-SVP (ds|pp) 1.01 /
+        // 1.06, (pp|pp) 0.90 / 0.79, 1.94 (pp| def2-TZVP (ds|pp) 1.35 / 1.54.  (dp|pp), 135 integrals: untiled /
+        // tiled single primitives 11.3 / 7.5 ms at 1.45, 3.7 / 4.5 at 1.9
         const bool few_prims = L >= 4 && all.ket_prims * 2 < all.quartets * 3;
         int var = VARIANT_UNTILED;
         if (can_tile && (L <= 4 || nsph <= 75 || (L == 5 && few_prims))) {
