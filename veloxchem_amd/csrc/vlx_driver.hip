@@ -1277,14 +1277,22 @@ int make_schedules(vlx_screener* s, int ithr, int k32, ScheduleUse use, int shar
     return VLX_OK;
 }
 
+// Whether the context's stream is being captured into a graph: nothing may be allocated or waited for.
+bool capturing(const vlx_context* ctx)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 // The screener's schedule at these settings, built on the first call.
-// create = false: only a schedule built earlier is returned (no host or device allocation);
-// without one the call fails.
+// create = false, or under capture: only a schedule built earlier is returned (no host or device
+// allocation); without one the call fails.
 int get_schedules(vlx_screener* s, int ithr, int k32, std::vector<std::unique_ptr<ClassSchedule>>** out,
                   bool create = true, ScheduleUse use = USE_BUILD)
 {
     const std::pair<int, int> key{((ithr + 1) * 128 + k32) * (NVARIANTS + 1) + (s->ctx->force_variant + 1), use};
     auto it = s->schedules.find(key);
+    if (it == s->schedules.end() && create) create = !capturing(s->ctx);
     // a build of several densities leaves the direct digestion's schedule, complete on the device
     if (it == s->schedules.end() && !create && use == USE_BUILD) it = s->schedules.find({key.first, USE_DIRECT});
     if (it == s->schedules.end()) {
@@ -2593,10 +2601,11 @@ int fock_build(vlx_context* ctx, vlx_screener* scr, const double* d_density, dou
     if (rc) return rc;
     // Coulomb alone: through Hermite densities, the classes of higher angular momentum by their kernels.
     // The lists and J_p are the screener's: a build without allocation, of which several may be in flight
-    // in captured graphs, keeps to the class kernels, as do forced variants, per-class timing and the
-    // modes that need quartets
-    const bool hermite = fk == 0.0 && fj != 0.0 && ithreshold >= 0 && k32 == NO_FP32 && glim == nullptr && !no_alloc &&
-                         !ctx->timing && ctx->force_variant < 0 && ctx->use_jengine;
+    // in captured graphs, keeps to the class kernels, as do forced variants, per-class timing, the
+    // modes that need quartets, and a first Coulomb build under capture, which could not make the lists
+    bool hermite = fk == 0.0 && fj != 0.0 && ithreshold >= 0 && k32 == NO_FP32 && glim == nullptr && !no_alloc &&
+                   !ctx->timing && ctx->force_variant < 0 && ctx->use_jengine;
+    if (hermite && !(scr->jengine.ready && scr->jengine.items.count(ithreshold))) hermite = !capturing(ctx);
     const int lmin = hermite ? J_LMAX + 1 : 0;
     JEngine::Items* ji = nullptr;
     if (hermite) {
